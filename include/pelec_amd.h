@@ -16,8 +16,8 @@
  *  - Which calls block: prc_react_box, prc_react_flat, prc_react_boxes and prc_react_state_box
  *    return only once the reactor's kernels on the stream have finished (react_state's unpack
  *    kernel excepted, which is left enqueued). The plain form synchronises because its argument
- *    block is reused by the next call; the batched form reads its work-queue counters back after
- *    every replay of its captured graph to decide whether another is needed. PeleC synchronises
+ *    block is reused by the next call; the batched form because its workspace is, and its work
+ *    queue reads the counters back after every replay of its captured graph. PeleC synchronises
  *    the stream right after react anyway (React.cpp:230), so the drop-in keeps the reference's
  *    observable ordering. prc_autotune and prc_last_failures also block. prc_adjoint,
  *    prc_compute_temp, the EOS helpers and prc_model_eval enqueue and return.
@@ -99,13 +99,14 @@ int prc_set_typ_vals_ode(prc_reactor* r, const double* typ, int n);
  * ReactorRK64 rk64.nsubsteps_guess / rk64.nsubsteps_min / rk64.nsubsteps_max, default 10 / 5 /
  * 100000: first step dt/guess, steps within [dt/max, dt/min]; the pelec.adaptrk_nsubsteps_* knobs
  * of Exec/Production/ChallengeProblem/challenge.inp:29-31) and the gfx950 execution form:
- * "prc.form" = 0 plain FP64 one-cell-per-lane drop-in, 1 batched persistent work-queue kernel
- * (ReactorCvode only); "prc.lu_fp32" = 1 runs the Newton-matrix LU in FP32, each solve followed
+ * "prc.form" = 0 plain FP64 one-cell-per-lane drop-in, 1 batched (ReactorCvode only): with FP64
+ * factors one kernel whose lane groups each integrate whole cells taken from a queue, with FP32
+ * factors a work queue of integration phases; "prc.lu_fp32" = 1 runs the Newton-matrix LU in FP32, each solve followed
  * by "prc.lu_refine" (0, 1 or 2, default 1) FP64 refinement steps against the FP64 Jacobian. In
  * the batched form the FP32 factors are those of D M D^-1, D the powers of two of the cell's error
  * weights (exact scaling); the plain form factors M unscaled and always refines at least once. */
 int prc_set_param_real(prc_reactor* r, const char* key, double value);
-/* (launch shape of the batched form: prc.iters_per_graph (multiple of 3), prc.cooperative (bit 0:
+/* (launch shape of the batched form's work queue, used with FP32 factors: prc.iters_per_graph (multiple of 3), prc.cooperative (bit 0:
  * the Newton kernel, bit 1: the Jacobian kernel run one cell per 32-lane group instead of one
  * cell per lane), prc.blocks_newton, prc.blocks_jac, prc.blocks_lu (blocks per CU, 0 =
  * occupancy-derived), prc.compact_pct (compact the work queue when fewer than this percentage
@@ -120,7 +121,8 @@ int prc_set_param_real(prc_reactor* r, const char* key, double value);
  * convergence-failure handling) */
 int prc_set_param_int(prc_reactor* r, const char* key, int value);
 /* Read back an integer knob (the prc.* launch-shape knobs report the values in use; "prc.slots"
- * gives the slot count of the batched workspace now allocated). */
+ * gives the slot count of the batched workspace now allocated, or, after a call with FP64 factors,
+ * the cells that call held in flight: at most prc.max_slots when that is set). */
 int prc_get_param_int(prc_reactor* r, const char* key, int* value);
 /* Launch-shape autotuner of the batched form (prc.form 1, ReactorCvode): times react calls on the
  * given sample of cells (device arrays, component-major; copied, not modified) over candidate
@@ -129,7 +131,8 @@ int prc_get_param_int(prc_reactor* r, const char* key, int* value);
  * Jacobian and LU kernels (prc.blocks_newton / _jac / _lu), the compaction threshold
  * and interval (prc.compact_pct, prc.compact_every) -- by coordinate descent from the
  * occupancy-derived defaults, keeps the
- * fastest in the reactor and returns its time (ms) in *best_ms. Synchronises the stream. No
+ * fastest in the reactor and returns its time (ms) in *best_ms. With FP64 factors there is no
+ * shape to search: the sample is timed as it is. Synchronises the stream. No
  * counterpart in the reference (its GPU launch shapes are fixed at compile time). */
 int prc_autotune(prc_reactor* r, int64_t ncells, const double* rY, const double* T,
                  const double* rE, double dt, double* best_ms, void* stream);
@@ -248,7 +251,7 @@ int64_t prc_last_failures(prc_reactor* r, void* stream);
 /* Per-kernel device time of the previous batched react call, when the reactor was configured
  * with prc_set_param_int(r, "prc.kernel_timing", 1): ms[0..2] = total milliseconds of the
  * k_newton, k_jac and k_lu launches (HIP events on the stream each kernel ran on), *launches =
- * launches of each. Instrumentation with no counterpart in the reference (which only times whole
+ * launches of each. A call with FP64 factors is one launch, its time in ms[0]. Instrumentation with no counterpart in the reference (which only times whole
  * fabs, Source/React.cpp:168-169). */
 int prc_kernel_times(prc_reactor* r, double* ms, int64_t* launches);
 

@@ -31,6 +31,10 @@ HIP_FLAGS = [
     # packed FP32 instructions are kept out of the generated code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
+    # machine-level loop-invariant code motion hoists the literals and table loads of the kinetics
+    # out of the kernels' cell loops and keeps them in registers: k_cell at n = 22 needs 168 VGPRs and
+    # 436 B of scratch per lane with it, 164 VGPRs and no scratch without
+    "-mllvm", "-disable-machine-licm",
     # per-kernel register / scratch / LDS figures, checked below
     "-Rpass-analysis=kernel-resource-usage",
 ]

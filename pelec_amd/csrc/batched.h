@@ -69,7 +69,8 @@ enum Ctr : int {
   CT_JAC0 = 10,    // lengths of Jacobian lists 0..2: the set-up entries that need a Jacobian
   CT_INGRAPH = 13, // 1: compactions inside the graph allowed (no cell of the call waits for a slot)
   CT_GATE = 14,    // the graph's compaction check of the current iteration decided to compact
-  CT_COUNT = 15
+  CT_NEXT = 15,    // whole-cell form: next cell of the call to integrate
+  CT_COUNT = 16
 };
 
 __host__ __device__ constexpr int list_next(int r) { return r == NLISTS - 1 ? 0 : r + 1; }

@@ -113,6 +113,7 @@ struct BdfCell {
 
   struct Vec : LaneComps {
     static constexpr bool kMemory = false;
+    static constexpr bool kRegister = false;
     BdfCell* c;
     __device__ double& Z(int j, int i) const { return c->zn[j][i]; }
     __device__ double& A(int i) const { return c->acor[i]; }

@@ -79,6 +79,7 @@ __device__ inline double sel(const double (&a)[K], int idx) {
 // Operations on the Nordsieck array are reported to the accessor (rec_* members), so a recording
 // accessor can tape the step sequence for the discrete adjoint. NoTape is the empty default.
 struct NoTape {
+  static constexpr bool kRegister = false;
   __device__ void rec_rescale(int, double) const {}
   __device__ void rec_pascal(int, double) const {}
   __device__ void rec_order_up(int, int, int, double, const double*) const {}
@@ -103,6 +104,23 @@ struct LaneComps {
   using Arr = double[m];
 };
 
+// Nordsieck column j of component i at a run-time j. Accessors in memory index it; a register
+// accessor selects, so that its history is never addressed.
+template <class V>
+__device__ inline double col_at(const V& v, int j, int i) {
+  if constexpr (V::kRegister)
+    return v.ZR(j, i);
+  else
+    return v.Z(j, i);
+}
+template <class V>
+__device__ inline void set_col_at(const V& v, int j, int i, double x) {
+  if constexpr (V::kRegister)
+    v.ZW(j, i, x);
+  else
+    v.Z(j, i) = x;
+}
+
 // Vector accessors declare kMemory = true when Z/A/E live in device memory (the batched form's
 // structure-of-arrays state). The Nordsieck updates below then run one component at a time and
 // end each component with a compiler memory fence: the compiler keeps one component's <= 6
@@ -111,6 +129,24 @@ struct LaneComps {
 template <class V>
 __device__ inline void component_fence() {
   if constexpr (V::kMemory) PELEC_MEMORY_FENCE();
+}
+
+// End of a component loop. A group accessor's lanes of absent components skip the loop, and the
+// integrator scalars that follow are one copy per group, updated by all of its lanes: the group has
+// to be together again, or an update that the compiler copies into both sides of the branch is
+// applied twice (no instruction is spent on it; it is the compiler that may not move code past it).
+template <class V>
+__device__ inline void group_join() {
+  if constexpr (V::kStep > 1 && !V::kRegister) __builtin_amdgcn_wave_barrier();
+}
+
+// The absolute tolerance of component i.
+template <class V>
+__device__ inline double atol_at(const V& v, const BdfParams& prm, int i) {
+  if constexpr (V::kRegister)
+    return v.at;
+  else
+    return prm.atolv[i];
 }
 
 // Components per chunk of a Nordsieck pass. With the batched form's structure-of-arrays state
@@ -163,6 +199,17 @@ __device__ inline void scalars_reset(BdfScalars& S, int qmax) {
   S.m = S.convfail = S.nflag = S.ncf = S.nef = 0;
 }
 
+// x^(1/k), x >= 0, for the step-size factors: exp(log(x) / k) is within a few ulp of pow at a third
+// of its chain of dependent instructions (pow carries the logarithm in two doubles).
+__device__ inline double root(double x, int k) { return exp(log(x) / k); }
+// x^k for the orders' small k.
+__device__ inline double ipow(double x, int k) {
+  double r = x;
+#pragma unroll
+  for (int i = 2; i <= BDF_QMAX + 1; ++i) r = i <= k ? r * x : r;
+  return r;
+}
+
 template <int n, class V>
 __device__ inline double wrms_acor(const V& v) {
   double s = 0.0;
@@ -199,10 +246,11 @@ __device__ inline void set_ewt(const V& v, const BdfParams& prm) {
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const int i = i0 + c * V::kStep;
-      if (i < n) v.E(i) = 1.0 / (prm.rtol * fabs(z0[c]) + prm.atolv[i]);
+      if (i < n) v.E(i) = 1.0 / (prm.rtol * fabs(z0[c]) + atol_at(v, prm, i));
     }
     component_fence<V>();
   }
+  group_join<V>();
 }
 
 template <int n, class V>
@@ -232,6 +280,7 @@ __device__ inline void rescale(BdfScalars& S, const V& v) {
     }
     component_fence<V>();
   }
+  group_join<V>();
   S.h = S.hscale * S.eta;
   S.hscale = S.h;
 }
@@ -273,6 +322,7 @@ __device__ inline void pascal(const V& v, int q, double sign) {
     }
     component_fence<V>();
   }
+  group_join<V>();
 }
 
 template <int n, class V>
@@ -425,7 +475,7 @@ __device__ inline void adjust_order(BdfScalars& S, const V& v, int dq, int qmax)
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const int i = i0 + c * V::kStep;
-      za[c] = (i < n && kind == 1) ? v.Z(ia, i) : 0.0;
+      za[c] = (i < n && kind == 1) ? col_at(v, ia, i) : 0.0;
       z[c][0] = z[c][1] = 0.0;
 #pragma unroll
       for (int j = 2; j <= BDF_QMAX; ++j) z[c][j] = (i < n && j <= q) ? v.Z(j, i) : 0.0;
@@ -440,6 +490,7 @@ __device__ inline void adjust_order(BdfScalars& S, const V& v, int dq, int qmax)
     }
     component_fence<V>();
   }
+  group_join<V>();
 }
 
 // Start of cvStep: order/step change decided at the end of the previous step.
@@ -524,14 +575,14 @@ __device__ inline bool next_attempt(BdfScalars& S, const V& v, const BdfParams& 
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const int i = i0 + c * V::kStep;
-      za[c] = (i < n && kind == 1) ? v.Z(ia, i) : 0.0;
+      za[c] = (i < n && kind == 1) ? col_at(v, ia, i) : 0.0;
 #pragma unroll
       for (int j = 0; j <= BDF_QMAX; ++j) z[c][j] = (i < n && j <= ql) ? v.Z(j, i) : 0.0;
     }
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const int i = i0 + c * V::kStep;
-      const double ew = i < n ? 1.0 / (prm.rtol * fabs(z[c][0]) + prm.atolv[i]) : 0.0;
+      const double ew = i < n ? 1.0 / (prm.rtol * fabs(z[c][0]) + atol_at(v, prm, i)) : 0.0;
       order_apply(kind, S.l, A1, q0, L0, za[c], z[c]);
       if (resc) {
 #pragma unroll
@@ -548,6 +599,7 @@ __device__ inline bool next_attempt(BdfScalars& S, const V& v, const BdfParams& 
     }
     component_fence<V>();
   }
+  group_join<V>();
   return attempt_setup(S);
 }
 
@@ -606,7 +658,7 @@ __device__ inline int error_test_fail(BdfScalars& S, const V& v, double dsm, int
   if (S.nef == cv::MXNEF) return CELL_ERRFAIL;
   S.etamax = 1.0;
   if (S.nef <= cv::MXNEF1) {
-    S.eta = 1.0 / (pow(cv::BIAS2 * dsm, 1.0 / S.L) + cv::ADDON);
+    S.eta = 1.0 / (root(cv::BIAS2 * dsm, S.L) + cv::ADDON);
     S.eta = fmax(cv::ETAMIN, S.eta);
     if (S.nef >= cv::SMALL_NEF) S.eta = fmin(S.eta, cv::ETAMXF);
     rescale<n>(S, v);
@@ -658,7 +710,7 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
   const bool test = S.etamax != 1.0 && S.qwait == 0;
   const bool down = test && q > 1;
   const bool up = test && q != qmax && S.saved_tq5 != 0.0;
-  const double cquot = up ? (S.tq[5] / S.saved_tq5) * pow(S.h / S.tau[2], (double)S.L) : 0.0;
+  const double cquot = up ? (S.tq[5] / S.saved_tq5) * ipow(S.h / S.tau[2], S.L) : 0.0;
   double sdn = 0.0, sup = 0.0;
   {
     constexpr int K = chunk_of<V>();
@@ -670,7 +722,7 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
         const int i = i0 + c * V::kStep;
         a[c] = i < n ? v.A(i) : 0.0;
         e[c] = (i < n && test) ? v.E(i) : 0.0;
-        zm[c] = (i < n && up) ? v.Z(qmax, i) : 0.0;
+        zm[c] = (i < n && up) ? col_at(v, qmax, i) : 0.0;
         if (i < n) {
           load_hist(v, i, q, z[c]);
         } else {
@@ -696,11 +748,12 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
 #pragma unroll
           for (int j = 0; j <= BDF_QMAX; ++j)
             if (j <= q) v.Z(j, i) = z[c][j];
-          if (save_acor) v.Z(qmax, i) = a[c];
+          if (save_acor) set_col_at(v, qmax, i, a[c]);
         }
       }
       component_fence<V>();
     }
+    group_join<V>();
   }
   if (save_acor) {
     S.saved_tq5 = S.tq[5];
@@ -713,7 +766,7 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
     S.hprime = S.h;
     S.eta = 1.0;
   } else {
-    const double etaq = 1.0 / (pow(cv::BIAS2 * dsm, 1.0 / S.L) + cv::ADDON);
+    const double etaq = 1.0 / (root(cv::BIAS2 * dsm, S.L) + cv::ADDON);
     if (S.qwait != 0) {
       S.eta = etaq;
       S.qprime = S.q;
@@ -723,12 +776,12 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
       double etaqm1 = 0.0;
       if (down) {
         const double ddn = sqrt(v.sum(sdn) / n) * S.tq[1];
-        etaqm1 = 1.0 / (pow(cv::BIAS1 * ddn, 1.0 / S.q) + cv::ADDON);
+        etaqm1 = 1.0 / (root(cv::BIAS1 * ddn, S.q) + cv::ADDON);
       }
       double etaqp1 = 0.0;
       if (up) {
         const double dup = sqrt(v.sum(sup) / n) * S.tq[3];
-        etaqp1 = 1.0 / (pow(cv::BIAS3 * dup, 1.0 / (S.L + 1)) + cv::ADDON);
+        etaqp1 = 1.0 / (root(cv::BIAS3 * dup, S.L + 1) + cv::ADDON);
       }
       const double etam = fmax(etaqm1, fmax(etaq, etaqp1));
       if (etam < cv::THRESH) {
@@ -756,10 +809,11 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
 #pragma unroll
           for (int c = 0; c < K; ++c) {
             const int i = i0 + c * V::kStep;
-            if (i < n) v.Z(qmax, i) = a[c];
+            if (i < n) set_col_at(v, qmax, i, a[c]);
           }
           component_fence<V>();
         }
+        group_join<V>();
       }
       set_eta(S);
     }
@@ -828,12 +882,14 @@ __device__ inline int newton_correct(BdfScalars& S, const V& v, const FT& ftemp,
   const double rl1 = 1.0 / S.l[1];
 #pragma unroll
   for (int i = v.c0(); i < n; i += V::kStep) tempv[i] = S.gamma * ftemp[i] - (rl1 * v.Z(1, i) + v.A(i));
+  group_join<V>();
   solve(tempv);
   if (S.gamrat != 1.0) {
     const double sc = 2.0 / (1.0 + S.gamrat);
 #pragma unroll
     for (int i = v.c0(); i < n; i += V::kStep) tempv[i] *= sc;
   }
+  group_join<V>();
   S.nni++;
   // one pass: the WRMS norm of the correction (del), acor += correction, and the WRMS norm of the
   // updated acor (cvNlsNewton's acnrm), each sum in component order
@@ -863,6 +919,7 @@ __device__ inline int newton_correct(BdfScalars& S, const V& v, const FT& ftemp,
       }
       component_fence<V>();
     }
+    group_join<V>();
   }
   const double del = sqrt(v.sum(sdel) / n);
   const double acn = sqrt(v.sum(sacor) / n);

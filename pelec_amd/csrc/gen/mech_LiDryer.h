@@ -3,6 +3,7 @@
 // species: 9  reactions: 21
 #pragma once
 #include <cmath>
+#include <cstdint>
 #ifndef PELEC_MEMORY_FENCE
 #define PELEC_MEMORY_FENCE() __asm__ __volatile__("" ::: "memory")
 #endif
@@ -1622,6 +1623,34 @@ struct LiDryer {
   static constexpr double T_CSR_NU[79] = {-1.0, -1.0, -1.0, 1.0, 1.0, -1.0, 1.0, -1.0, 1.0, 1.0, 1.0, 1.0, 1.0, 1.0, -1.0, 1.0, 1.0, 1.0, 1.0, 1.0, -1.0, 1.0, 1.0, 2.0, -1.0, -1.0, -1.0, -1.0, -1.0, -1.0, -1.0, 1.0, -1.0, -1.0, -2.0, -1.0, -1.0, -1.0, 1.0, 1.0, -1.0, 2.0, 1.0, -1.0, 2.0, 1.0, -1.0, 2.0, 1.0, 1.0, -1.0, -1.0, 1.0, -1.0, -1.0, -1.0, -1.0, -2.0, -2.0, 1.0, 1.0, 1.0, 1.0, 1.0, 1.0, -1.0, -1.0, -1.0, -1.0, -1.0, -1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   static constexpr int T_CSR_SLOT[79][6] = {{0, 4, -1, 3, 5, -1}, {0, 5, -1, 2, 3, -1}, {0, -1, -1, 3, -1, -1}, {3, 6, -1, 0, 1, -1}, {3, 7, -1, 0, 6, -1}, {1, 3, -1, 4, 5, -1}, {4, -1, -1, 1, -1, -1}, {1, 3, -1, 6, -1, -1}, {3, 6, -1, 0, 1, -1}, {4, 6, -1, 1, 5, -1}, {5, 6, -1, 1, 2, -1}, {6, -1, -1, 1, 7, -1}, {6, -1, -1, 1, 7, -1}, {0, 5, -1, 2, 3, -1}, {2, 4, -1, 5, -1, -1}, {3, 5, -1, 2, -1, -1}, {5, 6, -1, 1, 2, -1}, {3, 7, -1, 2, 5, -1}, {5, 7, -1, 2, 6, -1}, {5, 7, -1, 2, 6, -1}, {1, 3, -1, 4, 5, -1}, {0, 4, -1, 3, 5, -1}, {0, 5, -1, 2, 3, -1}, {0, -1, -1, 3, -1, -1}, {3, 4, -1, 5, -1, -1}, {3, 5, -1, 2, -1, -1}, {1, 3, -1, 6, -1, -1}, {3, 6, -1, 0, 1, -1}, {3, 6, -1, 5, -1, -1}, {3, 7, -1, 2, 5, -1}, {3, 7, -1, 0, 6, -1}, {1, 3, -1, 4, 5, -1}, {0, 4, -1, 3, 5, -1}, {2, 4, -1, 5, -1, -1}, {4, -1, -1, 1, -1, -1}, {3, 4, -1, 5, -1, -1}, {4, 6, -1, 1, 5, -1}, {4, 7, -1, 5, 6, -1}, {1, 3, -1, 4, 5, -1}, {0, 4, -1, 3, 5, -1}, {0, 5, -1, 2, 3, -1}, {2, 4, -1, 5, -1, -1}, {3, 4, -1, 5, -1, -1}, {3, 5, -1, 2, -1, -1}, {3, 6, -1, 5, -1, -1}, {4, 6, -1, 1, 5, -1}, {5, 6, -1, 1, 2, -1}, {7, -1, -1, 5, -1, -1}, {3, 7, -1, 2, 5, -1}, {4, 7, -1, 5, 6, -1}, {5, 7, -1, 2, 6, -1}, {5, 7, -1, 2, 6, -1}, {1, 3, -1, 6, -1, -1}, {3, 6, -1, 0, 1, -1}, {3, 6, -1, 5, -1, -1}, {4, 6, -1, 1, 5, -1}, {5, 6, -1, 1, 2, -1}, {6, -1, -1, 1, 7, -1}, {6, -1, -1, 1, 7, -1}, {3, 7, -1, 0, 6, -1}, {4, 7, -1, 5, 6, -1}, {5, 7, -1, 2, 6, -1}, {5, 7, -1, 2, 6, -1}, {6, -1, -1, 1, 7, -1}, {6, -1, -1, 1, 7, -1}, {7, -1, -1, 5, -1, -1}, {3, 7, -1, 2, 5, -1}, {3, 7, -1, 0, 6, -1}, {4, 7, -1, 5, 6, -1}, {5, 7, -1, 2, 6, -1}, {5, 7, -1, 2, 6, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}};
   static constexpr int T_CSR_EFF[79] = {-1, -1, 0, -1, -1, -1, 0, 1, -1, -1, -1, -1, -1, -1, -1, 0, -1, -1, -1, -1, -1, -1, -1, 0, 0, 0, 1, -1, -1, -1, -1, -1, -1, -1, 0, 0, -1, -1, -1, -1, -1, -1, 0, 0, -1, -1, -1, 0, -1, -1, -1, -1, 1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, 0, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
+  // ---- lane-group tables (whole_cell.h)
+  static constexpr bool G_OK = true;
+  static constexpr int G_W = 16;   // lanes per cell
+  static constexpr int G_RR = 2;  // reaction rounds
+  alignas(16) static constexpr double G_TMID[16] = {1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0, 1000.0};
+  alignas(16) static constexpr double G_WT[16] = {2.01594, 31.9988, 18.01534, 1.00797, 15.9994, 17.007369999999998, 33.006769999999996, 34.014739999999996, 28.0134, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  alignas(16) static constexpr double G_IWT[16] = {0.49604650932071387, 0.03125117191894696, 0.055508250191225926, 0.9920930186414277, 0.06250234383789392, 0.05879803873262004, 0.03029681486555637, 0.02939901936631002, 0.03569720205330306, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  alignas(16) static constexpr double G_E[2][3][16][2] = {{{{-41760012721.584656, 94782910.65151145}, {-2612005835.355053, 5750019.890860144}, {-139416853281.73718, 11015783.540270746}, {2101083518938.3674, 123730804.75837436}, {151472532212.07553, 10115073.789885493}, {16359238477.301249, 15278809.51884366}, {742626566.6440628, 8317286.461788826}, {-43175282361.06859, 5838999.75039175}, {-3030062358.3258877, 6822543.492653029}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{17011.834957792224, -11.194908878994598}, {1464.8112115909228, -0.498553008232421}, {8018.89055042963, -9.776091253662699}, {0.0, 0.0}, {-4256.556486283742, 4.193819781023616}, {-7884.193258540319, 10.637324920058875}, {-5981.558472625442, 17.766032421634424}, {8028.811040037399, -0.12099739775532213}, {2089.8496500582078, -3.9209879517709996}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-0.0009770025618790518, 3.4107402675524593e-06}, {0.0008534836619928971, -4.5567842824267206e-07}, {0.00804037090419511, -2.3136873603397435e-06}, {0.0, 0.0}, {-0.0020823871842488772, 4.043782448166599e-07}, {-0.0070868856247666085, 2.0164822405361935e-06}, {-0.015288161502173006, 4.681468412296513e-06}, {-0.0028267959027342975, 1.2082596590598668e-06}, {0.004186047175392025, -1.4512808516142303e-06}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}}, {{{-34439809606.868126, 82133456.80144538}, {-3206203000.868104, 7009297.673835451}, {-137991214074.95697, 7717309.475754812}, {2101083518938.3674, 123730804.75837436}, {151904692612.66907, 8013675.653430371}, {18008306717.04652, 9116176.33970538}, {281769000.368105, 7600406.5951120015}, {-44015681374.1868, 8734143.91817158}, {-2738891737.799691, 5718326.321916925}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{14436.58859911475, -0.7745313289345194}, {797.0746732925282, -0.1090311173248295}, {7052.721152812942, -1.343066897743044}, {0.0, 0.0}, {-71.58662202862139, -0.005374813962813966}, {2582.488357950532, -0.42219616287900336}, {2821.072880241255, -0.5320652905311182}, {5299.561407676278, -1.2015620839575023}, {2208.180574862709, -0.5624181383151804}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-9.518588126080866e-05, 1.3055678579528436e-08}, {1.153207894609931e-05, -5.905750419053826e-10}, {0.00013857130016074593, -5.899735328949149e-09}, {0.0, 0.0}, {5.912671169576799e-06, -4.5399208805517084e-10}, {3.7303375762027e-05, -1.302320266912726e-09}, {7.194714695081523e-05, -5.436469429981671e-09}, {0.0001435397896737607, -6.998985536934612e-09}, {7.492080721547366e-05, -4.0088303766602985e-09}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}}};
+  alignas(16) static constexpr double G_G[2][4][16][2] = {{{{6.592218, -0.0004124721}, {-2.821802, -0.000563743}, {0.7966090000000001, -0.001737491}, {2.9601176000000002, 0.0}, {-0.01756599999999997, 0.000819083}, {4.81573857, 0.001612724695}, {0.5851355599999999, 0.002374560255}, {-3.396609, -0.003284613}, {-0.6516950000000001, -0.00070412}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{1.3571691666666666e-07, 7.896194999999999e-12}, {9.593583333333333e-08, -1.0948975000000001e-10}, {1.059116e-06, -5.807150833333333e-10}, {0.0, 0.0}, {-4.035053333333333e-07, 1.3357024999999999e-10}, {-1.0879411516666667e-06, 4.832113691666666e-10}, {-3.5263815166666663e-06, 2.02303245e-09}, {2.4750216666666664e-08, 3.854838333333333e-10}, {6.605369999999999e-07, -4.701262500000001e-10}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-2.067436e-14, 3.298124}, {4.384277e-14, 3.212936}, {1.2532940000000001e-13, 3.386842}, {0.0, 2.5}, {-1.945348e-14, 2.946429}, {-1.0311868949999999e-13, 4.12530561}, {-4.646125620000001e-13, 4.30179801}, {-1.2357574999999998e-13, 3.388754}, {1.2224275000000001e-13, 3.298677}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-1012.521, 0.0}, {-1005.249, 0.0}, {-30208.11, 0.0}, {25471.63, 0.0}, {29147.64, 0.0}, {3346.30913, 0.0}, {294.80804, 0.0}, {-17663.15, 0.0}, {-1020.9, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}}, {{{4.346533, -0.0003500322}, {0.5084119999999999, -0.00030675985}, {-4.190671, -0.0015281465}, {2.9601176000000002, 0.0}, {-2.378248, 1.377531e-05}, {-2.8369118700000002, -0.00052825224}, {0.23210875000000009, -0.001119910065}, {4.07203, -0.002168068}, {-3.0538879999999997, -0.0007439885}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{9.389715e-09, 7.692981666666667e-13}, {2.09807e-08, -1.4794008333333333e-12}, {1.4550433333333335e-07, -1.00083e-11}, {0.0, 0.0}, {5.171338333333333e-10, -3.7925558333333335e-13}, {4.318045966666667e-08, -2.54348895e-12}, {1.0560969166666666e-07, -9.520530833333334e-12}, {2.457815e-07, -1.9574199999999998e-11}, {9.474601666666666e-08, -8.4142e-12}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-7.91376e-17, 2.991423}, {5.682175000000001e-17, 3.697578}, {3.195809e-16, 2.672146}, {0.0, 2.5}, {2.184026e-17, 2.54206}, {6.6597938e-17, 2.86472886}, {5.39542675e-16, 4.0172109}, {7.15827e-16, 4.573167}, {3.3766754999999997e-16, 2.92664}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-835.034, 0.0}, {-1233.93, 0.0}, {-29899.21, 0.0}, {25471.63, 0.0}, {29230.8, 0.0}, {3683.62875, 0.0}, {111.856713, 0.0}, {-18006.96, 0.0}, {-922.7977, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}}};
+  alignas(16) static constexpr double G_H[2][3][16][2] = {{{{3.298124, 0.0004124721}, {3.212936, 0.000563743}, {3.386842, 0.001737491}, {2.5, 0.0}, {2.946429, -0.000819083}, {4.12530561, -0.001612724695}, {4.30179801, -0.002374560255}, {3.388754, 0.003284613}, {3.298677, 0.00070412}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-2.714338333333333e-07, -2.3688585e-11}, {-1.9187166666666667e-07, 3.2846925e-10}, {-2.118232e-06, 1.74214525e-09}, {0.0, 0.0}, {8.070106666666666e-07, -4.0071075e-10}, {2.1758823033333334e-06, -1.4496341075e-09}, {7.0527630333333326e-06, -6.06909735e-09}, {-4.950043333333333e-08, -1.1564515e-09}, {-1.3210739999999999e-06, 1.41037875e-09}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{8.269744e-14, -1012.521}, {-1.7537108e-13, -1005.249}, {-5.013176000000001e-13, -30208.11}, {0.0, 25471.63}, {7.781392e-14, 29147.64}, {4.1247475799999997e-13, 3346.30913}, {1.8584502480000002e-12, 294.80804}, {4.943029999999999e-13, -17663.15}, {-4.889710000000001e-13, -1020.9}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}}, {{{2.991423, 0.0003500322}, {3.697578, 0.00030675985}, {2.672146, 0.0015281465}, {2.5, 0.0}, {2.54206, -1.377531e-05}, {2.86472886, 0.00052825224}, {4.0172109, 0.001119910065}, {4.573167, 0.002168068}, {2.92664, 0.0007439885}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{-1.877943e-08, -2.3078945e-12}, {-4.19614e-08, 4.4382025e-12}, {-2.910086666666667e-07, 3.00249e-11}, {0.0, 0.0}, {-1.0342676666666666e-09, 1.13776675e-12}, {-8.636091933333334e-08, 7.63046685e-12}, {-2.1121938333333332e-07, 2.85615925e-11}, {-4.91563e-07, 5.87226e-11}, {-1.8949203333333333e-07, 2.52426e-11}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}, {{3.165504e-16, -835.034}, {-2.2728700000000004e-16, -1233.93}, {-1.2783236e-15, -29899.21}, {0.0, 25471.63}, {-8.736104e-17, 29230.8}, {-2.66391752e-16, 3683.62875}, {-2.1581707e-15, 111.856713}, {-2.863308e-15, -18006.96}, {-1.3506701999999999e-15, -922.7977}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}}}};
+  static constexpr int G_MN = 3;
+  alignas(16) static constexpr int G_MI[3][16] = {{0, 0, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9}, {2, 1, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9}, {9, 2, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9, 9}};
+  alignas(16) static constexpr double G_MD[3][16] = {{1.5, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, {11.0, -0.21999999999999997, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, {0.0, 10.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
+  static constexpr int G_NFO = 2;  // falloff reactions: positions 0..G_NFO-1
+  static constexpr int G_NTB = 6;  // reactions with a third body
+  alignas(16) static constexpr int G_RORD[32] = {8, 15, 4, 5, 6, 7, 0, 1, 2, 3, 9, 10, 11, 12, 13, 14, 16, 17, 18, 19, 20, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
+  alignas(16) static constexpr double G_RA[32][2] = {{1475000000000.0, 0.6}, {295100000000000.0, 0.0}, {4.577e+19, -1.4}, {6165000000000000.0, -0.5}, {4.714e+18, -1.0}, {3.8e+22, -2.0}, {3547000000000000.0, -0.406}, {50800.0, 2.67}, {216000000.0, 1.51}, {2970000.0, 2.02}, {16600000000000.0, 0.0}, {70790000000000.0, 0.0}, {32500000000000.0, 0.0}, {28900000000000.0, 0.0}, {420000000000000.0, 0.0}, {130000000000.0, 0.0}, {24100000000000.0, 0.0}, {48200000000000.0, 0.0}, {9550000.0, 2.0}, {1000000000000.0, 0.0}, {580000000000000.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
+  alignas(16) static constexpr double G_RE[32] = {0.0, 24370.922007345227, 52526.05490660117, 0.0, 0.0, 0.0, 8352.941036546013, 3165.2508657072367, 1726.0429999007667, 6743.141748883461, 414.14967606948426, 148.4497623821359, 0.0, -250.1001081488866, 6029.576450382212, -819.895585929539, 1997.7815479901, 4000.595291315188, 1997.7815479901, 0.0, 4809.269081647704, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  alignas(16) static constexpr uint64_t G_RP[32] = {1009097725868311297ull, 2161737738301802759ull, 2089680135640385792ull, 936758656769786884ull, 936758656836895747ull, 936758656786564355ull, 1441161797905744641ull, 1441161797888967680ull, 1441161789282256128ull, 1441161797922522114ull, 1441161780658767363ull, 1441161797922522627ull, 1441161797855413764ull, 1441161784970511877ull, 1441161806445348358ull, 1441161806445348358ull, 1441161797872191235ull, 1441161802133604099ull, 1441161802217490180ull, 1441161802167158533ull, 1441161802167158533ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull};
+  alignas(16) static constexpr double G_LOW[3][2] = {{19.88299408302048, 6.009598019134351}, {-2.32, 0.0}, {264.08961118015225, -1474.4332331513833}};
+  alignas(16) static constexpr double G_TROE[8][2] = {{0.19999999999999996, 0.5}, {-9.999999999999999e+29, -9.999999999999999e+29}, {0.8, 0.5}, {-9.999999999999999e-31, -9.999999999999999e-31}, {0.0, 0.0}, {0.0, 0.0}, {-1.9999999999999995e+29, -4.9999999999999994e+29}, {-8e-31, -4.9999999999999995e-31}};
+  alignas(16) static constexpr int G_TROEK[2] = {1, 1};
+  static constexpr int G_L4 = 2;
+  static constexpr int G_CMAX = 3;  // chunks of a species
+  alignas(16) static constexpr int G_GE[2][16][4] = {{{-16777200, -16777160, -16777152, 16777296}, {-16777216, 16777240, -16777168, 16777296}, {16777328, 16777336, 256, 256}, {16777256, 16777280, -16777144, 16777320}, {16777376, 256, 256, 256}, {-16777216, 33554448, -16777184, -16777176}, {16777280, -16777136, -16777128, -16777088}, {-33554408, -16777184, 16777264, -16777160}, {-16777072, 256, 256, 256}, {33554440, 16777248, -16777176, 16777264}, {33554504, 33554520, 16777312, -16777112}, {-16777064, -16777056, 256, 256}, {16777216, -16777136, -16777128, -16777120}, {-33554312, 16777352, 16777360, 16777368}, {-16777208, 16777328, 16777336, -16777088}, {-16777064, -16777056, 256, 256}}, {{16777352, 256, 256, 256}, {16777312, 16777320, 256, 256}, {256, 256, 256, 256}, {16777344, 16777368, 256, 256}, {256, 256, 256, 256}, {-16777168, 16777272, 256, 256}, {-16777080, 256, 256, 256}, {-16777144, -16777120, 256, 256}, {256, 256, 256, 256}, {16777272, -16777152, 256, 256}, {16777344, 16777360, 256, 256}, {256, 256, 256, 256}, {-16777112, -33554320, 256, 256}, {16777376, 256, 256, 256}, {-16777080, -16777072, 256, 256}, {256, 256, 256, 256}}};
+  alignas(16) static constexpr int G_CP[16] = {256, 513, 515, 517, 519, 777, 524, 526, 16, 0, 0, 0, 0, 0, 0, 0};
+  alignas(16) static constexpr int G_JO[3] = {0, 10, 15};
+  alignas(16) static constexpr int G_JE[15][16] = {{65282, 65280, 261, 65280, 65027, 513, 256, 65281, 0, 0, 0, 0, 0, 0, 0, 0}, {65287, 259, 264, 514, 65284, 260, 65290, 270, 0, 0, 0, 0, 0, 0, 0, 0}, {65288, 65286, 65289, 65284, 262, 65285, 65291, 271, 0, 0, 0, 0, 0, 0, 0, 0}, {266, 266, 269, 65285, 65287, 262, 65292, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 268, 0, 65286, 65289, 263, 65293, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 269, 0, 263, 65292, 65288, 65038, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 270, 0, 264, 0, 521, 65039, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 271, 0, 65290, 0, 523, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 65291, 0, 268, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 65293, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {257, 0, 256, 65280, 65282, 256, 257, 65280, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 259, 65281, 0, 258, 258, 65281, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 260, 0, 0, 65283, 259, 65282, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 65284, 260, 65283, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 65284, 0, 0, 0, 0, 0, 0, 0, 0}};
 };
 }  // namespace mech
 }  // namespace pelec

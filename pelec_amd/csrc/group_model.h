@@ -76,6 +76,26 @@ __device__ inline T group_read(T x, int src) {
   return r;
 }
 
+// Both sides of a butterfly step across rows of 16 lanes, by a row or half-wave swap (VALU, no LDS
+// round trip): a and b receive x of the lower and of the upper row (off = 16) or half (off = 32) of
+// the lane's pair, so a op b is the step's result on every lane.
+template <int off>
+__device__ inline void swap_pair(double x, double& a, double& b) {
+  static_assert(off == 16 || off == 32, "rows of 16 lanes or halves of the wave");
+  const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
+  if constexpr (off == 16) {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    a = __hiloint2double((int)h[0], (int)l[0]);
+    b = __hiloint2double((int)h[1], (int)l[1]);
+  } else {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    a = __hiloint2double((int)h[0], (int)l[0]);
+    b = __hiloint2double((int)h[1], (int)l[1]);
+  }
+}
+
 template <int G>
 struct Group {
   static_assert(G <= 64 && G >= 16 && (G & (G - 1)) == 0,
@@ -83,8 +103,15 @@ struct Group {
   // butterfly sums and maxima: offsets G/2 .. 1 (IEEE addition and fmax are commutative, so
   // every lane of the group ends with the same bits)
   __device__ static double sum(double x) {
-    if constexpr (G > 32) x += xor_partner<G, 32>(x);
-    if constexpr (G > 16) x += xor_partner<G, 16>(x);
+    double a, b;
+    if constexpr (G > 32) {
+      swap_pair<32>(x, a, b);
+      x = a + b;
+    }
+    if constexpr (G > 16) {
+      swap_pair<16>(x, a, b);
+      x = a + b;
+    }
     x += xor_partner<G, 8>(x);
     x += xor_partner<G, 4>(x);
     x += xor_partner<G, 2>(x);
@@ -92,8 +119,15 @@ struct Group {
     return x;
   }
   __device__ static double max(double x) {
-    if constexpr (G > 32) x = fmax(x, xor_partner<G, 32>(x));
-    if constexpr (G > 16) x = fmax(x, xor_partner<G, 16>(x));
+    double a, b;
+    if constexpr (G > 32) {
+      swap_pair<32>(x, a, b);
+      x = fmax(a, b);
+    }
+    if constexpr (G > 16) {
+      swap_pair<16>(x, a, b);
+      x = fmax(a, b);
+    }
     x = fmax(x, xor_partner<G, 8>(x));
     x = fmax(x, xor_partner<G, 4>(x));
     x = fmax(x, xor_partner<G, 2>(x));

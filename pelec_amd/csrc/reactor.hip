@@ -1,7 +1,8 @@
 // gfx950 reactor library for one mechanism: host side and the C-ABI of include/pelec_amd.h.
 // Built once per mechanism with -DPELEC_MECH=<ident> -DPELEC_MECH_HEADER="gen/mech_<name>.h".
 //
-// prc.form 0 (plain): one launch of react_plain per box; prc.form 1 (batched): k_start, then a
+// prc.form 0 (plain): one launch of react_plain per box; prc.form 1 (batched) with FP64 factors: one
+// launch of k_cell for the call (whole_cell.h); with FP32 factors the work queue: k_start, then a
 // captured graph of a fixed number of iterations replayed until every started cell is done, with a
 // compaction of the live slots whenever fewer than half remain alive. Each iteration forks into
 // two branches that run concurrently on disjoint cells: k_jac -> k_lu (set-up list) and k_newton
@@ -136,6 +137,12 @@ struct prc_reactor {
   int ncu = 0;
   int occ_newton = 1, occ_jac = 1, occ_lu = 1, occ_tail = 1;
   int64_t last_iterations = 0;
+  // whole-cell form: device memory for the Jacobians of the cells in flight, its size in groups of
+  // lanes, and the waves of k_cell that fit the GPU (0: not looked up yet)
+  double* wws = nullptr;
+  int64_t wws_groups = 0;
+  int whole_blocks = 0;
+  int64_t whole_cells = 0;  // cells in flight of the last whole-cell call (0: the last was not one)
   // PELEC_AMD_TRACE=1: one stderr line per graph replay of the batched form (live-cell counts)
   bool trace = false;
   // adjoint: checkpoint segment length, checkpoints and tape records per cell; workspace
@@ -525,6 +532,106 @@ int run_batched(prc_reactor* r, Args& a, hipStream_t s, Args* dargs, unsigned lo
   return PRC_OK;
 }
 
+// The work queue in the handle's factor precision. FP64 factors run in the whole-cell form wherever
+// the mechanism has its tables, so the FP64 queue is built for the other mechanisms only.
+template <class M = Mech>
+int run_queue(prc_reactor* r, Args& a, hipStream_t s, Args* dargs, unsigned long long* dctr,
+              bool graphs) {
+  if constexpr (!whole_ok<M>())
+    if (!r->lu_fp32) return run_batched<double>(r, a, s, dargs, dctr, graphs);
+  return run_batched<float>(r, a, s, dargs, dctr, graphs);
+}
+
+template <class M = Mech>
+int queue_occupancy(prc_reactor* r) {
+  if constexpr (!whole_ok<M>())
+    if (!r->lu_fp32) return occupancy_setup<double>(r);
+  return occupancy_setup<float>(r);
+}
+
+// ---- whole-cell form (k_cell, whole_cell.h): FP64 factors, any number of cells, one launch.
+#ifdef PELEC_WHOLE_WAVES
+constexpr int WHOLE_WAVES = PELEC_WHOLE_WAVES;
+#else
+constexpr int WHOLE_WAVES = NV <= 32 ? 3 : 2;
+#endif
+
+// Grid of a call: one wave per block, as many as fit the GPU at once. With fewer cells than groups
+// of lanes each wave takes fewer cells at a time (gpw): the groups of a wave run in lockstep, so a
+// cell alone on its wave never waits for another cell's phases, and the spare waves cost nothing.
+struct WholeGrid {
+  int blocks = 0, gpw = 0;
+  int64_t groups = 0;  // groups of lanes that own workspace
+};
+template <class M = Mech>
+constexpr int whole_gpw() {
+  if constexpr (whole_ok<M>())
+    return 64 / M::G_W;
+  else
+    return 1;
+}
+
+template <class M = Mech>
+int whole_grid(prc_reactor* r, int64_t ncells, WholeGrid& w) {
+  if constexpr (whole_ok<M>()) {
+    if (!r->whole_blocks) {
+      int dev = 0, o = 0;
+      HIP_OK(hipGetDevice(&dev));
+      HIP_OK(hipDeviceGetAttribute(&r->ncu, hipDeviceAttributeMultiprocessorCount, dev));
+      HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, (k_cell<M, WHOLE_WAVES>), 64, 0));
+      r->whole_blocks = std::max(o, 1) * r->ncu;
+    }
+    int64_t groups = std::max<int64_t>(ncells, 1);
+    if (r->max_slots > 0) groups = std::min<int64_t>(groups, r->max_slots);
+    const int64_t per = (groups + r->whole_blocks - 1) / r->whole_blocks;
+    w.gpw = (int)std::min<int64_t>(std::max<int64_t>(per, 1), whole_gpw());
+    w.blocks = (int)std::min<int64_t>((groups + w.gpw - 1) / w.gpw, r->whole_blocks);
+    w.groups = (int64_t)w.blocks * whole_gpw();
+  }
+  return PRC_OK;
+}
+
+// Bytes of Jacobian workspace of one group of lanes.
+template <class M = Mech>
+constexpr size_t whole_bytes() {
+  if constexpr (whole_ok<M>())
+    return sizeof(double) * NV * M::G_W;
+  else
+    return 0;
+}
+
+template <class M = Mech>
+int run_whole(prc_reactor* r, Args& a, hipStream_t s, const WholeGrid& w, double* J) {
+  if constexpr (whole_ok<M>()) {
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (r->kernel_timing) {
+      while (r->kt_ev.size() < 2) {
+        hipEvent_t e = nullptr;
+        HIP_OK(hipEventCreate(&e));
+        r->kt_ev.push_back(e);
+      }
+      e0 = r->kt_ev[0];
+      e1 = r->kt_ev[1];
+    }
+    hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(64), 0, s, a.ctr, (int64_t)0, 0);
+    if (e0) HIP_OK(hipEventRecord(e0, s));
+    hipLaunchKernelGGL((k_cell<M, WHOLE_WAVES>), dim3(w.blocks), dim3(64), 0, s, a,
+                       CellArgs{J, w.gpw});
+    HIP_OK(hipGetLastError());
+    if (e1) HIP_OK(hipEventRecord(e1, s));
+    HIP_OK(hipStreamSynchronize(s));
+    r->kt_ms[0] = r->kt_ms[1] = r->kt_ms[2] = 0.0;
+    r->kt_launches = 0;
+    if (e0) {
+      float t = 0.0f;
+      HIP_OK(hipEventElapsedTime(&t, e0, e1));
+      r->kt_ms[0] = t;
+      r->kt_launches = 1;
+    }
+  }
+  return PRC_OK;
+}
+
 // Integrator parameters, diagnostics and counters of the handle into the call's argument block.
 void fill_params(const prc_reactor* r, Args& a, unsigned long long* ctr) {
   a.prm.rtol = r->rtol;
@@ -574,7 +681,25 @@ int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_coun
     HIP_OK(hipStreamSynchronize(s));
     return PRC_OK;
   }
-  int e = ensure_workspace(r, a.ncells, has_src);
+  int e = PRC_OK;
+  if (WHOLE && !r->lu_fp32) {
+    WholeGrid w;
+    e = whole_grid(r, a.ncells, w);
+    if (e) return e;
+    if (w.groups > r->wws_groups) {
+      if (r->wws) (void)hipFree(r->wws);
+      r->wws = nullptr;
+      r->wws_groups = 0;
+      if (hipMalloc(&r->wws, whole_bytes() * w.groups) != hipSuccess) return PRC_ENOMEM;
+      r->wws_groups = w.groups;
+    }
+    a.has_src = has_src ? 1 : 0;
+    a.test_lu_fail = r->test_lu_fail;
+    r->whole_cells = (int64_t)w.blocks * w.gpw;
+    return run_whole(r, a, s, w, r->wws);
+  }
+  r->whole_cells = 0;
+  e = ensure_workspace(r, a.ncells, has_src);
   if (e) return e;
   const Args& L = r->ws_layout;
   a.st[0] = L.st[0];
@@ -590,8 +715,20 @@ int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_coun
   a.ring = L.ring;
   a.has_src = has_src ? 1 : 0;
   a.test_lu_fail = r->test_lu_fail;
-  return r->lu_fp32 ? run_batched<float>(r, a, s, r->d_args, r->d_ctr, true)
-                    : run_batched<double>(r, a, s, r->d_args, r->d_ctr, true);
+  return run_queue(r, a, s, r->d_args, r->d_ctr, true);
+}
+
+// prc_model_eval with one cell per group of lanes; false: the mechanism has no lane-group tables.
+template <class M = Mech>
+bool launch_model(int64_t nc, double t, const double* y, const double* rhoe0, const double* rhoesrc,
+                  const double* src, double* ydot, double* J, hipStream_t s) {
+  if constexpr (whole_ok<M>()) {
+    constexpr int CPB = 64 / M::G_W;  // cells per block
+    hipLaunchKernelGGL(k_model_cell<M>, dim3((unsigned)((nc + CPB - 1) / CPB)), dim3(64), 0, s, nc,
+                       t, y, rhoe0, rhoesrc, src, ydot, J);
+    return true;
+  }
+  return false;
 }
 
 int ensure_init(prc_reactor* r) {
@@ -646,6 +783,11 @@ void release(prc_reactor* r) {
   if (r->pws) (void)hipFree(r->pws);
   r->pws = nullptr;
   r->pws_cells = 0;
+  if (r->wws) (void)hipFree(r->wws);
+  r->wws = nullptr;
+  r->wws_groups = 0;
+  r->whole_blocks = 0;
+  r->whole_cells = 0;
   r->graph_lu_fp32 = -1;
   r->ncu = 0;
   r->initialised = false;
@@ -867,8 +1009,8 @@ int prc_get_param_int(prc_reactor* r, const char* key, int* v) {
     *v = r->shape.refine;
   else if (!std::strcmp(key, "prc.max_slots"))
     *v = r->max_slots;
-  else if (!std::strcmp(key, "prc.slots"))  // slots of the current batched workspace
-    *v = (int)r->ws_cap;
+  else if (!std::strcmp(key, "prc.slots"))  // slots of the batched workspace, or cells in flight
+    *v = (int)(r->whole_cells ? r->whole_cells : r->ws_cap);
   else
     return PRC_EINVAL;
   return PRC_OK;
@@ -968,16 +1110,8 @@ int prc_react_flat_noalloc(prc_reactor* r, double* rY, const double* rYsrc, doub
   const size_t o_ws = o_ctr + align_up(CT_COUNT * sizeof(unsigned long long));
   const bool has_src = rYsrc != nullptr;
   Args a{};
-  const size_t per64 = workspace_layout(a, nullptr, 64, r->lu_fp32, has_src);
-  if (o_ws + per64 > NOALLOC_SCRATCH_BYTES) return PRC_ENOMEM;  // not even 64 slots fit
-  int64_t C = 64;
-  while (o_ws + workspace_layout(a, nullptr, C + 64, r->lu_fp32, has_src) <= NOALLOC_SCRATCH_BYTES &&
-         C < ncells)
-    C += 64;
-  workspace_layout(a, base + o_ws, C, r->lu_fp32, has_src);
   Args* dargs = reinterpret_cast<Args*>(base);
   unsigned long long* dctr = reinterpret_cast<unsigned long long*>(base + o_ctr);
-  fill_params(r, a, dctr);
   auto view = [&](const double* p) {
     A4 v{};
     v.p = const_cast<double*>(p);
@@ -1002,8 +1136,30 @@ int prc_react_flat_noalloc(prc_reactor* r, double* rY, const double* rYsrc, doub
   a.dt = *dt_react;
   a.has_src = has_src ? 1 : 0;
   a.test_lu_fail = r->test_lu_fail;
-  e = r->lu_fp32 ? run_batched<float>(r, a, s, dargs, dctr, false)
-                 : run_batched<double>(r, a, s, dargs, dctr, false);
+  fill_params(r, a, dctr);
+  if (WHOLE && !r->lu_fp32) {
+    // the Jacobians of the cells in flight in the scratch array; a grid it cannot hold is cut
+    WholeGrid w;
+    e = whole_grid(r, ncells, w);
+    if (e) return e;
+    const int64_t fit = (int64_t)((NOALLOC_SCRATCH_BYTES - o_ws) / whole_bytes()) / whole_gpw();
+    w.blocks = (int)std::min<int64_t>(w.blocks, fit);
+    if (w.blocks < 1) return PRC_ENOMEM;
+    e = run_whole(r, a, s, w, reinterpret_cast<double*>(base + o_ws));
+    if (e) return e;
+    HIP_OK(hipMemcpyAsync(r->d_ctr, dctr, CT_COUNT * sizeof(unsigned long long),
+                          hipMemcpyDeviceToDevice, s));
+    *time += *dt_react;
+    return PRC_OK;
+  }
+  const size_t per64 = workspace_layout(a, nullptr, 64, r->lu_fp32, has_src);
+  if (o_ws + per64 > NOALLOC_SCRATCH_BYTES) return PRC_ENOMEM;  // not even 64 slots fit
+  int64_t C = 64;
+  while (o_ws + workspace_layout(a, nullptr, C + 64, r->lu_fp32, has_src) <= NOALLOC_SCRATCH_BYTES &&
+         C < ncells)
+    C += 64;
+  workspace_layout(a, base + o_ws, C, r->lu_fp32, has_src);
+  e = run_queue(r, a, s, dargs, dctr, false);
   if (e) return e;
   // prc_last_failures reads the handle's counters
   HIP_OK(hipMemcpyAsync(r->d_ctr, dctr, CT_COUNT * sizeof(unsigned long long),
@@ -1141,9 +1297,19 @@ int prc_autotune(prc_reactor* r, int64_t ncells, const double* rY, const double*
   {
     // occupancy-derived defaults are the starting point
     Shape base = r->shape;
-    if (!r->ncu) rc = r->lu_fp32 ? occupancy_setup<float>(r) : occupancy_setup<double>(r);
+    if (!r->ncu) rc = queue_occupancy(r);
     if (!rc) rc = measure(best);
     Shape cur = r->shape;
+    if (WHOLE && !r->lu_fp32) {
+      // one launch whose grid follows from the occupancy: no shape to search
+      r->diag = diag;
+      r->diag_cap = diag_cap;
+      (void)hipEventDestroy(e0);
+      (void)hipEventDestroy(e1);
+      (void)hipFree(work);
+      if (best_ms) *best_ms = best;
+      return rc;
+    }
     // kernel pair first (each one cell per lane or per group), at occupancy-derived block counts
     for (int c = 0; c <= (COOP ? 3 : 0) && !rc; ++c) {
       Shape trial = cur;
@@ -1159,7 +1325,7 @@ int prc_autotune(prc_reactor* r, int64_t ncells, const double* rY, const double*
       }
     }
     r->shape = cur;
-    if (!rc) rc = r->lu_fp32 ? occupancy_setup<float>(r) : occupancy_setup<double>(r);
+    if (!rc) rc = queue_occupancy(r);
     const int on = r->occ_newton, oj = r->occ_jac, ol = r->occ_lu, ot = r->occ_tail;
     // tail graph thresholds relative to the sample (slots in use when the tail graph takes over)
     const int nt = (int)std::min<int64_t>(ncells, 1 << 30);
@@ -1397,14 +1563,7 @@ int prc_model_eval(int64_t nc, double t, const double* y, const double* rhoe0,
   if (nc == 0) return PRC_OK;
   hipStream_t s = (hipStream_t)stream;
   if (cooperative) {
-    if constexpr (COOP)
-      hipLaunchKernelGGL(k_model_group<64>, dim3((unsigned)((nc + 1) / 2)), dim3(64), 0, s, nc, t,
-                         y, rhoe0, rhoesrc, rYsrc, ydot, J);
-    else if constexpr (COOP64)
-      hipLaunchKernelGGL((k_model_group<64, GroupModel<Mech, 64>>), dim3((unsigned)nc), dim3(64), 0,
-                         s, nc, t, y, rhoe0, rhoesrc, rYsrc, ydot, J);
-    else
-      return PRC_EINVAL;  // this mechanism has no cooperative kernels
+    if (!launch_model(nc, t, y, rhoe0, rhoesrc, rYsrc, ydot, J, s)) return PRC_EINVAL;
   } else
     hipLaunchKernelGGL(k_model_lane, dim3((unsigned)((nc + 63) / 64)), dim3(64), 0, s, nc, t, y,
                        rhoe0, rhoesrc, rYsrc, ydot, J);

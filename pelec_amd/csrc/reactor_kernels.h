@@ -14,6 +14,7 @@
 #include "bdf_cell.h"
 #include "rk64.h"
 #include "adjoint.h"
+#include "whole_cell.h"
 
 namespace {
 
@@ -842,6 +843,262 @@ __global__ void __launch_bounds__(BS) k_newton_g(const Args* __restrict__ ap, in
   }
 }
 
+// ------------------------------------------------------------------ whole-cell form
+// One group of lanes integrates a cell from start to end with its state in registers
+// (whole_cell.h). The groups of a persistent grid take cells from a queue (CT_NEXT) until it is empty.
+template <class M>
+constexpr bool whole_ok() {
+  if constexpr (M::G_OK)
+    return M::G_W >= M::NSP + 1 && M::T_NSETS <= M::G_W;
+  else
+    return false;
+}
+constexpr bool WHOLE = whole_ok<Mech>();
+
+// What a group's next right-hand side is for.
+enum CellPhase : int { CP_FETCH, CP_F0, CP_HIN, CP_NEWTON, CP_RESTART, CP_SETUP, CP_IDLE };
+
+struct CellArgs {
+  double* J;  // G * n doubles per group of the grid: the cells' Jacobians
+  int gpw;    // groups of each wave that take cells
+};
+
+// A block is one wave: its 64 / G groups run in lockstep, every group on a cell of its own. Each turn
+// of the loop evaluates one right-hand side per group -- f(t0, y0), an evaluation of the
+// initial-step iteration, a Newton iteration or an order-1 restart -- so the kinetics are one copy
+// of code that all groups of a wave run together whatever phase their cells are in.
+template <class M, int MINW>
+__global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs ca) {
+  using K = GroupKin<M>;
+  constexpr int G = K::G;
+  using Grp = Group<G>;
+  constexpr int GPW = 64 / G;
+  __shared__ __attribute__((aligned(16))) double lds[GPW * K::WORDS];
+  __shared__ CellState cst[GPW];
+  const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
+  lds_double* sh = lds_ptr(lds) + gid * K::WORDS;
+  CellState& cs = cst[gid];
+  BdfScalars& S = cs.S;
+  double* Jg = ca.J + ((int64_t)blockIdx.x * GPW + gid) * (int64_t)(NV * G);
+  const double tm = M::G_TMID[l];
+  const bool in = l < NV;
+  double z[BDF_QMAX + 1], ac = 0.0, ew = 0.0, Mi[NV];
+#pragma unroll
+  for (int j = 0; j <= BDF_QMAX; ++j) z[j] = 0.0;
+#pragma unroll
+  for (int c = 0; c < NV; ++c) Mi[c] = 0.0;
+  const RegV<NV, G> v{{}, z, ac, ew, l < NV ? a.prm.atolv[l] : 1.0};
+  int ph = gid < ca.gpw ? CP_FETCH : CP_IDLE;
+  int kap = 0;
+  int64_t g = 0;
+  double rhoe0 = 0.0, rhoesrc = 0.0, srcl = 0.0;
+  for (;;) {
+    while (ph == CP_FETCH) {
+      unsigned long long nx = 0;
+      if (l == 0) nx = atomicAdd(&a.ctr[CT_NEXT], 1ull);
+      g = (int64_t)__shfl(nx, 0, G);
+      if (g >= a.ncells) {
+        ph = CP_IDLE;
+        break;
+      }
+      int64_t loc;
+      const BoxDev& b = box_of(a, g, loc);
+      int i, j, k;
+      cell_ijk(b, loc, i, j, k);
+      if (b.mask.p && b.mask.at(i, j, k) == 0) {
+        if (l == 0) {
+          if (b.FC.p) b.FC.at(i, j, k, 0) = 0.0;
+          write_diag(a, g, CELL_OK, nullptr);
+        }
+        continue;
+      }
+      const double y0 = l < NSP ? b.rY.at(i, j, k, l) : l == NSP ? b.T.at(i, j, k, 0) : 0.0;
+      rhoe0 = b.rE.at(i, j, k, 0);
+      rhoesrc = b.rEsrc.p ? b.rEsrc.at(i, j, k, 0) : 0.0;
+      srcl = b.rYsrc.p && l < NSP ? b.rYsrc.at(i, j, k, l) : 0.0;
+      const double rho = Grp::sum(l < NSP ? y0 : 0.0);
+      if (!(rho > 0.0) || !(Grp::bcast(y0, NSP) > 0.0) || !(a.dt > 0.0)) {
+        if (l == 0) {
+          atomicAdd(&a.ctr[CT_FAILED], 1ull);
+          if (b.FC.p) b.FC.at(i, j, k, 0) = 0.0;
+          write_diag(a, g, CELL_BADINPUT, nullptr);
+        }
+        continue;
+      }
+      Grp::sync();
+      scalars_reset(S, a.prm.qmax);
+      z[0] = y0;
+#pragma unroll
+      for (int e = 1; e <= BDF_QMAX; ++e) z[e] = 0.0;
+      ac = 0.0;
+      set_ewt<NV>(v, a.prm);
+      ph = CP_F0;
+    }
+    if (__ballot(ph != CP_IDLE) == 0ull) break;
+    bool need_setup = false;
+    int status = -1;  // < 0 running, else the cell's final status
+    if (ph == CP_SETUP) {
+      need_setup = true;
+    } else if (ph != CP_IDLE) {
+      double yl = z[0], t = S.tn;
+      if (ph == CP_NEWTON) {
+        if (S.m > 0)
+          yl += ac;
+        else
+          ac = 0.0;
+      } else if (ph == CP_HIN) {
+        yl += cs.hg * z[1];
+        t += cs.hg;
+      }
+      LaneVal f;
+      f.x = K::rhs(t, yl, l, rhoe0, rhoesrc, srcl, tm, sh);
+      S.nfe++;
+      if (ph == CP_NEWTON) {
+        const int r = newton_correct<NV>(S, v, f, [&](LaneVal& b) {
+          b.x = K::solve(Mi, kap, b.x, l, sh);
+        });
+        if (r == 2) {
+          S.convfail = 2;  // stale Jacobian: rebuild and restart the Newton iteration
+          S.m = 0;
+          need_setup = true;
+        } else if (r != 1) {
+          bool attempt = false;
+          if (r == 3) {
+            const int e = conv_fail<NV>(S, v);
+            if (e >= 0)
+              status = e;
+            else
+              attempt = true;
+          } else {
+            const double dsm = S.acnrm * S.tq[2];
+            if (dsm <= 1.0) {
+              finish_step<NV>(S, v, dsm, a.prm.qmax);
+              if (reached_tstop(S, a.dt))
+                status = CELL_OK;
+              else if (S.nst >= a.prm.max_steps)
+                status = CELL_MAXSTEPS;
+              else
+                need_setup = next_attempt<NV>(S, v, a.prm, a.dt);
+            } else {
+              const int e = error_test_fail<NV>(S, v, dsm, a.prm.qmax);
+              if (e >= 0)
+                status = e;
+              else if (e == -2)
+                ph = CP_RESTART;  // z_1 = h f(tn, z_0) with the next evaluation
+              else
+                attempt = true;
+            }
+          }
+          if (attempt) need_setup = begin_attempt<NV>(S, v, a.dt);
+        }
+      } else if (ph == CP_RESTART) {
+        z[1] = S.h * f.x;
+        need_setup = begin_attempt<NV>(S, v, a.dt);
+        ph = CP_NEWTON;
+      } else {
+        // f(t0, y0), then cvHin's iteration (hin), one evaluation per turn
+        bool have_h = false;
+        double h0 = 0.0;
+        if (ph == CP_F0) {
+          z[1] = f.x;  // 0 on lanes without a component
+          const double tdist = a.dt - S.tn;
+          const double hlb = 100.0 * cv::UROUND * fmax(fabs(S.tn), fabs(a.dt));
+          const double hub_inv = Grp::max(fabs(z[1]) / (0.1 * fabs(z[0]) + 1.0 / ew));
+          double hub = 0.1 * tdist;
+          if (hub * hub_inv > 1.0) hub = 1.0 / hub_inv;
+          h0 = sqrt(hlb * hub);
+          have_h = hub < hlb;
+          cs.hg = h0;
+          cs.hub = hub;
+          cs.hlb = hlb;
+          cs.count = 1;
+          ph = CP_HIN;
+        } else {
+          const double hg = cs.hg, hub = cs.hub;
+          const double w = (f.x - z[1]) / hg * ew;
+          const double yddnrm = sqrt(Grp::sum(w * w) / NV);
+          double hnew = (yddnrm * hub * hub > 2.0) ? sqrt(2.0 / yddnrm) : sqrt(hg * hub);
+          const double hrat = hnew / hg;
+          bool last = cs.count == 4 || (hrat > 0.5 && hrat < 2.0);
+          if (!last && cs.count > 1 && hrat > 2.0) {
+            hnew = hg;
+            last = true;
+          }
+          if (last) {
+            h0 = fmin(fmax(0.5 * hnew, cs.hlb), hub);
+            have_h = true;
+          } else {
+            cs.hg = hnew;
+            cs.count++;
+          }
+        }
+        if (have_h) {
+          S.h = h0;
+          if ((S.tn + S.h - a.dt) * S.h > 0.0) S.h = (a.dt - S.tn) * (1.0 - 4.0 * cv::UROUND);
+          S.hscale = S.h;
+          S.hprime = S.h;
+          z[1] *= S.h;
+          step_prologue<NV>(S, v, a.prm.qmax);
+          need_setup = begin_attempt<NV>(S, v, a.dt);  // nst == 0: a set-up with a Jacobian
+          ph = CP_NEWTON;
+        }
+      }
+    }
+    if (need_setup) {
+      if (jac_decide(S)) K::jac(S.tn, z[0], l, rhoe0, rhoesrc, srcl, tm, sh, Jg);
+      const double gamma = S.gamma;
+      // (the columns' addresses are formed here, not kept across the cell loop)
+      const double* Jl = Jg + after(l, gamma);
+#pragma unroll
+      for (int c = 0; c < NV; ++c) {
+        const double m = in ? -gamma * K::load_l2(Jl + c * G) : 0.0;
+        Mi[c] = c == l ? m + 1.0 : m;  // I - gamma J
+      }
+      Grp::sync();
+      int ier = K::invert(Mi, l, kap, sh);
+      if (a.test_lu_fail && ier == 0) ier = 1;
+      after_setup(S);
+      ph = CP_NEWTON;
+      if (ier != 0) {  // singular: CVODE's convergence-failure handling
+        const int e = conv_fail<NV>(S, v);
+        if (e >= 0) {
+          status = e;
+        } else {
+          begin_attempt<NV>(S, v, a.dt);
+          ph = CP_SETUP;
+        }
+      }
+    }
+    if (status >= 0) {
+      int64_t loc;
+      const BoxDev& b = box_of(a, g, loc);
+      int i, j, k;
+      cell_ijk(b, loc, i, j, k);
+      if (status == CELL_OK) {
+        const double yl = z[0];
+        const double irho = 1.0 / Grp::sum(l < NSP ? yl : 0.0);
+        const double rEn = rhoe0 + a.dt * rhoesrc;
+        double ec[6], ek, cvk;
+        const double Tn = K::T_from_e(rEn * irho, l < NSP ? yl * irho : 0.0, l,
+                                      Grp::bcast(yl, NSP), tm, ec, ek, cvk);
+        if (l < NSP) b.rY.at(i, j, k, l) = yl;
+        if (l == 0) {
+          b.T.at(i, j, k, 0) = Tn;
+          b.rE.at(i, j, k, 0) = rEn;
+        }
+      } else if (l == 0) {
+        atomicAdd(&a.ctr[CT_FAILED], 1ull);
+      }
+      if (l == 0) {
+        const Counters cn = counters(S);
+        if (b.FC.p) b.FC.at(i, j, k, 0) = (double)cn.nfe;
+        write_diag(a, g, status, &cn);
+      }
+      ph = CP_FETCH;
+    }
+  }
+}
+
 // The compaction check a graph makes between two iterations (the host makes the same check between
 // replays): compact when fewer than pct % of the slots in use are alive, more than 4096 slots are
 // in use, and no cell of the call waits for a slot (refills stay with the host).
@@ -1302,7 +1559,7 @@ __global__ void eos_rty2hi(int64_t nc, const double* T, double* hi) {
   for (int s = 0; s < NSP; ++s) hi[s * nc + c] = ek[s] + 8.31446261815324e7 * t * Mech::IW[s];
 }
 
-__global__ void eos_rty2wdot(int64_t nc, const double* rho, const double* T, const double* Y,
+__global__ void __launch_bounds__(256) eos_rty2wdot(int64_t nc, const double* rho, const double* T, const double* Y,
                              double* wdot) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= nc) return;
@@ -1334,24 +1591,27 @@ __global__ void __launch_bounds__(64) k_model_lane(int64_t nc, double t, const d
   if (J) Model::template jac<double>(t, yy, rhoe0[c], r1, src ? src + c : nullptr, nc, J + c * (int64_t)(NV * NV));
 }
 
-// ... or one cell per G-lane group (GroupModel), BS / G per block.
-template <int BS, class GM = GModel>
-__global__ void __launch_bounds__(BS) k_model_group(int64_t nc, double t, const double* y,
-                                                     const double* rhoe0, const double* rhoesrc,
-                                                     const double* src, double* ydot, double* J) {
-  constexpr int G = GM::GS;
-  constexpr int CPB = BS / G;
-  __shared__ double lds[CPB * GM::JAC_WORDS];
-  const int64_t c = (int64_t)blockIdx.x * CPB + threadIdx.x / G;
-  const int l = threadIdx.x & (G - 1);
+// ... or one cell per group of lanes (GroupKin, the whole-cell form's kinetics), 64 / G per block.
+template <class M>
+__global__ void __launch_bounds__(64) k_model_cell(int64_t nc, double t, const double* y,
+                                                    const double* rhoe0, const double* rhoesrc,
+                                                    const double* src, double* ydot, double* J) {
+  using K = GroupKin<M>;
+  constexpr int G = K::G;
+  __shared__ __attribute__((aligned(16))) double lds[64 / G * K::WORDS];
+  const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
+  const int64_t c = (int64_t)blockIdx.x * (64 / G) + gid;
   if (c >= nc) return;
-  double* sh = lds + (threadIdx.x / G) * GM::JAC_WORDS;
+  lds_double* sh = lds_ptr(lds) + gid * K::WORDS;
   const double yl = l < NV ? y[l * nc + c] : 0.0;
   const double srcl = (src && l < NSP) ? src[l * nc + c] : 0.0;
   const double r1 = rhoesrc ? rhoesrc[c] : 0.0;
-  const double f = GM::rhs(t, yl, l, rhoe0[c], r1, srcl, sh);
+  const double tm = M::G_TMID[l];
+  const double f = K::rhs(t, yl, l, rhoe0[c], r1, srcl, tm, sh);
   if (l < NV) ydot[l * nc + c] = f;
-  if (J) GM::jac(t, yl, l, rhoe0[c], r1, srcl, sh, J + c * (int64_t)(NV * NV));
+  if (J)
+    K::template jac<false, 1, NV>(t, yl, l, rhoe0[c], r1, srcl, tm, sh,
+                                  J + c * (int64_t)(NV * NV));
 }
 
 }  // namespace

@@ -649,6 +649,149 @@ class Gen:
         arr("T_CSR_SLOT", "int", slots, [len(flat) + pad, 6])
         arr("T_CSR_EFF", "int", [eff[j] for j, _ in flat] + [-1] * pad, [len(flat) + pad])
 
+    # ------------------------------------------------------------------ lane-group tables
+    def emit_group_tables(self):
+        """The mechanism as data in the order the lanes of a group read it (whole_cell.h): species k
+        on lane k, reaction at position p = G r + l of T_RORD on lane l in round r, every table
+        [...][lane] so that a group's loads are contiguous. Entries of absent lanes and positions are
+        neutral: species slot N (concentration and exp(g/RT) of 1), coefficient 0."""
+        if self.table_form_issue() is not None:
+            self.w("  static constexpr bool G_OK = false;")
+            return
+        N, R, rx, sp = self.N, self.R, self.m.reactions, self.m.species
+        for r in rx:
+            sides = (r.reactants, r.products) if r.reversible else (r.reactants,)
+            nu = list(self.nu_of(r).values())
+            if any(sum(s.values()) > 3 for s in sides) or any(v != int(v) for v in nu) or N > 63:
+                self.w("  static constexpr bool G_OK = false;")
+                return
+        w = self.w
+        n = N + 1
+        G = 16 if n <= 16 else 32 if n <= 32 else 64
+        RR = (R + G - 1) // G
+        P = RR * G
+
+        def arr(name, ctype, vals, shape):
+            dims = "".join(f"[{d}]" for d in shape)
+
+            def fmt(v):
+                if isinstance(v, list):
+                    return "{" + ", ".join(fmt(x) for x in v) + "}"
+                return f(v) if ctype == "double" else f"{int(v)}ull" if "64" in ctype else str(int(v))
+            w(f"  alignas(16) static constexpr {ctype} {name}{dims} = {fmt(vals)};")
+
+        def lanes(rows, width, pad):
+            """rows[lane][branch][coef] -> [branch][coef pair][lane][2]"""
+            full = [list(map(list, r)) for r in rows] + [[[pad] * width] * 2] * (G - len(rows))
+            for k in range(len(rows)):
+                full[k] = [c + [0.0] * (width - len(c)) for c in full[k]]
+            return [[[full[k][b][i:i + 2] for k in range(G)] for i in range(0, width, 2)] for b in (0, 1)]
+
+        w("  // ---- lane-group tables (whole_cell.h)")
+        w("  static constexpr bool G_OK = true;")
+        w(f"  static constexpr int G_W = {G};   // lanes per cell")
+        w(f"  static constexpr int G_RR = {RR};  // reaction rounds")
+        arr("G_TMID", "double", [s.Tmid for s in sp] + [1000.0] * (G - N), [G])
+        arr("G_WT", "double", [s.W for s in sp] + [0.0] * (G - N), [G])
+        arr("G_IWT", "double", [1.0 / s.W for s in sp] + [0.0] * (G - N), [G])
+        gco = [[[a[0] - a[6], -a[1] / 2, -a[2] / 6, -a[3] / 12, -a[4] / 20, a[0], a[5]]
+                for a in (s.low, s.high)] for s in sp]
+        hco = [[[a[0], a[1] / 2, a[2] / 3, a[3] / 4, a[4] / 5, a[5]] for a in (s.low, s.high)]
+               for s in sp]
+        arr("G_E", "double", lanes([self.ecoef[k] for k in range(N)], 6, 0.0), [2, 3, G, 2])
+        arr("G_G", "double", lanes(gco, 8, 0.0), [2, 4, G, 2])
+        arr("G_H", "double", lanes(hco, 6, 0.0), [2, 3, G, 2])
+        # efficiency sets: the species with an efficiency other than 1, set s on lane s
+        sets = sorted(self.effsets.items(), key=lambda kv: kv[1])
+        sparse = [[(m, a - 1.0) for m, a in enumerate(key) if a != 1.0] for key, _ in sets]
+        MN = max([len(x) for x in sparse] + [0])
+        w(f"  static constexpr int G_MN = {MN};")
+        sparse = [x + [(N, 0.0)] * (MN - len(x)) for x in sparse]
+        sparse += [[(N, 0.0)] * MN for _ in range(G - len(sparse))]
+        m1 = max(MN, 1)
+        sparse = [x + [(N, 0.0)] * (m1 - MN) for x in sparse]
+        arr("G_MI", "int", [[sparse[s][e][0] for s in range(G)] for e in range(m1)], [m1, G])
+        arr("G_MD", "double", [[sparse[s][e][1] for s in range(G)] for e in range(m1)], [m1, G])
+        # reactions in lane order (T_RORD: falloff, then three-body, then elementary)
+        kind_id = {"elementary": 0, "three-body": 1, "falloff": 2}
+        order = sorted(range(R), key=lambda j: (-kind_id[rx[j].kind], j))
+        pos = {j: p for p, j in enumerate(order)}
+        ab, ear, pack, low, troe, troek = [], [], [], [], [], []
+        for j in order:
+            r = rx[j]
+            ab.append([r.A, r.b])
+            ear.append(r.Ea_R)
+            def slots(side):
+                s = [k for k, v in sorted(side.items()) for _ in range(int(v))]
+                return s + [N] * (3 - len(s))
+            sl = slots(r.reactants) + (slots(r.products) if r.reversible else [N] * 3)
+            dnu = int(sum(r.products.values()) - sum(r.reactants.values())) if r.reversible else 0
+            eff = self.effsets[tuple(r.efficiencies)] if r.efficiencies is not None else 0
+            v = sum(k << (8 * i) for i, k in enumerate(sl)) | eff << 48 | kind_id[r.kind] << 56
+            pack.append(v | (1 << 58 if r.reversible else 0) | (dnu + 2) << 59)
+            if r.kind == "falloff":
+                A0, b0, E0 = r.low
+                low.append([math.log(A0) - math.log(r.A), b0 - r.b, E0 - r.Ea_R])
+                if r.troe is None:
+                    troek.append(0)
+                    troe.append([0.0] * 8)
+                else:
+                    a, T3, T1 = r.troe[:3]
+                    T2 = r.troe[3] if len(r.troe) > 3 else 0.0
+                    troek.append(1)
+                    troe.append([1.0 - a, -1.0 / T3, a, -1.0 / T1, T2,
+                                 1.0 if len(r.troe) > 3 else 0.0, -(1.0 - a) / T3, -a / T1])
+        NFO, NTB = len(low), sum(r.kind == "three-body" for r in rx)
+        none = sum(N << (8 * i) for i in range(6)) | 2 << 59
+        ab += [[0.0, 0.0]] * (P - R)
+        ear += [0.0] * (P - R)
+        pack += [none] * (P - R)
+        w(f"  static constexpr int G_NFO = {NFO};  // falloff reactions: positions 0..G_NFO-1")
+        w(f"  static constexpr int G_NTB = {NFO + NTB};  // reactions with a third body")
+        arr("G_RORD", "int", order + [-1] * (P - R), [P])
+        arr("G_RA", "double", ab, [P, 2])
+        arr("G_RE", "double", ear, [P])
+        arr("G_RP", "uint64_t", pack, [P])
+        q = max(NFO, 1)
+        low = low or [[0.0] * 3]
+        troe = troe or [[0.0] * 8]
+        arr("G_LOW", "double", [[x[i] for x in low] for i in range(3)], [3, q])
+        arr("G_TROE", "double", [[x[i] for x in troe] for i in range(8)], [8, q])
+        arr("G_TROEK", "int", troek or [0], [q])
+        # production rates: each species' (reaction, nu) list cut into chunks of at most L entries,
+        # one chunk per lane; L the smallest for which all chunks fit the group
+        rows = [[] for _ in range(N)]
+        for p, j in enumerate(order):
+            for k, v in sorted(self.nu_of(rx[j]).items()):
+                if v != 0:
+                    rows[k].append((p, int(v)))
+        L = 1
+        while sum((len(x) + L - 1) // L for x in rows) > G:
+            L += 1
+        L4 = (L + 3) // 4
+        chunks, begin = [], []
+        for x in rows:
+            begin.append(len(chunks) | ((len(x) + L - 1) // L) << 8)
+            chunks += [x[i:i + L] for i in range(0, len(x), L)]
+        chunks += [[]] * (G - len(chunks))
+        entry = lambda c, i: (c[i][0] * 8 | (c[i][1] & 0xff) << 24) if i < len(c) else P * 8
+        sgn = lambda v: v - (1 << 32) if v >= 1 << 31 else v
+        w(f"  static constexpr int G_L4 = {L4};")
+        w(f"  static constexpr int G_CMAX = {max(b >> 8 for b in begin)};  // chunks of a species")
+        arr("G_GE", "int", [[[sgn(entry(c, 4 * i + u)) for u in range(4)] for c in chunks]
+                            for i in range(L4)], [L4, G, 4])
+        arr("G_CP", "int", begin + [0] * (G - N), [G])
+        # Jacobian rows: per round, each species' entries (position in the round, nu)
+        offs, ent = [0], []
+        for r in range(RR):
+            own = [[(p - G * r, v) for p, v in x if p // G == r] for x in rows]
+            own += [[]] * (G - N)
+            for i in range(max(len(x) for x in own)):
+                ent.append([(x[i][0] | (x[i][1] & 0xff) << 8) if i < len(x) else 0 for x in own])
+            offs.append(len(ent))
+        arr("G_JO", "int", offs, [RR + 1])
+        arr("G_JE", "int", ent, [len(ent), G])
+
     # ------------------------------------------------------------------ top level
     def generate(self) -> str:
         m = self.m
@@ -660,6 +803,7 @@ class Gen:
         w(f"// species: {N}  reactions: {self.R}")
         w("#pragma once")
         w("#include <cmath>")
+        w("#include <cstdint>")
         w("#ifndef PELEC_MEMORY_FENCE")
         w("#define PELEC_MEMORY_FENCE() __asm__ __volatile__(\"\" ::: \"memory\")")
         w("#endif")
@@ -694,6 +838,7 @@ class Gen:
         self.emit_thermo()
         self.emit_rates()
         self.emit_tables()
+        self.emit_group_tables()
         w("};")
         w("}  // namespace mech")
         w("}  // namespace pelec")
