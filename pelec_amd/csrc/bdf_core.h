@@ -199,15 +199,34 @@ __device__ inline void scalars_reset(BdfScalars& S, int qmax) {
   S.m = S.convfail = S.nflag = S.ncf = S.nef = 0;
 }
 
+// sqrt of a finite x >= 0 without subnormal scaling, within an ulp: the hardware's reciprocal root
+// and two coupled Newton steps.
+__device__ inline double root2(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  double g = x * r, h = 0.5 * r;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, x), h, g);
+  return x == 0.0 ? 0.0 : g;
+}
 // x^(1/k), x >= 0, for the step-size factors: exp(log(x) / k) is within a few ulp of pow at a third
 // of its chain of dependent instructions (pow carries the logarithm in two doubles).
-__device__ inline double root(double x, int k) { return exp(log(x) / k); }
+__device__ inline double root(double x, int k) { return exp(log(x) * recip((double)k)); }
 // x^k for the orders' small k.
 __device__ inline double ipow(double x, int k) {
   double r = x;
 #pragma unroll
   for (int i = 2; i <= BDF_QMAX + 1; ++i) r = i <= k ? r * x : r;
   return r;
+}
+
+// x of lane j of the caller's quad of lanes.
+template <int j>
+__device__ inline double quad_read(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0x55 * j, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0x55 * j, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
 }
 
 template <int n, class V>
@@ -285,13 +304,13 @@ __device__ inline void rescale(BdfScalars& S, const V& v) {
   S.hscale = S.h;
 }
 
-// Pascal-triangle update of one component's history in registers (rows 0..q).
-__device__ inline void pascal_apply(double (&z)[BDF_QMAX + 1], int q, double sign) {
+// Pascal-triangle update of one component's history in registers, rows 0..q. Rows above q hold
+// zeros: their terms add nothing, so no row is selected on q.
+__device__ inline void pascal_apply(double (&z)[BDF_QMAX + 1], double sign) {
 #pragma unroll
   for (int k = 1; k <= BDF_QMAX; ++k)
 #pragma unroll
-    for (int j = BDF_QMAX; j >= k; --j)
-      z[j - 1] = (k <= q && j <= q) ? z[j - 1] + sign * z[j] : z[j - 1];
+    for (int j = BDF_QMAX; j >= k; --j) z[j - 1] += sign * z[j];
 }
 
 // Pascal-triangle update of the Nordsieck array (sign +1: predict, -1: undo the prediction),
@@ -314,7 +333,7 @@ __device__ inline void pascal(const V& v, int q, double sign) {
       }
     }
 #pragma unroll
-    for (int c = 0; c < K; ++c) pascal_apply(z[c], q, sign);
+    for (int c = 0; c < K; ++c) pascal_apply(z[c], sign);
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const int i = i0 + c * V::kStep;
@@ -338,41 +357,59 @@ __device__ inline void restore(BdfScalars& S, const V& v) {
   pascal<n>(v, S.q, -1.0);
 }
 
+// a[idx] of an integrator scalar array: a select chain where the record may be in registers, a
+// plain read where it is in LDS.
+template <class V, int K>
+__device__ inline double scalar_at(const double (&a)[K], int idx) {
+  if constexpr (V::kRegister)
+    return a[idx];
+  else
+    return sel(a, idx);
+}
+
+template <class V>
 __device__ inline void set_bdf(BdfScalars& S) {
   double alpha0, alpha0_hat, xi_inv, xistar_inv, hsum;
   const int q = S.q;
-  S.l[0] = S.l[1] = xi_inv = xistar_inv = 1.0;
+  const double h = S.h;
+  double l[BDF_QMAX + 2];
+  l[0] = l[1] = xi_inv = xistar_inv = 1.0;
 #pragma unroll
-  for (int i = 2; i < BDF_QMAX + 2; ++i) S.l[i] = 0.0;
+  for (int i = 2; i < BDF_QMAX + 2; ++i) l[i] = 0.0;
   alpha0 = alpha0_hat = -1.0;
-  hsum = S.h;
+  hsum = h;
   if (q > 1) {
+    // the factors of orders the method does not have are 0, and l has zeros above its degree: the
+    // products are formed without selecting on q
 #pragma unroll
     for (int j = 2; j < BDF_QMAX; ++j) {
       const bool on = j < q;
-      hsum = on ? hsum + S.tau[j - 1] : hsum;
-      const double xij = S.h / hsum;
-      xi_inv = on ? xij : xi_inv;
-      alpha0 = on ? alpha0 - 1.0 / j : alpha0;
+      hsum += on ? S.tau[j - 1] : 0.0;
+      const double xij = on ? h * recip(hsum) : 0.0;
+      alpha0 -= on ? 1.0 / j : 0.0;
 #pragma unroll
-      for (int i = j; i >= 1; --i) S.l[i] = on ? S.l[i] + S.l[i - 1] * xij : S.l[i];
+      for (int i = j; i >= 1; --i) l[i] = l[i] + l[i - 1] * xij;
     }
-    alpha0 -= 1.0 / q;
-    xistar_inv = -S.l[1] - alpha0;
-    hsum += sel(S.tau, q - 1);
-    xi_inv = S.h / hsum;
-    alpha0_hat = -S.l[1] - xi_inv;
+    const double iq = recip((double)q);
+    alpha0 -= iq;
+    xistar_inv = -l[1] - alpha0;
+    hsum += scalar_at<V>(S.tau, q - 1);
+    xi_inv = h * recip(hsum);
+    alpha0_hat = -l[1] - xi_inv;
 #pragma unroll
-    for (int i = BDF_QMAX; i >= 1; --i) S.l[i] = (i <= q) ? S.l[i] + S.l[i - 1] * xistar_inv : S.l[i];
+    for (int i = BDF_QMAX; i >= 1; --i) l[i] = l[i] + l[i - 1] * xistar_inv;
   }
-  const double lq = sel(S.l, q);
+#pragma unroll
+  for (int i = 0; i < BDF_QMAX + 2; ++i) S.l[i] = l[i];
+  const double lq = sel(l, q);
   const double A1 = 1.0 - alpha0_hat + alpha0;
   const double A2 = 1.0 + q * A1;
-  S.tq[2] = fabs(A1 / (alpha0 * A2));
-  S.tq[5] = fabs(A2 * xistar_inv / (lq * xi_inv));
+  const double tq2 = fabs(A1 * recip(alpha0 * A2));
+  S.tq[2] = tq2;
+  S.tq[5] = fabs(A2 * xistar_inv * recip(lq * xi_inv));
   if (S.qwait == 1) {
     if (q > 1) {
-      const double Cc = xistar_inv / lq;
+      const double Cc = xistar_inv * recip(lq);
       const double A3 = alpha0 + 1.0 / q;
       const double A4 = alpha0_hat + xi_inv;
       const double Cpinv = (1.0 - A4 + A3) / A3;
@@ -380,14 +417,14 @@ __device__ inline void set_bdf(BdfScalars& S) {
     } else {
       S.tq[1] = 1.0;
     }
-    hsum += sel(S.tau, q);
-    xi_inv = S.h / hsum;
-    const double A5 = alpha0 - 1.0 / (q + 1);
+    hsum += scalar_at<V>(S.tau, q);
+    xi_inv = h * recip(hsum);
+    const double A5 = alpha0 - recip((double)(q + 1));
     const double A6 = alpha0_hat - xi_inv;
-    const double Cppinv = (1.0 - A6 + A5) / A2;
-    S.tq[3] = fabs(Cppinv / (xi_inv * (q + 2) * A5));
+    const double Cppinv = (1.0 - A6 + A5) * recip(A2);
+    S.tq[3] = fabs(Cppinv * recip(xi_inv * (q + 2) * A5));
   }
-  S.tq[4] = cv::NLSCOEF / S.tq[2];
+  S.tq[4] = cv::NLSCOEF * recip(tq2);
 }
 
 // Scalar part of an order change (cvIncreaseBDF / cvDecreaseBDF): the coefficients in S.l, and
@@ -513,11 +550,12 @@ __device__ inline void step_prologue(BdfScalars& S, const V& v, int qmax) {
 // Predict, compute BDF coefficients and gamma, decide whether the Newton matrix must be
 // (re)built (cvNls). Returns true when a set-up is needed; S.convfail is its argument.
 // begin_attempt after the prediction: coefficients, gamma and the set-up decision.
+template <class V>
 __device__ inline bool attempt_setup(BdfScalars& S) {
-  set_bdf(S);
-  S.gamma = S.h / S.l[1];
+  set_bdf<V>(S);
+  S.gamma = S.h * recip(S.l[1]);
   if (S.nst == 0) S.gammap = S.gamma;
-  S.gamrat = (S.nst > 0) ? S.gamma / S.gammap : 1.0;
+  S.gamrat = (S.nst > 0) ? S.gamma * recip(S.gammap) : 1.0;
   S.convfail = (S.nflag == 0 || S.nflag == 2) ? 0 : 1;
   S.m = 0;
   return (S.nflag == 1) || (S.nflag == 2) || (S.nst == 0) || (S.nst >= S.nstlp + cv::MSBP) ||
@@ -527,15 +565,16 @@ __device__ inline bool attempt_setup(BdfScalars& S) {
 template <int n, class V>
 __device__ inline bool begin_attempt(BdfScalars& S, const V& v, double tstop) {
   predict<n>(S, v, tstop);
-  return attempt_setup(S);
+  return attempt_setup<V>(S);
 }
 
 // set_ewt, step_prologue and begin_attempt after a successful step, in one pass over the
 // components: a component's error weight from z_0, then its order change, rescaling and
 // prediction -- the operations of the three calls, in their order, on one component's history
-// in registers. Returns begin_attempt's set-up decision.
+// in registers. next_predict leaves begin_attempt's coefficients and set-up decision to the caller
+// (attempt_setup); next_attempt takes them too.
 template <int n, class V>
-__device__ inline bool next_attempt(BdfScalars& S, const V& v, const BdfParams& prm,
+__device__ inline void next_predict(BdfScalars& S, const V& v, const BdfParams& prm,
                                     double tstop) {
   // step_prologue
   S.saved_t = S.tn;
@@ -582,14 +621,18 @@ __device__ inline bool next_attempt(BdfScalars& S, const V& v, const BdfParams& 
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const int i = i0 + c * V::kStep;
-      const double ew = i < n ? 1.0 / (prm.rtol * fabs(z[c][0]) + atol_at(v, prm, i)) : 0.0;
+      const double ew = i < n ? recip(prm.rtol * fabs(z[c][0]) + atol_at(v, prm, i)) : 0.0;
       order_apply(kind, S.l, A1, q0, L0, za[c], z[c]);
       if (resc) {
 #pragma unroll
         for (int j = 1; j <= BDF_QMAX; ++j)
           if (j <= q) z[c][j] = z[c][j] * f[j];
       }
-      pascal_apply(z[c], q, 1.0);
+      if (q < q0) {  // the row an order decrease leaves behind
+#pragma unroll
+        for (int j = 1; j <= BDF_QMAX; ++j) z[c][j] = j <= q ? z[c][j] : 0.0;
+      }
+      pascal_apply(z[c], 1.0);
       if (i < n) {
         v.E(i) = ew;
 #pragma unroll
@@ -600,7 +643,13 @@ __device__ inline bool next_attempt(BdfScalars& S, const V& v, const BdfParams& 
     component_fence<V>();
   }
   group_join<V>();
-  return attempt_setup(S);
+}
+
+template <int n, class V>
+__device__ inline bool next_attempt(BdfScalars& S, const V& v, const BdfParams& prm,
+                                    double tstop) {
+  next_predict<n>(S, v, prm, tstop);
+  return attempt_setup<V>(S);
 }
 
 // Jacobian re-evaluation decision of the dense linear solver set-up (cvDlsSetup).
@@ -724,7 +773,8 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
         e[c] = (i < n && test) ? v.E(i) : 0.0;
         zm[c] = (i < n && up) ? col_at(v, qmax, i) : 0.0;
         if (i < n) {
-          load_hist(v, i, q, z[c]);
+          // (a register accessor's rows are all at hand: those above q keep their values)
+          load_hist(v, i, V::kRegister ? BDF_QMAX : q, z[c]);
         } else {
 #pragma unroll
           for (int j = 0; j <= BDF_QMAX; ++j) z[c][j] = 0.0;
@@ -735,8 +785,8 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
         const int i = i0 + c * V::kStep;
         if (i < n) {
 #pragma unroll
-          for (int j = 0; j <= BDF_QMAX; ++j)
-            if (j <= q) z[c][j] = z[c][j] + S.l[j] * a[c];
+          for (int j = 0; j <= BDF_QMAX; ++j)  // l_j = 0 above q
+            z[c][j] = z[c][j] + S.l[j] * a[c];
           if (down) {
             const double w = sel(z[c], q) * e[c];
             sdn += w * w;
@@ -747,7 +797,7 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
           }
 #pragma unroll
           for (int j = 0; j <= BDF_QMAX; ++j)
-            if (j <= q) v.Z(j, i) = z[c][j];
+            if (V::kRegister || j <= q) v.Z(j, i) = z[c][j];
           if (save_acor) set_col_at(v, qmax, i, a[c]);
         }
       }
@@ -766,23 +816,33 @@ __device__ inline void finish_step(BdfScalars& S, const V& v, double dsm, int qm
     S.hprime = S.h;
     S.eta = 1.0;
   } else {
-    const double etaq = 1.0 / (root(cv::BIAS2 * dsm, S.L) + cv::ADDON);
+    // eta at the order kept (x = BIAS2 dsm, k = L), and when the test runs at one order less and one
+    // more: x^(1/k) each
+    double etaq, etaqm1 = 0.0, etaqp1 = 0.0;
+    if constexpr (V::kRegister) {
+      // lane 4i + j of the group takes the j-th root; each reads the other two of its quad
+      double xd = 0.0, xu = 0.0;
+      if (test) {
+        xd = cv::BIAS1 * root2(v.sum(sdn) * (1.0 / n)) * S.tq[1];
+        xu = cv::BIAS3 * root2(v.sum(sup) * (1.0 / n)) * S.tq[3];
+      }
+      const int j = (int)(threadIdx.x & 3);
+      const double x = j == 1 ? xd : j == 2 ? xu : cv::BIAS2 * dsm;
+      const double e = recip(root(x, S.q + (j == 1 ? 0 : j == 2 ? 2 : 1)) + cv::ADDON);
+      etaq = quad_read<0>(e);
+      if (down) etaqm1 = quad_read<1>(e);
+      if (up) etaqp1 = quad_read<2>(e);
+    } else {
+      etaq = recip(root(cv::BIAS2 * dsm, S.L) + cv::ADDON);
+      if (down) etaqm1 = recip(root(cv::BIAS1 * sqrt(v.sum(sdn) / n) * S.tq[1], S.q) + cv::ADDON);
+      if (up) etaqp1 = recip(root(cv::BIAS3 * sqrt(v.sum(sup) / n) * S.tq[3], S.L + 1) + cv::ADDON);
+    }
     if (S.qwait != 0) {
       S.eta = etaq;
       S.qprime = S.q;
       set_eta(S);
     } else {
       S.qwait = 2;
-      double etaqm1 = 0.0;
-      if (down) {
-        const double ddn = sqrt(v.sum(sdn) / n) * S.tq[1];
-        etaqm1 = 1.0 / (root(cv::BIAS1 * ddn, S.q) + cv::ADDON);
-      }
-      double etaqp1 = 0.0;
-      if (up) {
-        const double dup = sqrt(v.sum(sup) / n) * S.tq[3];
-        etaqp1 = 1.0 / (root(cv::BIAS3 * dup, S.L + 1) + cv::ADDON);
-      }
       const double etam = fmax(etaqm1, fmax(etaq, etaqp1));
       if (etam < cv::THRESH) {
         S.eta = 1.0;
@@ -879,13 +939,13 @@ __device__ inline double hin(BdfScalars& S, const V& v, double tout, F&& f) {
 template <int n, class V, class FT, class Solve>
 __device__ inline int newton_correct(BdfScalars& S, const V& v, const FT& ftemp, Solve&& solve) {
   typename V::template Arr<n> tempv;
-  const double rl1 = 1.0 / S.l[1];
+  const double rl1 = recip(S.l[1]);
 #pragma unroll
   for (int i = v.c0(); i < n; i += V::kStep) tempv[i] = S.gamma * ftemp[i] - (rl1 * v.Z(1, i) + v.A(i));
   group_join<V>();
   solve(tempv);
   if (S.gamrat != 1.0) {
-    const double sc = 2.0 / (1.0 + S.gamrat);
+    const double sc = 2.0 * recip(1.0 + S.gamrat);
 #pragma unroll
     for (int i = v.c0(); i < n; i += V::kStep) tempv[i] *= sc;
   }
@@ -921,12 +981,12 @@ __device__ inline int newton_correct(BdfScalars& S, const V& v, const FT& ftemp,
     }
     group_join<V>();
   }
-  const double del = sqrt(v.sum(sdel) / n);
-  const double acn = sqrt(v.sum(sacor) / n);
-  if (S.m > 0) S.crate = fmax(cv::CRDOWN * S.crate, del / S.delp);
-  const double dcon = del * fmin(1.0, S.crate) / S.tq[4];
+  const double del = root2(v.sum(sdel) * (1.0 / n));
+  const double sac = v.sum(sacor);
+  if (S.m > 0) S.crate = fmax(cv::CRDOWN * S.crate, del * recip(S.delp));
+  const double dcon = del * fmin(1.0, S.crate) * recip(S.tq[4]);
   if (dcon <= 1.0) {
-    S.acnrm = (S.m == 0) ? del : acn;
+    S.acnrm = (S.m == 0) ? del : root2(sac * (1.0 / n));
     S.jcur = 0;
     return 0;
   }

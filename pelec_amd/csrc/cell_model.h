@@ -19,6 +19,15 @@
 
 namespace pelec {
 
+// 1 / x for normal, finite x: the hardware's estimate and two Newton steps, within 1 ulp of the
+// division at half its instructions (no scaling for subnormal operands, no special cases: 0 and
+// infinity give NaN).
+__device__ inline double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
+}
+
 // Mechanisms above this ODE size (the 53-species ones) call their production rates and rate
 // Jacobian as out-of-line device functions: the straight-line kinetics of 229-325 reactions,
 // inlined into every kernel that evaluates the model, made one library take tens of minutes to

@@ -1643,14 +1643,20 @@ struct LiDryer {
   alignas(16) static constexpr double G_RE[32] = {0.0, 24370.922007345227, 52526.05490660117, 0.0, 0.0, 0.0, 8352.941036546013, 3165.2508657072367, 1726.0429999007667, 6743.141748883461, 414.14967606948426, 148.4497623821359, 0.0, -250.1001081488866, 6029.576450382212, -819.895585929539, 1997.7815479901, 4000.595291315188, 1997.7815479901, 0.0, 4809.269081647704, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   alignas(16) static constexpr uint64_t G_RP[32] = {1009097725868311297ull, 2161737738301802759ull, 2089680135640385792ull, 936758656769786884ull, 936758656836895747ull, 936758656786564355ull, 1441161797905744641ull, 1441161797888967680ull, 1441161789282256128ull, 1441161797922522114ull, 1441161780658767363ull, 1441161797922522627ull, 1441161797855413764ull, 1441161784970511877ull, 1441161806445348358ull, 1441161806445348358ull, 1441161797872191235ull, 1441161802133604099ull, 1441161802217490180ull, 1441161802167158533ull, 1441161802167158533ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull, 1152931439017789705ull};
   alignas(16) static constexpr double G_LOW[3][2] = {{19.88299408302048, 6.009598019134351}, {-2.32, 0.0}, {264.08961118015225, -1474.4332331513833}};
-  alignas(16) static constexpr double G_TROE[8][2] = {{0.19999999999999996, 0.5}, {-9.999999999999999e+29, -9.999999999999999e+29}, {0.8, 0.5}, {-9.999999999999999e-31, -9.999999999999999e-31}, {0.0, 0.0}, {0.0, 0.0}, {-1.9999999999999995e+29, -4.9999999999999994e+29}, {-8e-31, -4.9999999999999995e-31}};
+  alignas(16) static constexpr double G_TROE[8][2] = {{-0.09691001300805639, -0.3010299956639812}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
   alignas(16) static constexpr int G_TROEK[2] = {1, 1};
-  static constexpr int G_L4 = 2;
+  static constexpr bool G_TCONST = true;  // no Fc depends on T
+  static constexpr int G_L8 = 1;
   static constexpr int G_CMAX = 3;  // chunks of a species
-  alignas(16) static constexpr int G_GE[2][16][4] = {{{-16777200, -16777160, -16777152, 16777296}, {-16777216, 16777240, -16777168, 16777296}, {16777328, 16777336, 256, 256}, {16777256, 16777280, -16777144, 16777320}, {16777376, 256, 256, 256}, {-16777216, 33554448, -16777184, -16777176}, {16777280, -16777136, -16777128, -16777088}, {-33554408, -16777184, 16777264, -16777160}, {-16777072, 256, 256, 256}, {33554440, 16777248, -16777176, 16777264}, {33554504, 33554520, 16777312, -16777112}, {-16777064, -16777056, 256, 256}, {16777216, -16777136, -16777128, -16777120}, {-33554312, 16777352, 16777360, 16777368}, {-16777208, 16777328, 16777336, -16777088}, {-16777064, -16777056, 256, 256}}, {{16777352, 256, 256, 256}, {16777312, 16777320, 256, 256}, {256, 256, 256, 256}, {16777344, 16777368, 256, 256}, {256, 256, 256, 256}, {-16777168, 16777272, 256, 256}, {-16777080, 256, 256, 256}, {-16777144, -16777120, 256, 256}, {256, 256, 256, 256}, {16777272, -16777152, 256, 256}, {16777344, 16777360, 256, 256}, {256, 256, 256, 256}, {-16777112, -33554320, 256, 256}, {16777376, 256, 256, 256}, {-16777080, -16777072, 256, 256}, {256, 256, 256, 256}}};
+  alignas(16) static constexpr uint32_t G_GE[1][16][4] = {{{4030263312, 273739840, 16781448, 16777472}, {270069760, 273739824, 275255392, 16777472}, {276303984, 16777472, 16777472, 16777472}, {272633896, 275312712, 278401152, 16777472}, {16781472, 16777472, 16777472, 16777472}, {537980928, 4029214752, 272166960, 16777472}, {4031778880, 4034981976, 16838792, 16777472}, {4028686360, 4030206000, 4032884808, 16777472}, {16838800, 16777472, 16777472, 16777472}, {270540808, 271642664, 4030730296, 16777472}, {542646344, 4033351776, 277876864, 16777472}, {4037079192, 16777472, 16777472, 16777472}, {4031778816, 4032884824, 3765497960, 16777472}, {277405816, 278401168, 16781472, 16777472}, {275836936, 4034924664, 4036030600, 16777472}, {4037079192, 16777472, 16777472, 16777472}}};
   alignas(16) static constexpr int G_CP[16] = {256, 513, 515, 517, 519, 777, 524, 526, 16, 0, 0, 0, 0, 0, 0, 0};
-  alignas(16) static constexpr int G_JO[3] = {0, 10, 15};
-  alignas(16) static constexpr int G_JE[15][16] = {{65282, 65280, 261, 65280, 65027, 513, 256, 65281, 0, 0, 0, 0, 0, 0, 0, 0}, {65287, 259, 264, 514, 65284, 260, 65290, 270, 0, 0, 0, 0, 0, 0, 0, 0}, {65288, 65286, 65289, 65284, 262, 65285, 65291, 271, 0, 0, 0, 0, 0, 0, 0, 0}, {266, 266, 269, 65285, 65287, 262, 65292, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 268, 0, 65286, 65289, 263, 65293, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 269, 0, 263, 65292, 65288, 65038, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 270, 0, 264, 0, 521, 65039, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 271, 0, 65290, 0, 523, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 65291, 0, 268, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 65293, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {257, 0, 256, 65280, 65282, 256, 257, 65280, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 259, 65281, 0, 258, 258, 65281, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 260, 0, 0, 65283, 259, 65282, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 65284, 260, 65283, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 65284, 0, 0, 0, 0, 0, 0, 0, 0}};
+  static constexpr int G_NJ = 116;  // values per cell
+  static constexpr int G_DT = 78;  // of them dq/dT from here, by position
+  static constexpr int G_DM = 110;  // and dq/dM of the third-body reactions
+  static constexpr int G_JC = 13;  // columns
+  static constexpr int G_JT4 = 6;  // terms per lane, in fours
+  alignas(16) static constexpr int G_JD[32] = {0, 3, 6, 9, 12, 15, 18, 22, 26, 30, 34, 38, 42, 46, 50, 54, 58, 62, 66, 70, 74, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  alignas(16) static constexpr uint32_t G_JE[6][16][4] = {{{11149316, 11149317, 11145230, 11202576}, {25829455, 25825362, 25882707, 25825364}, {13373442, 13430819, 13430823, 13430827}, {6746113, 6692871, 6692872, 6746124}, {25620558, 25567312, 25620562, 25620563}, {25956430, 26013784, 26013785, 26013786}, {2289664, 2232331, 2289682, 2232357}, {12775426, 12718115, 12718123, 12718127}, {25358414, 25301073, 25358420, 25301080}, {10752016, 10752027, 10809376, 10809377}, {10940430, 10940432, 10940437, 10883097}, {8970249, 8970250, 8974349, 8917012}, {13504562, 13504563, 13504566, 13504567}, {15659011, 15601717, 15601721, 15659067}, {26144847, 26087516, 26087517, 26144862}, {4460561, 4460572, 4517918, 4460593}}, {{11145237, 11145241, 11202587, 11149344}, {25825365, 25882710, 25829463, 25829465}, {13430831, 13426738, 13426739, 13426742}, {6746127, 6746131, 6688792, 6688797}, {25620564, 25563221, 25563222, 25620568}, {26013787, 26009692, 26009693, 25956447}, {2232364, 2232368, 2232372, 2297912}, {12718130, 12718131, 12718134, 12783671}, {25301082, 25301083, 25301084, 25366621}, {10752046, 10752061, 10752070, 10817610}, {10883099, 10940456, 10940457, 11006013}, {8974359, 8974367, 8974378, 9039938}, {13561921, 13561925, 13561929, 13627469}, {15659071, 15659075, 15659079, 15724619}, {26144863, 26144864, 26144865, 26210402}, {4460604, 4460616, 4526156, 25432147}}, {{11149345, 11149352, 11149353, 11145261}, {25825370, 25882715, 25825374, 25825376}, {13426743, 13373505, 13373509, 13373513}, {6746146, 6746150, 6746170, 6811710}, {25620569, 25620574, 25686111, 15523893}, {25956448, 25956449, 26021986, 11464708}, {11071502, 11014165, 11071513, 11071520}, {25747537, 25751634, 25694292, 25751637}, {4911121, 4911132, 4857886, 4911153}, {6950924, 7008271, 6950931, 6950936}, {11333672, 11333673, 11333677, 11333678}, {6352903, 6352904, 6352920, 6352925}, {9048077, 9048084, 9048087, 9052191}, {13246503, 13242411, 13299759, 13242437}, {2887680, 2945061, 2945068, 2945072}, {25432150, 25489495, 25432155, 25432158}}, {{11202606, 11145277, 11145284, 11202630}, {25882721, 25948258, 401414, 397334}, {13439053, 25227344, 25227349, 25227350}, {61446, 61462, 61466, 4132}, {15523897, 15470655, 15470659, 15470663}, {11464709, 11464765, 11464772, 11464774}, {11071521, 11071533, 11137092, 10678293}, {25751639, 25751642, 25817184, 6557711}, {4853820, 4911176, 4976716, 12849199}, {7008285, 6955046, 7016506, 14946363}, {11276356, 11276358, 11341898, 2551808}, {6295586, 6361150, 15343619, 15339579}, {9048106, 9113666, 8523785, 8523786}, {13299785, 13365325, 13037570, 13037603}, {2940980, 3006520, 7081985, 7139362}, {25432161, 25497698, 6483969, 6483987}}, {{11268170, 4648977, 4591644, 4714556}, {397338, 454692, 520256, 21553265}, {25170008, 25235551, 2756626, 2756652}, {69696, 8843277, 8843284, 8851479}, {15536203, 21373040, 21426290, 21491827}, {11530314, 2678795, 2625554, 2748460}, {10620973, 10686510, 21635183, 21631090}, {6557725, 6623290, 5042225, 4984904}, {12849225, 12914765, 5173308, 5173320}, {14946375, 15011915, 10547225, 10612763}, {2551826, 2617381, 12587043, 12652609}, {15339587, 15396935, 15462475, 659478}, {8581140, 8589354, 14815285, 14880825}, {13037607, 13103169, 15134779, 15200319}, {7139366, 7147582, 13168683, 13234245}, {6492194, 6877196, 6819859, 6942744}}, {{847908, 856128, 1044544, 116}, {21622898, 4395057, 9433154, 116}, {2879536, 21172337, 22016111, 116}, {9236522, 9244738, 116, 116}, {3018804, 3084344, 116, 116}, {7270458, 7335998, 116, 116}, {21753971, 23326830, 116, 116}, {5050444, 331802, 116, 116}, {5238860, 2428976, 116, 116}, {2166821, 8777759, 116, 116}, {4321308, 21303411, 116, 116}, {782362, 23588974, 116, 116}, {8515607, 651286, 116, 116}, {14749759, 4845598, 116, 116}, {21098608, 15331395, 116, 116}, {200740, 23924846, 116, 116}}};
 };
 }  // namespace mech
 }  // namespace pelec

@@ -585,7 +585,9 @@ int whole_grid(prc_reactor* r, int64_t ncells, WholeGrid& w) {
     if (r->max_slots > 0) groups = std::min<int64_t>(groups, r->max_slots);
     const int64_t per = (groups + r->whole_blocks - 1) / r->whole_blocks;
     w.gpw = (int)std::min<int64_t>(std::max<int64_t>(per, 1), whole_gpw());
-    w.blocks = (int)std::min<int64_t>((groups + w.gpw - 1) / w.gpw, r->whole_blocks);
+    // (prc.max_slots is a bound on the cells in flight)
+    const int64_t up = groups < ncells ? groups / w.gpw : (groups + w.gpw - 1) / w.gpw;
+    w.blocks = (int)std::min<int64_t>(std::max<int64_t>(up, 1), r->whole_blocks);
     w.groups = (int64_t)w.blocks * whole_gpw();
   }
   return PRC_OK;
@@ -595,7 +597,7 @@ int whole_grid(prc_reactor* r, int64_t ncells, WholeGrid& w) {
 template <class M = Mech>
 constexpr size_t whole_bytes() {
   if constexpr (whole_ok<M>())
-    return sizeof(double) * NV * M::G_W;
+    return sizeof(double) * GroupKin<M>::JAC_SIZE;
   else
     return 0;
 }
@@ -998,7 +1000,6 @@ int prc_get_param_int(prc_reactor* r, const char* key, int* v) {
     *v = r->shape.coop;
   else if (!std::strcmp(key, "prc.coop_tail_slots"))
     *v = r->shape.tail_slots;
-
   else if (!std::strcmp(key, "prc.blocks_tail"))
     *v = r->shape.bpc_tail > 0 ? r->shape.bpc_tail : r->occ_tail;
   else if (!std::strcmp(key, "prc.form"))

@@ -858,8 +858,38 @@ constexpr bool WHOLE = whole_ok<Mech>();
 // What a group's next right-hand side is for.
 enum CellPhase : int { CP_FETCH, CP_F0, CP_HIN, CP_NEWTON, CP_RESTART, CP_SETUP, CP_IDLE };
 
+// Final write-back of a cell (store_cell) by its group: component l of the state on lane l.
+template <class M>
+__device__ inline void store_whole(const Args& a, int64_t g, int status, const Counters& cn,
+                                   double yl, int l, double tm, double rhoe0, double rhoesrc) {
+  using K = GroupKin<M>;
+  using Grp = Group<K::G>;
+  int64_t loc;
+  const BoxDev& b = box_of(a, g, loc);
+  int i, j, k;
+  cell_ijk(b, loc, i, j, k);
+  if (status == CELL_OK) {
+    const double irho = 1.0 / Grp::sum(l < NSP ? yl : 0.0);
+    const double rEn = rhoe0 + a.dt * rhoesrc;
+    double ec[6], ek, cvk;
+    const double Tn = K::T_from_e(rEn * irho, l < NSP ? yl * irho : 0.0, l, Grp::bcast(yl, NSP),
+                                  tm, ec, ek, cvk);
+    if (l < NSP) b.rY.at(i, j, k, l) = yl;
+    if (l == 0) {
+      b.T.at(i, j, k, 0) = Tn;
+      b.rE.at(i, j, k, 0) = rEn;
+    }
+  } else if (l == 0) {
+    atomicAdd(&a.ctr[CT_FAILED], 1ull);
+  }
+  if (l == 0) {
+    if (b.FC.p) b.FC.at(i, j, k, 0) = (double)cn.nfe;
+    write_diag(a, g, status, &cn);
+  }
+}
+
 struct CellArgs {
-  double* J;  // G * n doubles per group of the grid: the cells' Jacobians
+  double* J;  // JAC_SIZE doubles per group of the grid: the cells' Jacobians
   int gpw;    // groups of each wave that take cells
 };
 
@@ -867,19 +897,29 @@ struct CellArgs {
 // of the loop evaluates one right-hand side per group -- f(t0, y0), an evaluation of the
 // initial-step iteration, a Newton iteration or an order-1 restart -- so the kinetics are one copy
 // of code that all groups of a wave run together whatever phase their cells are in.
+//
+// What bounds it: vector instruction issue. At drm19 64^3 the VALUs are busy 66 % of the time
+// (dodecane_lu 64^3: 79 %; waves per SIMD: 3 and 2, by the registers of the state), 42 % of the vector
+// instructions are FP64 arithmetic and the rest moves, selects and lane exchanges; HBM carries
+// 28 GB per call, 0.55 TB/s, nearly all of it Jacobian workspace. Compulsory traffic is 146 MB.
+// Measured against the work queue (a cell's state crossing HBM on every Newton iteration, 16 to 1100
+// launches a call): drm19 64^3 300 -> 50 ms, H2/air 32^3 6.5 -> 1.9 ms, 512 cells 4.6 -> 0.53 ms,
+// dodecane_lu 8192 cells 281 -> 39 ms.
 template <class M, int MINW>
 __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs ca) {
   using K = GroupKin<M>;
   constexpr int G = K::G;
   using Grp = Group<G>;
   constexpr int GPW = 64 / G;
-  __shared__ __attribute__((aligned(16))) double lds[GPW * K::WORDS];
+  __shared__ __attribute__((aligned(16))) double lds[GPW * K::WORDS + XT_WORDS];
   __shared__ CellState cst[GPW];
+  lds_double* xt = lds_ptr(lds) + GPW * K::WORDS;
+  fill_tables(xt);
   const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
   lds_double* sh = lds_ptr(lds) + gid * K::WORDS;
   CellState& cs = cst[gid];
   BdfScalars& S = cs.S;
-  double* Jg = ca.J + ((int64_t)blockIdx.x * GPW + gid) * (int64_t)(NV * G);
+  double* Jg = ca.J + ((int64_t)blockIdx.x * GPW + gid) * (int64_t)K::JAC_SIZE;
   const double tm = M::G_TMID[l];
   const bool in = l < NV;
   double z[BDF_QMAX + 1], ac = 0.0, ew = 0.0, Mi[NV];
@@ -935,10 +975,11 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
       ph = CP_F0;
     }
     if (__ballot(ph != CP_IDLE) == 0ull) break;
-    bool need_setup = false;
+    // att: a step attempt starts (prediction, coefficients); nxt: its prediction is made already
+    bool need_setup = false, att = ph == CP_SETUP, nxt = false;
     int status = -1;  // < 0 running, else the cell's final status
     if (ph == CP_SETUP) {
-      need_setup = true;
+      ph = CP_NEWTON;
     } else if (ph != CP_IDLE) {
       double yl = z[0], t = S.tn;
       if (ph == CP_NEWTON) {
@@ -951,7 +992,7 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
         t += cs.hg;
       }
       LaneVal f;
-      f.x = K::rhs(t, yl, l, rhoe0, rhoesrc, srcl, tm, sh);
+      f.x = K::rhs(t, yl, l, rhoe0, rhoesrc, srcl, tm, sh, xt);
       S.nfe++;
       if (ph == CP_NEWTON) {
         const int r = newton_correct<NV>(S, v, f, [&](LaneVal& b) {
@@ -962,13 +1003,12 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
           S.m = 0;
           need_setup = true;
         } else if (r != 1) {
-          bool attempt = false;
           if (r == 3) {
             const int e = conv_fail<NV>(S, v);
             if (e >= 0)
               status = e;
             else
-              attempt = true;
+              att = true;
           } else {
             const double dsm = S.acnrm * S.tq[2];
             if (dsm <= 1.0) {
@@ -978,7 +1018,7 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
               else if (S.nst >= a.prm.max_steps)
                 status = CELL_MAXSTEPS;
               else
-                need_setup = next_attempt<NV>(S, v, a.prm, a.dt);
+                nxt = true;
             } else {
               const int e = error_test_fail<NV>(S, v, dsm, a.prm.qmax);
               if (e >= 0)
@@ -986,14 +1026,13 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
               else if (e == -2)
                 ph = CP_RESTART;  // z_1 = h f(tn, z_0) with the next evaluation
               else
-                attempt = true;
+                att = true;
             }
           }
-          if (attempt) need_setup = begin_attempt<NV>(S, v, a.dt);
         }
       } else if (ph == CP_RESTART) {
         z[1] = S.h * f.x;
-        need_setup = begin_attempt<NV>(S, v, a.dt);
+        att = true;
         ph = CP_NEWTON;
       } else {
         // f(t0, y0), then cvHin's iteration (hin), one evaluation per turn
@@ -1038,22 +1077,25 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
           S.hscale = S.h;
           S.hprime = S.h;
           z[1] *= S.h;
-          step_prologue<NV>(S, v, a.prm.qmax);
-          need_setup = begin_attempt<NV>(S, v, a.dt);  // nst == 0: a set-up with a Jacobian
+          S.saved_t = S.tn;  // step_prologue at nst == 0
+          att = true;        // nst == 0: a set-up with a Jacobian
           ph = CP_NEWTON;
         }
       }
     }
+    if (nxt) next_predict<NV>(S, v, a.prm, a.dt);
+    if (att) predict<NV>(S, v, a.dt);
+    if (att || nxt) need_setup |= attempt_setup<RegV<NV, G>>(S);
     if (need_setup) {
-      if (jac_decide(S)) K::jac(S.tn, z[0], l, rhoe0, rhoesrc, srcl, tm, sh, Jg);
+      if (jac_decide(S)) K::jac(S.tn, z[0], l, rhoe0, rhoesrc, srcl, tm, sh, xt, Jg);
       const double gamma = S.gamma;
-      // (the columns' addresses are formed here, not kept across the cell loop)
-      const double* Jl = Jg + after(l, gamma);
+      // (the columns' addresses and the diagonal's masks are formed here, not kept across the cell loop)
+      const int lo = after(l, gamma);
+      const double* Jl = Jg + lo;
 #pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        const double m = in ? -gamma * K::load_l2(Jl + c * G) : 0.0;
-        Mi[c] = c == l ? m + 1.0 : m;  // I - gamma J
-      }
+      for (int c = 0; c < NV; ++c) Mi[c] = K::load_l2(Jl + c * G);
+#pragma unroll
+      for (int c = 0; c < NV; ++c) Mi[c] = fma(-gamma, Mi[c], c == lo ? 1.0 : 0.0);  // I - gamma J
       Grp::sync();
       int ier = K::invert(Mi, l, kap, sh);
       if (a.test_lu_fail && ier == 0) ier = 1;
@@ -1064,36 +1106,12 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
         if (e >= 0) {
           status = e;
         } else {
-          begin_attempt<NV>(S, v, a.dt);
-          ph = CP_SETUP;
+          ph = CP_SETUP;  // the next turn starts the attempt: another set-up
         }
       }
     }
     if (status >= 0) {
-      int64_t loc;
-      const BoxDev& b = box_of(a, g, loc);
-      int i, j, k;
-      cell_ijk(b, loc, i, j, k);
-      if (status == CELL_OK) {
-        const double yl = z[0];
-        const double irho = 1.0 / Grp::sum(l < NSP ? yl : 0.0);
-        const double rEn = rhoe0 + a.dt * rhoesrc;
-        double ec[6], ek, cvk;
-        const double Tn = K::T_from_e(rEn * irho, l < NSP ? yl * irho : 0.0, l,
-                                      Grp::bcast(yl, NSP), tm, ec, ek, cvk);
-        if (l < NSP) b.rY.at(i, j, k, l) = yl;
-        if (l == 0) {
-          b.T.at(i, j, k, 0) = Tn;
-          b.rE.at(i, j, k, 0) = rEn;
-        }
-      } else if (l == 0) {
-        atomicAdd(&a.ctr[CT_FAILED], 1ull);
-      }
-      if (l == 0) {
-        const Counters cn = counters(S);
-        if (b.FC.p) b.FC.at(i, j, k, 0) = (double)cn.nfe;
-        write_diag(a, g, status, &cn);
-      }
+      store_whole<M>(a, g, status, counters(S), z[0], l, tm, rhoe0, rhoesrc);
       ph = CP_FETCH;
     }
   }
@@ -1598,7 +1616,10 @@ __global__ void __launch_bounds__(64) k_model_cell(int64_t nc, double t, const d
                                                     const double* src, double* ydot, double* J) {
   using K = GroupKin<M>;
   constexpr int G = K::G;
-  __shared__ __attribute__((aligned(16))) double lds[64 / G * K::WORDS];
+  __shared__ __attribute__((aligned(16))) double lds[64 / G * K::WORDS + XT_WORDS];
+  lds_double* xt = lds_ptr(lds) + 64 / G * K::WORDS;
+  fill_tables(xt);
+  __shared__ double ws[64 / G][K::JAC_SIZE];
   const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
   const int64_t c = (int64_t)blockIdx.x * (64 / G) + gid;
   if (c >= nc) return;
@@ -1607,11 +1628,13 @@ __global__ void __launch_bounds__(64) k_model_cell(int64_t nc, double t, const d
   const double srcl = (src && l < NSP) ? src[l * nc + c] : 0.0;
   const double r1 = rhoesrc ? rhoesrc[c] : 0.0;
   const double tm = M::G_TMID[l];
-  const double f = K::rhs(t, yl, l, rhoe0[c], r1, srcl, tm, sh);
+  const double f = K::rhs(t, yl, l, rhoe0[c], r1, srcl, tm, sh, xt);
   if (l < NV) ydot[l * nc + c] = f;
-  if (J)
-    K::template jac<false, 1, NV>(t, yl, l, rhoe0[c], r1, srcl, tm, sh,
-                                  J + c * (int64_t)(NV * NV));
+  if (J) {
+    K::jac(t, yl, l, rhoe0[c], r1, srcl, tm, sh, xt, ws[gid]);
+    if (l < NV)
+      for (int m = 0; m < NV; ++m) J[c * (int64_t)(NV * NV) + l * NV + m] = ws[gid][m * G + l];
+  }
 }
 
 }  // namespace

@@ -18,7 +18,7 @@ namespace pelec {
 typedef double dv2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) dv2 lds_dv2;
 typedef __attribute__((address_space(3))) char lds_char;
-typedef int iv4 __attribute__((ext_vector_type(4)));
+typedef unsigned uv4 __attribute__((ext_vector_type(4)));
 
 // Register accessor of the step logic: component l of the cell on lane l. Every lane runs every
 // component loop once, with its own registers whatever the index, so the lanes of a group never
@@ -47,6 +47,60 @@ struct RegV : NoTape {
   }
 };
 
+// exp and log of the kinetics by table (P. T. P. Tang, ACM TOMS 15 (1989) 144 and 16 (1990) 378): a
+// third of the instructions of the library's, which are the larger part of a right-hand side
+// (GRI-Mech 3.0, 16,384 cells: 23.6 -> 22.0 ms; H2/air 32^3: 2.10 -> 1.97 ms). The
+// tables are XT_WORDS doubles of LDS per wave: 2^(j/32), and c_j = 2 / (1 + (j + 1/2)/32) with -log c_j / 2.
+constexpr int XT_WORDS = 96;
+__device__ inline void fill_tables(lds_double* xt) {
+  const int j = threadIdx.x & 31;
+  if ((threadIdx.x & 63) < 32) {
+    const double c = 1.0 / (1.0 + (j + 0.5) / 32.0);
+    xt[j] = exp2(j / 32.0);
+    xt[32 + j] = 2.0 * c;
+    xt[64 + j] = -log(c);
+  }
+  Group<64>::sync();
+}
+// e^x = 2^k 2^(j/32) e^r, |r| <= ln 2 / 64, e^r by its series to r^6 (r^7/5040 < 2^-58); below -746: 0.
+__device__ inline double fexp(double x, const lds_double* xt) {
+  x = x < -746.0 ? -746.0 : x;
+  const double kd = __builtin_rint(x * 46.16624130844683);  // 32 / ln 2
+  const int k = (int)kd;
+  const double t = xt[k & 31];
+  // ln 2 / 32 in two parts, the first with 27 zero bits: k times it is exact
+  double r = fma(-kd, 0x1.62e42f8p-6, x);
+  r = fma(-kd, 4.06140840434059e-10, r);
+  double q = fma(r, 1.0 / 720.0, 1.0 / 120.0);
+  q = fma(r, q, 1.0 / 24.0);
+  q = fma(r, q, 1.0 / 6.0);
+  q = fma(r, q, 0.5);
+  q = fma(r * r, q, r);
+  return ldexp(fma(t, q, t), k >> 5);
+}
+// log x of a positive, normal x: e ln 2 - log c_j + log(1 + r), |r| <= 1/64, by its series to r^8
+// (r^9/9 < 2^-57); within an ulp of the result or of 1, whichever is larger.
+__device__ inline double flog(double x, const lds_double* xt) {
+  const double m = __builtin_amdgcn_frexp_mant(x);  // [1/2, 1)
+  const int e = __builtin_amdgcn_frexp_exp(x) - 1;
+  const int j = (__double2hiint(m) >> 15) & 31;
+  const double r = fma(m, xt[32 + j], -1.0);
+  const double l = xt[64 + j];
+  double q = fma(r, -1.0 / 8.0, 1.0 / 7.0);
+  q = fma(r, q, -1.0 / 6.0);
+  q = fma(r, q, 1.0 / 5.0);
+  q = fma(r, q, -1.0 / 4.0);
+  q = fma(r, q, 1.0 / 3.0);
+  q = fma(r, q, -0.5);
+  q = fma(r * r, q, r);
+  return fma((double)e, 0.69314718055994530942, l) + q;
+}
+
+// What jac() leaves beside the matrix: the lane's e_k, rho c_v, and df/d(rho e0) of its component.
+struct JacOut {
+  double ek, D, fe;
+};
+
 // Kinetics, Jacobian and Newton matrix of one cell on a group of lanes.
 template <class Mech>
 struct GroupKin {
@@ -64,19 +118,19 @@ struct GroupKin {
   static constexpr int O_M = O_PP + 2 * (N + 1);    // third-body concentration per set
   static constexpr int O_Q = O_M + even(NS);        // q by position; entry P: 0
   static constexpr int O_PS = O_Q + P + 2;          // partial production rates
-  static constexpr int O_V = O_PS + G;              // vector exchange
-  static constexpr int RHS_WORDS = O_V + G;
-  static constexpr int O_PR = O_RP;                 // pivot row and pivot of the factorisation (n + 3 <= 4(N+1))
+  static constexpr int RHS_WORDS = O_PS + G;
+  // between right-hand sides their block serves the linear algebra
+  static constexpr int O_V = O_RP;                  // vector exchange (G <= 4(N+1))
+  static constexpr int O_PR = O_RP;                 // pivot row of the factorisation (n + 1 <= 4(N+1))
   // Jacobian part
   static constexpr int O_HR = RHS_WORDS;            // h_k/RT, entry N: 0
-  static constexpr int O_RB = O_HR + even(N + 1);   // per-round reaction derivatives, 8 x G
-  static constexpr int WORDS = O_RB + 8 * G;
-  typedef __attribute__((address_space(1))) double glb_double;
+  static constexpr int O_JV = O_HR + even(N + 1);   // the Jacobian's terms (G_NJ, and a 0)
+  static constexpr int WORDS = O_JV + even(Mech::G_NJ + 1);
+  // the cell's Jacobian workspace: element (k, c) at [c * G + k], G_JC columns (the n of the
+  // Jacobian, and the sums over dq/dM of each efficiency set and over dq/dT)
+  static constexpr int JAC_SIZE = Mech::G_JC * G;
 
-  // The cell's Jacobian lives in device memory, element (l, c) at Jg[c * CS + l * RS] (columns of G
-  // in the workspace of a group, rows of n for a caller's array): every element is read and written
-  // by one lane only, the adds of jac() are performed at the L2 (in program order per address), and
-  // reads go there too.
+  // Jacobian elements are written by whichever lane sums them and read by their row's lane: from the L2.
   __device__ static double load_l2(const double* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -114,7 +168,7 @@ struct GroupKin {
       e_cv(ec, T, ek, cvk);
       const double fv = Grp::sum(Yl * ek) - e;
       const double dv = Grp::sum(Yl * cvk);
-      const double dT = -fv / dv;
+      const double dT = -fv * recip(dv);
       T += dT;
       const bool lo2 = T < tm;
       const bool flip = any(lo2 != lo);
@@ -128,14 +182,26 @@ struct GroupKin {
     return T;
   }
 
+  // Arrhenius record of the reaction at position p, loaded ahead of its use.
+  struct Record {
+    dv2 ab;
+    double ear;
+    uint64_t pk;
+  };
+  __device__ static Record record(int p) {
+    return Record{reinterpret_cast<const dv2*>(&Mech::G_RA[0][0])[p], Mech::G_RE[p],
+                  Mech::G_RP[p]};
+  }
+
   // Reaction at position p (lane l of a round). JAC: also its derivatives into rb (8 x G).
   template <bool JAC, bool MUL>
-  __device__ static void reaction(int p, int l, double T, double lnT, double invT, lds_double* sh,
+  __device__ static void reaction(const Record& rc_, int p, int l, double T, double lnT,
+                                  double invT, lds_double* sh, const lds_double* xt,
                                   const double* rmul) {
-    const dv2 ab = reinterpret_cast<const dv2*>(&Mech::G_RA[0][0])[p];
-    const double ear = Mech::G_RE[p];
-    const uint64_t pk = Mech::G_RP[p];
-    const double karr = ab.x * exp(ab.y * lnT - ear * invT);
+    const dv2 ab = rc_.ab;
+    const double ear = rc_.ear;
+    const uint64_t pk = rc_.pk;
+    const double karr = ab.x * fexp(ab.y * lnT - ear * invT, xt);
     double kf = karr, dkdM = 0.0, dlnk = 0.0;
     if (JAC) dlnk = (ab.y + ear * invT) * invT;
     const int kind = (int)(pk >> 56) & 3;
@@ -145,29 +211,38 @@ struct GroupKin {
       dkdM = karr;
       if (Mech::G_NFO > 0 && kind == 2) {
         const double l0 = Mech::G_LOW[0][p], l1 = Mech::G_LOW[1][p], l2 = Mech::G_LOW[2][p];
-        const double k0r = exp(l0 + l1 * lnT - l2 * invT);
+        const double k0r = fexp(l0 + l1 * lnT - l2 * invT, xt);
         const double Pr = fmax(k0r * Mj, 1e-300);
-        const double iPr1 = 1.0 / (1.0 + Pr);
+        const double iPr1 = recip(1.0 + Pr);
         double F = 1.0, g = 0.0, dlnF_T = 0.0;
         if (Mech::G_TROEK[p]) {
-          const double t0 = Mech::G_TROE[0][p], t2 = Mech::G_TROE[2][p], t4 = Mech::G_TROE[4][p];
-          const double e3 = exp(Mech::G_TROE[1][p] * T), e1 = exp(Mech::G_TROE[3][p] * T);
-          const double e2 = Mech::G_TROE[5][p] != 0.0 ? exp(-t4 * invT) : 0.0;
-          const double Fc = t0 * e3 + t2 * e1 + e2;
-          const double lFc = log10(Fc);
+          constexpr double LOG10E = 0.43429448190325182765;
+          double lFc, iFc = 0.0, dFc = 0.0;
+          if constexpr (Mech::G_TCONST) {
+            lFc = Mech::G_TROE[0][p];
+          } else {
+            const double t0 = Mech::G_TROE[0][p], t2 = Mech::G_TROE[2][p], t4 = Mech::G_TROE[4][p];
+            const double e3 = fexp(Mech::G_TROE[1][p] * T, xt);
+            const double e1 = fexp(Mech::G_TROE[3][p] * T, xt);
+            const double e2 = Mech::G_TROE[5][p] != 0.0 ? fexp(-t4 * invT, xt) : 0.0;
+            const double Fc = fmax(t0 * e3 + t2 * e1 + e2, 1e-300);
+            lFc = flog(Fc, xt) * LOG10E;
+            if (JAC) {
+              iFc = 1.0 / Fc;
+              dFc = Mech::G_TROE[6][p] * e3 + Mech::G_TROE[7][p] * e1 + t4 * invT * invT * e2;
+            }
+          }
           const double cc = -0.4 - 0.67 * lFc, nn = 0.75 - 1.27 * lFc;
-          const double xx = log10(Pr) + cc;
-          const double DD = 1.0 / (nn - 0.14 * xx);
+          const double xx = flog(Pr, xt) * LOG10E + cc;
+          const double DD = recip(nn - 0.14 * xx);
           const double f1 = xx * DD;
-          const double iden = 1.0 / (1.0 + f1 * f1);
-          F = exp(Mech::T_LN10 * lFc * iden);
+          const double iden = recip(1.0 + f1 * f1);
+          F = fexp(Mech::T_LN10 * lFc * iden, xt);
           if (JAC) {
             g = -lFc * 2.0 * f1 * nn * DD * DD * iden * iden;
             const double df1 = (-0.67 * nn + 1.27 * xx) * DD * DD;
             const double dlF = iden - lFc * 2.0 * f1 * df1 * iden * iden;
-            const double dFc = Mech::G_TROE[6][p] * e3 + Mech::G_TROE[7][p] * e1 +
-                               t4 * invT * invT * e2;
-            dlnF_T = dlF * dFc / Fc;
+            dlnF_T = dlF * dFc * iFc;
           }
         }
         kf = karr * Pr * iPr1 * F;
@@ -196,48 +271,50 @@ struct GroupKin {
     double fac = dnu == 0 ? 1.0 : f1;
     if (dnu == 2 || dnu == -2) fac *= f1;
     const bool rev = (hi >> 26) & 1;
-    // 1/Kc = prod exp(g_p/RT) prod exp(-g_r/RT) (P_atm/RT)^-dnu
+    // 1/Kc = prod fexp(g_p/RT) prod fexp(-g_r/RT) (P_atm/RT)^-dnu
     const double iKc = rev ? (b0.y * b1.y * b2.y) * (a0.y * a1.y * a2.y) * fac : 0.0;
     const double r01 = a0.x * a1.x, p01 = b0.x * b1.x;
     const double Pb = p01 * b2.x;
     const double net = r01 * a2.x - iKc * Pb;
     sh[O_Q + p] = kf * net;
     if constexpr (JAC) {
-      lds_double* rb = sh + O_RB + l;
+      lds_double* jv = sh + O_JV;
       const lds_double* hr = sh + O_HR;
       const double dlnKc =
           ((hr[p0] + hr[p1] + hr[p2]) - (hr[r0] + hr[r1] + hr[r2]) - double(dnu)) * invT;
-      rb[0] = kf * a1.x * a2.x;
-      rb[G] = kf * a0.x * a2.x;
-      rb[2 * G] = kf * r01;
       const double kb = -kf * iKc;
-      rb[3 * G] = kb * b1.x * b2.x;
-      rb[4 * G] = kb * b0.x * b2.x;
-      rb[5 * G] = kb * p01;
-      rb[6 * G] = rev ? kf * (dlnk * net + iKc * Pb * dlnKc) : kf * dlnk * net;
-      rb[7 * G] = kind ? dkdM * net : 0.0;
+      const double d[6] = {kf * a1.x * a2.x, kf * a0.x * a2.x, kf * r01,
+                           kb * b1.x * b2.x, kb * b0.x * b2.x, kb * p01};
+      const int sl[6] = {r0, r1, r2, p0, p1, p2};
+      int o = Mech::G_JD[p];
+#pragma unroll
+      for (int u = 0; u < 6; ++u)
+        if (sl[u] != N) jv[o++] = d[u];
+      jv[Mech::G_DT + p] = rev ? kf * (dlnk * net + iKc * Pb * dlnKc) : kf * dlnk * net;
+      if (kind) jv[Mech::G_DM + p] = dkdM * net;
     }
   }
 
   // Species thermo of lane l into LDS and the third-body sums: what the reactions read.
+  __device__ static void load_g(double (&c)[8], bool lo, int l) {
+    const dv2* p = reinterpret_cast<const dv2*>(&Mech::G_G[lo ? 0 : 1][0][l][0]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const dv2 v = p[i * G];
+      c[2 * i] = v.x;
+      c[2 * i + 1] = v.y;
+    }
+  }
+  // c: the g/RT coefficients of branch lo0, loaded before T was known
   template <bool JAC>
   __device__ static void prelude(double T, double lnT, double invT, double Cl, int l, double tm,
-                                 lds_double* sh) {
+                                 double (&c)[8], bool lo0, lds_double* sh, const lds_double* xt) {
     const bool lo = T < tm;
-    double c[8];
-    {
-      const dv2* p = reinterpret_cast<const dv2*>(&Mech::G_G[lo ? 0 : 1][0][l][0]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const dv2 v = p[i * G];
-        c[2 * i] = v.x;
-        c[2 * i + 1] = v.y;
-      }
-    }
+    if (any(lo != lo0)) load_g(c, lo, l);
     const double gRT = fma(T, fma(T, fma(T, fma(T, c[4], c[3]), c[2]), c[1]), c[0]) - c[5] * lnT +
                        c[6] * invT;
-    const double E = exp(gRT);
-    const double iE = 1.0 / E;  // lanes >= N: coefficients 0, so E = iE = 1
+    const double E = fexp(gRT, xt);
+    const double iE = recip(E);  // lanes >= N: coefficients 0, so E = iE = 1
     if (l <= N) {
       const double C = l < N ? Cl : 1.0;
       ((lds_dv2*)(sh + O_RP))[l] = dv2{C, iE};
@@ -265,16 +342,24 @@ struct GroupKin {
 
   // production rate of species l from the q in LDS: a chunk of entries per lane, then the chunks
   // of each species
-  __device__ static double gather(int l, lds_double* sh) {
+  __device__ static void load_gather(uv4 (&e)[Mech::G_L8], int l) {
+#pragma unroll
+    for (int i = 0; i < Mech::G_L8; ++i)
+      e[i] = *reinterpret_cast<const uv4*>(&Mech::G_GE[i][l][0]);
+  }
+  __device__ static double gather(const uv4 (&e)[Mech::G_L8], int l, lds_double* sh) {
     double acc = 0.0;
     const lds_char* q = (const lds_char*)(sh + O_Q);
 #pragma unroll
-    for (int i = 0; i < Mech::G_L4; ++i) {
-      const iv4 e = *reinterpret_cast<const iv4*>(&Mech::G_GE[i][l][0]);
+    for (int i = 0; i < Mech::G_L8; ++i)
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        acc = fma((double)(e[u] >> 24), *(const lds_double*)(q + (e[u] & 0xffff)), acc);
-    }
+      for (int u = 0; u < 4; ++u) {
+        const unsigned w = e[i][u];
+        const double q0 = *(const lds_double*)(q + (w & 0xfff));
+        const double q1 = *(const lds_double*)(q + ((w >> 16) & 0xfff));
+        acc = fma((double)((int)(w << 16) >> 28), q0, acc);
+        acc = fma((double)((int)w >> 28), q1, acc);
+      }
     sh[O_PS + l] = acc;
     Grp::sync();
     const int cp = Mech::G_CP[l], b = cp & 255, m = cp >> 8;
@@ -285,84 +370,112 @@ struct GroupKin {
     return wd;
   }
 
+  // log of a temperature (NaN where it is not one)
+  __device__ static double log_T(double T, const lds_double* xt) {
+    return T > 0.0 ? flog(T, xt) : __builtin_nan("");
+  }
+
   // f(t, y) for the lane's component (0 on lanes >= n).
   template <bool MUL = false>
   __device__ static double rhs(double t, double yl, int l, double rhoe0, double rhoesrc,
-                               double srcl, double tm, lds_double* sh,
+                               double srcl, double tm, lds_double* sh, const lds_double* xt,
                                const double* rmul = nullptr) {
     l = after(l, yl);
     const bool sp = l < N;
     const double ys = sp ? yl : 0.0;
-    const double irho = 1.0 / Grp::sum(ys);
+    // the tables of the first phases are loaded ahead of the temperature
+    Record nx = record(l);
+    const double Tg = Grp::bcast(yl, N);
+    const bool lo0 = Tg < tm;
+    double gc[8];
+    load_g(gc, lo0, l);
+    const double irho = recip(Grp::sum(ys));
     double ec[6], ek, cvk;
-    const double T = T_from_e((rhoe0 + t * rhoesrc) * irho, ys * irho, l, Grp::bcast(yl, N), tm,
-                              ec, ek, cvk);
-    const double lnT = log(T), invT = 1.0 / T;
-    prelude<false>(T, lnT, invT, ys * Mech::G_IWT[l], l, tm, sh);
+    const double T = T_from_e((rhoe0 + t * rhoesrc) * irho, ys * irho, l, Tg, tm, ec, ek, cvk);
+    const double lnT = log_T(T, xt), invT = recip(T);
+    prelude<false>(T, lnT, invT, ys * Mech::G_IWT[l], l, tm, gc, lo0, sh, xt);
+    uv4 ge[Mech::G_L8];
+    load_gather(ge, after(l, T));
 #pragma unroll 1
-    for (int r = 0; r < RR; ++r) reaction<false, MUL>(after(G * r + l, lnT), l, T, lnT, invT, sh, rmul);
+    for (int r = 0; r < RR; ++r) {
+      const Record rc = nx;
+      const int p = G * r + l;
+      nx = record(p + (r + 1 < RR ? G : 0));
+      reaction<false, MUL>(rc, p, l, T, lnT, invT, sh, xt, rmul);
+    }
     Grp::sync();
-    const double wd = gather(l, sh);
+    const double wd = gather(ge, l, sh);
     const double fk = sp ? Mech::G_WT[l] * wd + srcl : 0.0;
     const double num = rhoesrc - Grp::sum(ek * fk);
     const double D = Grp::sum(ys * cvk);
     Grp::sync();
-    return l == N ? num / D : fk;
+    return l == N ? num * recip(D) : fk;
   }
 
-  // Exact Jacobian of rhs() into Jg (row l on lane l). The rows are summed in device memory rather
-  // than LDS: n x n doubles of LDS per cell (23 KB at n = 54) would leave one wave per SIMD.
-  template <bool MUL = false, int CS = G, int RS = 1>
-  __device__ static void jac(double t, double yl, int l, double rhoe0, double rhoesrc, double srcl,
-                             double tm, lds_double* sh, double* Jg, const double* rmul = nullptr) {
+  // Exact Jacobian of rhs() into ws (JAC_SIZE doubles; columns 0..n-1). The reactions leave their
+  // derivatives in LDS, each lane sums the elements that the schedule deals it (terms in fours, an
+  // element's sum stored when its last term is added), then the rows' lanes finish them. Adding each
+  // reaction's terms to the rows instead would take n x n doubles of LDS per cell (23 KB at n = 54: one wave
+  // per SIMD) or an L2 atomic per term (107 k to 312 k cycles a Jacobian, n = 22 to 54; 34 k to 65 k
+  // this way).
+  template <bool MUL = false>
+  __device__ static JacOut jac(double t, double yl, int l, double rhoe0, double rhoesrc, double srcl,
+                             double tm, lds_double* sh, const lds_double* xt, double* ws,
+                             const double* rmul = nullptr) {
     l = after(l, yl);
     const bool sp = l < N;
-    double* Jr = Jg + l * RS;
-    if (l < n)
+    double* wl = ws + l;
 #pragma unroll 4
-      for (int m = 0; m < n; ++m) Jr[m * CS] = 0.0;  // column N stays 0
+    for (int c = 0; c < Mech::G_JC; ++c) wl[c * G] = 0.0;
     const double ys = sp ? yl : 0.0;
+    const double Tg = Grp::bcast(yl, N);
+    const bool lo0 = Tg < tm;
+    double gc[8];
+    load_g(gc, lo0, l);
     const double irho = 1.0 / Grp::sum(ys);
     double ec[6], ek, cvk;
-    const double T = T_from_e((rhoe0 + t * rhoesrc) * irho, ys * irho, l, Grp::bcast(yl, N), tm,
-                              ec, ek, cvk);
-    const double lnT = log(T), invT = 1.0 / T;
-    prelude<true>(T, lnT, invT, ys * Mech::G_IWT[l], l, tm, sh);
-    double dwdT = 0.0, tb[NS > 0 ? NS : 1];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) tb[s] = 0.0;
+    const double T = T_from_e((rhoe0 + t * rhoesrc) * irho, ys * irho, l, Tg, tm, ec, ek, cvk);
+    const double lnT = log_T(T, xt), invT = recip(T);
+    prelude<true>(T, lnT, invT, ys * Mech::G_IWT[l], l, tm, gc, lo0, sh, xt);
+    if (l == 0) sh[O_JV + Mech::G_NJ] = 0.0;
 #pragma unroll 1
     for (int r = 0; r < RR; ++r) {
-      Grp::sync();  // the previous round's derivatives have been read
-      reaction<true, MUL>(after(G * r + l, lnT), l, T, lnT, invT, sh, rmul);
-      Grp::sync();
-      const int e1 = Mech::G_JO[r + 1];
+      const int p = after(G * r + l, lnT);
+      reaction<true, MUL>(record(p), p, l, T, lnT, invT, sh, xt, rmul);
+    }
+    uv4 ge[Mech::G_L8];
+    load_gather(ge, after(l, T));
+    // the zeros are in memory before other lanes store over them; the terms are in LDS
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    Grp::sync();
+    const double wd = gather(ge, l, sh);
+    double acc = 0.0;
+    uv4 nx = *reinterpret_cast<const uv4*>(&Mech::G_JE[0][l][0]);
 #pragma unroll 1
-      for (int i = Mech::G_JO[r]; i < e1; ++i) {
-        const int je = Mech::G_JE[i][l];
-        if (je) {
-          const int q = je & 255;
-          const double nu = (double)((je << 16) >> 24);
-          const uint64_t pk = Mech::G_RP[G * r + q];
-          const lds_double* rb = sh + O_RB + q;
-          dwdT += nu * rb[6 * G];
+    for (int i = 0; i < Mech::G_JT4; ++i) {
+      const uv4 e = nx;
+      nx = *reinterpret_cast<const uv4*>(&Mech::G_JE[i + 1 < Mech::G_JT4 ? i + 1 : i][l][0]);
+      double v[4];
 #pragma unroll
-          for (int u = 0; u < 6; ++u) {
-            const int m = (int)(pk >> (8 * u)) & 255;
-            if (m < N)
-              __builtin_amdgcn_global_atomic_fadd_f64((glb_double*)(Jr + m * CS), nu * rb[u * G]);
-          }
-          if (NS > 0 && G * r < Mech::G_NTB) {
-            const int kind = (int)(pk >> 56) & 3, ef = (int)(pk >> 48) & 255;
-            const double c = kind ? nu * rb[7 * G] : 0.0;
+      for (int u = 0; u < 4; ++u) v[u] = sh[O_JV + (e[u] & 0xfff)];
 #pragma unroll
-            for (int s = 0; s < NS; ++s) tb[s] += s == ef ? c : 0.0;
-          }
+      for (int u = 0; u < 4; ++u) {
+        acc = fma((double)((int)(e[u] << 16) >> 28), v[u], acc);
+        if (e[u] & 0x10000u) {
+          ws[e[u] >> 17] = acc;
+          acc = 0.0;
         }
       }
     }
-    const double wd = gather(l, sh);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
     // energy row and the T-elimination (CellModel::jac)
+    double tb[NS > 0 ? NS : 1], tbs = 0.0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      tb[s] = load_l2(wl + (n + s) * G);
+      tbs += tb[s];
+    }
+    const double dwdT = load_l2(wl + (n + NS) * G);
     const double Wk = Mech::G_WT[l];
     const double fk = sp ? Wk * wd + srcl : 0.0;
     const double Bk = Wk * dwdT;
@@ -375,72 +488,142 @@ struct GroupKin {
     const double fT = num * iD;
     const double dfTdT = (dNdT - fT * dDdT) * iD;
     const double b = Bk * iD;
-    double tbs = 0.0;
+    // columns in batches: a batch's loads are in flight together
+    constexpr int CBJ = 6;
+#pragma unroll 1
+    for (int m0 = 0; m0 < N; m0 += CBJ) {
+      double av[CBJ];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) tbs += tb[s];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // the adds are done
-#pragma unroll 2
-    for (int m = 0; m < N; ++m) {
-      double a = sp ? load_l2(Jr + m * CS) + tbs : 0.0;
+      for (int u = 0; u < CBJ; ++u) av[u] = load_l2(wl + (m0 + u < N ? m0 + u : N) * G);
 #pragma unroll
-      for (int s = 0; s < NS; ++s) a += tb[s] * Mech::T_EFFD[s][m];
-      a *= Wk * Mech::IW[m];
-      // T row, column m: dNdx_m = -sum_k e_k A_km
-      const double dNdx = -Grp::sum(ek * a);
-      const double em = Grp::bcast(ek, m), cm = Grp::bcast(cvk, m);
-      if (l < n) Jr[m * CS] = sp ? a - b * em : (dNdx - fT * cm) * iD - dfTdT * em * iD;
+      for (int u = 0; u < CBJ; ++u) {
+        const int m = m0 + u;
+        if (m >= N) break;
+        double a = av[u] + tbs;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) a += tb[s] * Mech::T_EFFD[s][m];
+        a *= Wk * Mech::IW[m];  // 0 on lanes without a species
+        // T row, column m: dNdx_m = -sum_k e_k A_km
+        const double dNdx = -Grp::sum(ek * a);
+        const double em = Grp::bcast(ek, m), cm = Grp::bcast(cvk, m);
+        const double tr = (dNdx - fT * cm) * iD - dfTdT * em * iD;
+        wl[m * G] = l == N ? tr : a - b * em;
+      }
     }
     Grp::sync();
+    return JacOut{ek, D, l == N ? dfTdT * iD : b};
+  }
+
+  // a b + c into a register of its own: the row shift of invert() would otherwise cost a move per
+  // column (the compiler prefers the two-address form).
+  __device__ static double fma3(double a, double b, double c) {
+    double r;
+    __asm__("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+  }
+  __device__ static double fma3_uniform(double a, double b, double c) {  // b in scalar registers
+    double r;
+    __asm__("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+    return r;
+  }
+
+  // The group's pivot for a column: the largest of the rows' high words of |a| with the lane in the
+  // low six bits (used rows: the lane alone), so the pivot is within 2^-14 of the largest entry.
+  __device__ static unsigned pivot_key(double a, bool used, int l) {
+    const unsigned hi = (unsigned)__double2hiint(a) & 0x7fffffc0u;
+    unsigned x = (used ? 0u : hi) | (unsigned)l;
+    if constexpr (G > 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+      x = max(r[0], r[1]);
+    }
+    if constexpr (G > 16) {
+      const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+      x = max(r[0], r[1]);
+    }
+    x = max(x, (unsigned)row_ror<8>((int)x));
+    x = max(x, (unsigned)row_ror<4>((int)x));
+    x = max(x, (unsigned)row_ror<2>((int)x));
+    return max(x, (unsigned)row_ror<1>((int)x));
   }
 
   // a <- row of the inverse of the matrix whose row l is in a (lanes < n), by Gauss-Jordan
   // elimination with partial pivoting, rows staying on their lanes: with lane p the pivot of
   // column kap(p), lane p ends with row kap(p) of the inverse, its columns in pivot order (column c
   // belongs to the right-hand side component of the lane that was column c's pivot). The pivot search
-  // is a maximum over |a| with the lane in the low six mantissa bits (a choice among values equal to
-  // 2^-46). Pivot rows are broadcast through LDS as they stand and scaled once at the end: the other
-  // rows' multipliers carry 1 / pivot. Returns 0, or k + 1 when column k has no usable pivot.
+  // is one 32-bit maximum (pivot_key). Pivot rows are broadcast as they stand -- by v_readlane where a
+  // wave holds one cell (VALU time, no LDS round trip and no share of the CU's LDS bandwidth), through
+  // LDS where it holds several (a read per cell and a select per column) -- and scaled once at the end: the
+  // other rows' multipliers carry 1 / pivot. Measured: GRI-Mech 3.0 (n = 54), 16,384 cells, 25.4 ms
+  // through LDS, 23.0 ms by v_readlane; four cells per wave (n = 10) 7.7 k cycles an inversion
+  // through LDS, 11.5 k by v_readlane. Returns 0, or k + 1 when column k has no usable pivot.
   __device__ static int invert(double (&a)[n], int l, int& kap, lds_double* sh) {
     l = after(l, a[0]);
-    lds_dv2* pr = (lds_dv2*)(sh + O_PR);
+    [[maybe_unused]] lds_dv2* pr = (lds_dv2*)(sh + O_PR);
     bool used = l >= n;
     kap = 0;
     int ier = 0;
     double scale = 0.0;
+    unsigned best = pivot_key(a[0], used, l);
     // every step eliminates the column in a[0] and stores the row shifted down by one, so the loop
     // is rolled (unrolled it is n times the code, more than the instruction cache at n = 54) and
     // after n steps every column is back in its place
 #pragma unroll 1
     for (int k = 0; k < n; ++k) {
-      const double v = used ? 0.0 : fabs(a[0]);
-      const long long key = (__double_as_longlong(v) & ~63ll) | l;
-      const double best = Grp::max(__longlong_as_double(key));
-      if (!(best >= 2.3e-308) && ier == 0) ier = k + 1;
-      const bool piv = !used && l == (int)(__double_as_longlong(best) & 63);
-      if (piv) {
-        pr[(n + 1) / 2] = dv2{a[0], 0.0};
-#pragma unroll
-        for (int c = 0; c < n; c += 2)
-          pr[c / 2] = dv2{c + 1 < n ? a[c + 1 < n ? c + 1 : 0] : 1.0,
-                          c + 2 < n ? a[c + 2 < n ? c + 2 : 0] : 1.0};
+      if (best < 64u && ier == 0) ier = k + 1;
+      const bool piv = !used && l == (int)(best & 63u);
+      double pv;
+      int pl = 0;
+      if constexpr (G == 64) {
+        pl = __builtin_amdgcn_readfirstlane((int)(best & 63u));
+        pv = lane_read(a[0], pl);
+      } else {
+        pv = __shfl(a[0], (int)(best & 63u), G);
       }
-      Grp::sync();
-      const double inv = 1.0 / pr[(n + 1) / 2].x;
-      const double f = piv ? 0.0 : a[0] * inv;
+      if constexpr (G < 64) {
+        if (piv) {
+#pragma unroll
+          for (int c = 0; c < n; c += 2)
+            pr[c / 2] = dv2{c + 1 < n ? a[c + 1 < n ? c + 1 : 0] : 1.0,
+                            c + 2 < n ? a[c + 2 < n ? c + 2 : 0] : 1.0};
+        }
+        Grp::sync();
+      }
+      const double inv = recip(pv);
+      const double nf = piv ? 0.0 : -a[0] * inv;
       const double last = piv ? 1.0 : 0.0;
       if (piv) {
         scale = inv;
         used = true;
         kap = k;
       }
+      if constexpr (G == 64) {
+        // one cell per wave: the pivot row by v_readlane, four columns ahead of their use (a scalar
+        // register read back at once stalls); the row's last entry is 1
 #pragma unroll
-      for (int c = 0; c < n; c += 2) {
-        const dv2 p = pr[c / 2];
-        a[c] = fma(-f, p.x, c + 1 < n ? a[c + 1 < n ? c + 1 : 0] : last);
-        if (c + 1 < n) a[c + 1 < n ? c + 1 : 0] = fma(-f, p.y, c + 2 < n ? a[c + 2 < n ? c + 2 : 0] : last);
-        if (c % 16 == 14) __asm__ __volatile__("" ::: "memory");  // at most 16 columns in flight
+        for (int c = 0; c < n - 1; c += 4) {
+          double p[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (c + u < n - 1) p[u] = lane_read(a[c + u + 1], pl);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (c + u < n - 1) a[c + u] = fma3_uniform(nf, p[u], a[c + u + 1]);
+          if (c == 0) best = pivot_key(a[0], used, l);  // the next search, beside the update
+        }
+        a[n - 1] = nf + last;
+      } else {
+#pragma unroll
+        for (int c = 0; c < n; c += 2) {
+          const dv2 p = pr[c / 2];
+          a[c] = fma3(nf, p.x, c + 1 < n ? a[c + 1 < n ? c + 1 : 0] : last);
+          if (c + 1 < n)
+            a[c + 1 < n ? c + 1 : 0] = fma3(nf, p.y, c + 2 < n ? a[c + 2 < n ? c + 2 : 0] : last);
+          if (c == 0) best = pivot_key(a[0], used, l);
+          if (c % 16 == 14) __asm__ __volatile__("" ::: "memory");  // at most 16 columns in flight
+        }
+        Grp::sync();
       }
-      Grp::sync();
     }
 #pragma unroll
     for (int c = 0; c < n; ++c) a[c] *= scale;

@@ -717,6 +717,8 @@ class Gen:
         order = sorted(range(R), key=lambda j: (-kind_id[rx[j].kind], j))
         pos = {j: p for p, j in enumerate(order)}
         ab, ear, pack, low, troe, troek = [], [], [], [], [], []
+        tconst = all(r.troe is None or self.troe_const(r.troe) is not None
+                     for r in rx if r.kind == "falloff")
         for j in order:
             r = rx[j]
             ab.append([r.A, r.b])
@@ -741,7 +743,10 @@ class Gen:
                     troek.append(1)
                     troe.append([1.0 - a, -1.0 / T3, a, -1.0 / T1, T2,
                                  1.0 if len(r.troe) > 3 else 0.0, -(1.0 - a) / T3, -a / T1])
+                    if tconst:  # log10 Fc itself
+                        troe[-1] = [math.log10(self.troe_const(r.troe))] + [0.0] * 7
         NFO, NTB = len(low), sum(r.kind == "three-body" for r in rx)
+        ns_ = len(self.effsets)
         none = sum(N << (8 * i) for i in range(6)) | 2 << 59
         ab += [[0.0, 0.0]] * (P - R)
         ear += [0.0] * (P - R)
@@ -758,6 +763,7 @@ class Gen:
         arr("G_LOW", "double", [[x[i] for x in low] for i in range(3)], [3, q])
         arr("G_TROE", "double", [[x[i] for x in troe] for i in range(8)], [8, q])
         arr("G_TROEK", "int", troek or [0], [q])
+        w(f"  static constexpr bool G_TCONST = {'true' if tconst else 'false'};  // no Fc depends on T")
         # production rates: each species' (reaction, nu) list cut into chunks of at most L entries,
         # one chunk per lane; L the smallest for which all chunks fit the group
         rows = [[] for _ in range(N)]
@@ -768,29 +774,62 @@ class Gen:
         L = 1
         while sum((len(x) + L - 1) // L for x in rows) > G:
             L += 1
-        L4 = (L + 3) // 4
+        L8 = (L + 7) // 8
         chunks, begin = [], []
         for x in rows:
             begin.append(len(chunks) | ((len(x) + L - 1) // L) << 8)
             chunks += [x[i:i + L] for i in range(0, len(x), L)]
         chunks += [[]] * (G - len(chunks))
-        entry = lambda c, i: (c[i][0] * 8 | (c[i][1] & 0xff) << 24) if i < len(c) else P * 8
-        sgn = lambda v: v - (1 << 32) if v >= 1 << 31 else v
-        w(f"  static constexpr int G_L4 = {L4};")
+        # entry: byte offset of q (12 bits), nu (signed, 4 bits); two entries to a word
+        entry = lambda c, i: (c[i][0] * 8 | (c[i][1] & 0xf) << 12) if i < len(c) else P * 8
+        pair = lambda c, i: entry(c, i) | entry(c, i + 1) << 16
+        w(f"  static constexpr int G_L8 = {L8};")
         w(f"  static constexpr int G_CMAX = {max(b >> 8 for b in begin)};  // chunks of a species")
-        arr("G_GE", "int", [[[sgn(entry(c, 4 * i + u)) for u in range(4)] for c in chunks]
-                            for i in range(L4)], [L4, G, 4])
+        arr("G_GE", "uint32_t", [[[pair(c, 8 * i + 2 * u) for u in range(4)] for c in chunks]
+                                 for i in range(L8)], [L8, G, 4])
         arr("G_CP", "int", begin + [0] * (G - N), [G])
-        # Jacobian rows: per round, each species' entries (position in the round, nu)
-        offs, ent = [0], []
-        for r in range(RR):
-            own = [[(p - G * r, v) for p, v in x if p // G == r] for x in rows]
-            own += [[]] * (G - N)
-            for i in range(max(len(x) for x in own)):
-                ent.append([(x[i][0] | (x[i][1] & 0xff) << 8) if i < len(x) else 0 for x in own])
-            offs.append(len(ent))
-        arr("G_JO", "int", offs, [RR + 1])
-        arr("G_JE", "int", ent, [len(ent), G])
+        # Jacobian: every value that an element of it is summed from is left in LDS by the reactions
+        # (dq_j/dC of each mass-action slot, dq_j/dT, and dq_j/dM of the third-body reactions); the
+        # terms are sorted by element and dealt to the lanes whole elements at a time, longest
+        # first to the least loaded lane. Columns beyond n hold sum nu dq/dM per efficiency set
+        # and sum nu dq/dT.
+        off, src = 0, []  # src[p]: (offset of each reactant slot, of each product slot, dqdT, dqdM)
+        for p, j in enumerate(order):
+            r = rx[j]
+            slots = [pack[p] >> (8 * u) & 255 for u in range(6)]
+            live = [u for u in range(6) if slots[u] != N]
+            src.append((off, {u: off + i for i, u in enumerate(live)}, slots))
+            off += len(live)
+        DQ, DT, DM = 0, off, off + P
+        NJ = DM + NFO + NTB
+        elems = {}
+        for k in range(N):
+            for p, nu in rows[k]:
+                for u, o in src[p][1].items():
+                    elems.setdefault((k, src[p][2][u]), []).append((DQ + o, nu))
+                elems.setdefault((k, n + ns_), []).append((DT + p, nu))
+                if pack[p] >> 56 & 3:
+                    elems.setdefault((k, n + (pack[p] >> 48 & 255)), []).append((DM + p, nu))
+        load, sched = [0] * G, [[] for _ in range(G)]
+        for (k, c), terms in sorted(elems.items(), key=lambda kv: (-len(kv[1]), kv[0])):
+            lane = load.index(min(load))
+            load[lane] += len(terms)
+            for i, (o, nu) in enumerate(terms):
+                last = i + 1 == len(terms)
+                sched[lane].append(o | (nu & 0xf) << 12 | (1 << 16 if last else 0)
+                                   | (c * G + k) << 17)
+        JT = (max(load) + 3) // 4 * 4
+        assert NJ < 4096 and (n + ns_ + 1) * G < 1 << 15
+        pad = DM + NFO + NTB  # an entry that stays 0
+        sched = [x + [pad] * (JT - len(x)) for x in sched]
+        w(f"  static constexpr int G_NJ = {NJ};  // values per cell")
+        w(f"  static constexpr int G_DT = {DT};  // of them dq/dT from here, by position")
+        w(f"  static constexpr int G_DM = {DM};  // and dq/dM of the third-body reactions")
+        w(f"  static constexpr int G_JC = {n + ns_ + 1};  // columns")
+        w(f"  static constexpr int G_JT4 = {JT // 4};  // terms per lane, in fours")
+        arr("G_JD", "int", [s[0] for s in src] + [0] * (P - R), [P])
+        arr("G_JE", "uint32_t", [[sched[q][i:i + 4] for q in range(G)] for i in range(0, JT, 4)],
+            [JT // 4, G, 4])
 
     # ------------------------------------------------------------------ top level
     def generate(self) -> str:

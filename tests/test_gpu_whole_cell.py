@@ -1,0 +1,135 @@
+"""GPU: the kernels that give a lane group a whole cell (batched FP64 form, ReactorRK64, adjoint),
+and the launch shape that the FP32-factor queue takes by itself, at the sizes where they can go wrong.
+
+A cell's arithmetic does not depend on its neighbours, on the group or wave that takes it or on how
+many cells share the call, so a cell taken out of a larger call has to give the same bits: that is the
+tolerance of the size tests (none). The larger calls themselves are held to the oracle here or in the
+parity tests.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from pelec_amd import inputs, mechanism as M  # noqa: E402
+from pelec_amd.reactor import Reactor  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+GATE_T = 1e-3
+GATE_Y = 1e-8
+#: n = 10 (16 lanes), 22 (32 lanes), 54 (64 lanes) unknowns per cell
+WORKLOADS = ["lidryer_32", "drm19_64", "gri30_flat", "dodecane_64"]
+NBIG = 200
+
+
+def to_dev(a, dtype=torch.float64):
+    return torch.tensor(np.ascontiguousarray(a), dtype=dtype, device=DEV)
+
+
+def react(wl, d, idx, dt=None, rk64=False, noalloc=False, **opts):
+    """The cells idx of d in one flat call -> dict of numpy arrays."""
+    W = inputs.WORKLOADS[wl]
+    r = Reactor(W.mech, chem_integrator="ReactorRK64" if rk64 else "ReactorCvode")
+    if not rk64:
+        opts = dict(dict(form="batched", lu_fp32=False), **opts)
+    shape = {k: opts.pop(k) for k in list(opts) if k.startswith("prc.")}
+    r.configure(rtol=W.rtol, atol=W.atol, **opts)
+    for k, v in shape.items():
+        r.set_param(k, v)
+    a = {k: to_dev(d[k][..., idx]) for k in ("rY", "T", "rE")}
+    n = len(idx)
+    diag = torch.zeros((8, n), dtype=torch.int32, device=DEV)
+    r.set_diagnostics(diag)
+    src = {k: to_dev(d[k][..., idx]) for k in ("rYsrc", "rEsrc") if k in d}
+    mask = to_dev(d["mask"][idx], torch.int32) if "mask" in d else None
+    call = r.react_flat_noalloc if noalloc else r.react_flat
+    call(a["rY"], a["T"], a["rE"], W.dt if dt is None else dt, mask=mask, **src)
+    torch.cuda.synchronize()
+    out = {k: v.cpu().numpy() for k, v in a.items()}
+    out["diag"] = diag.cpu().numpy()
+    out["nfail"] = r.last_failures()
+    r.close()
+    return out
+
+
+def same(out, big, idx):
+    for k in ("rY", "T", "rE", "diag"):
+        np.testing.assert_array_equal(out[k], big[k][..., idx], err_msg=k)
+
+
+@pytest.fixture(scope="module")
+def big():
+    """NBIG cells of each workload with sources and a mask (some waves of four, two and one cells
+    lose part of their cells, one loses all), in one call."""
+    cache = {}
+
+    def get(wl):
+        if wl not in cache:
+            d = inputs.make_inputs(wl, NBIG)
+            rng = np.random.default_rng(31)
+            d = dict(d)
+            d["rEsrc"] = rng.normal(0, 1e8, NBIG)
+            d["rYsrc"] = rng.normal(0, 1e-4, d["rY"].shape) * d["rY"]
+            d["mask"] = (rng.uniform(size=NBIG) > 0.2).astype(np.int32)
+            d["mask"][64:72] = 0
+            cache[wl] = d, react(wl, d, np.arange(NBIG))
+        return cache[wl]
+    return get
+
+
+@pytest.mark.parametrize("wl", WORKLOADS)
+@pytest.mark.parametrize("first,n", [(0, 1), (3, 2), (64, 8), (1, 63), (60, 65), (7, 193)])
+def test_cells_do_not_depend_on_the_call(wl, first, n, big):
+    d, ref = big(wl)
+    idx = np.arange(first, first + n)
+    out = react(wl, d, idx)
+    assert out["nfail"] == ref["nfail"] == 0
+    same(out, ref, idx)
+    off = d["mask"][idx] == 0
+    for k in ("rY", "T", "rE"):
+        np.testing.assert_array_equal(out[k][..., off], d[k][..., idx[off]])
+
+
+@pytest.mark.parametrize("wl", WORKLOADS)
+@pytest.mark.parametrize("max_slots", [1, 5, 130])
+def test_refilled_groups(wl, max_slots, big):
+    """Fewer cells in flight than cells in the call: every group takes several cells in turn."""
+    d, ref = big(wl)
+    idx = np.arange(60 if max_slots == 1 else NBIG)
+    same(react(wl, d, idx, max_slots=max_slots), ref, idx)
+
+
+def test_noalloc_gives_the_same_cells(big):
+    for wl in WORKLOADS[:2]:
+        d, ref = big(wl)
+        idx = np.arange(NBIG)
+        same(react(wl, d, idx, noalloc=True), ref, idx)
+
+
+@pytest.mark.parametrize("wl", ["lidryer_32", "drm19_64"])
+def test_big_call_vs_oracle(wl, big, oracle_lib):
+    W = inputs.WORKLOADS[wl]
+    d, out = big(wl)
+    ref = oracle_lib.OracleMech(M.load(W.mech)).react(
+        d["rY"], d["T"], d["rE"], W.dt, rYsrc=d["rYsrc"], rEsrc=d["rEsrc"], mask=d["mask"],
+        rtol=W.rtol, atol=W.atol)
+    on = d["mask"] == 1
+    rho = ref["rY"].sum(0)
+    assert np.abs(out["T"] - ref["T"])[on].max() <= GATE_T
+    assert (np.abs(out["rY"] - ref["rY"]) / rho)[:, on].max() <= GATE_Y
+    np.testing.assert_array_equal(out["rE"][on], (d["rE"] + W.dt * d["rEsrc"])[on])
+
+
+@pytest.mark.parametrize("wl", WORKLOADS)
+def test_singular_newton_matrix(wl):
+    """Every inversion reports a singular matrix: ten convergence failures, the inputs kept."""
+    n = 67
+    d = inputs.make_inputs(wl, n)
+    out = react(wl, d, np.arange(n), **{"prc.test_lu_fail": 1})
+    assert out["nfail"] == n
+    for row, v in ((0, 3), (1, 0), (4, 10), (7, 10)):  # status, steps, set-ups, failures
+        np.testing.assert_array_equal(out["diag"][row], v)
+    for k in ("rY", "T", "rE"):
+        np.testing.assert_array_equal(out[k], d[k])
