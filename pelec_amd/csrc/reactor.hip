@@ -646,6 +646,19 @@ void fill_params(const prc_reactor* r, Args& a, unsigned long long* ctr) {
   a.ctr = ctr;
 }
 
+// ReactorRK64 on a.box: one cell per group of lanes where the mechanism has its tables.
+template <class M = Mech>
+void launch_rk64(const Args& a, const Args* dargs, hipStream_t s) {
+  if constexpr (whole_ok<M>()) {
+    constexpr int CPB = 64 / M::G_W;  // cells per block
+    hipLaunchKernelGGL(react_rk64_g<M>, dim3((unsigned)((a.box.ncells + CPB - 1) / CPB)), dim3(64),
+                       0, s, a);
+  } else {
+    hipLaunchKernelGGL(react_rk64<M>, dim3((unsigned)((a.box.ncells + 63) / 64)), dim3(64), 0, s,
+                       dargs);
+  }
+}
+
 // One react call: a.box (single box) or a.boxes / a.nboxes (device table), a.ncells cells.
 int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_counters = true) {
   if (r->integrator == 1 && r->rk_min > r->rk_max) return PRC_EINVAL;
@@ -671,7 +684,7 @@ int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_coun
     HIP_OK(hipMemcpyAsync(r->d_args, &a, sizeof(Args), hipMemcpyHostToDevice, s));
     const int64_t nb = (a.box.ncells + 63) / 64;
     if (r->integrator == 1)
-      hipLaunchKernelGGL(react_rk64, dim3((unsigned)nb), dim3(64), 0, s, r->d_args);
+      launch_rk64(a, r->d_args, s);
     else if (r->lu_fp32 && r->shape.refine >= 2)
       hipLaunchKernelGGL((react_plain<float, 2>), dim3((unsigned)nb), dim3(64), 0, s, r->d_args);
     else if (r->lu_fp32)

@@ -217,6 +217,7 @@ __global__ void __launch_bounds__(64) react_plain(const Args* __restrict__ ap) {
 
 // ------------------------------------------------------------------ ReactorRK64 drop-in
 // One cell per lane over a static grid of the box, explicit RK64 with error control (rk64.h).
+template <class M>
 __global__ void __launch_bounds__(64) react_rk64(const Args* __restrict__ ap) {
   const Args& a = *ap;
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -230,7 +231,7 @@ __global__ void __launch_bounds__(64) react_rk64(const Args* __restrict__ ap) {
     write_diag(a, g, CELL_OK, nullptr);
     return;
   }
-  Rk64Cell<Mech> cell;
+  Rk64Cell<M> cell;
   double y[NV];
   double rho = 0.0;
 #pragma unroll
@@ -1115,6 +1116,93 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
       ph = CP_FETCH;
     }
   }
+}
+
+// ReactorRK64 (rk64.h's method and step control) with one cell per group of lanes: the registers Q,
+// S and E are one value per lane. A static grid: cells share nothing, so the scheduler is the queue.
+// Bound as k_cell is, by the instruction issue of the right-hand side. One cell per lane holds Q, S, E
+// and the kinetics in private memory and 4096 cells are 64 waves: drm19, dt = 1e-7 s, 4096 cells
+// 17.5 ms, 1.5 ms in groups.
+template <class M>
+__global__ void __launch_bounds__(64) react_rk64_g(const Args a) {
+  using K = GroupKin<M>;
+  constexpr int G = K::G;
+  using Grp = Group<G>;
+  __shared__ __attribute__((aligned(16))) double lds[64 / G * K::RHS_WORDS + XT_WORDS];
+  lds_double* xt = lds_ptr(lds) + 64 / G * K::RHS_WORDS;
+  fill_tables(xt);
+  const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
+  lds_double* sh = lds_ptr(lds) + gid * K::RHS_WORDS;
+  const int64_t c = (int64_t)blockIdx.x * (64 / G) + gid;
+  const BoxDev& b = a.box;
+  if (c >= b.ncells) return;
+  int i, j, k;
+  cell_ijk(b, c, i, j, k);
+  const int64_t g = b.first + c;
+  if (b.mask.p && b.mask.at(i, j, k) == 0) {
+    if (l == 0) {
+      if (b.FC.p) b.FC.at(i, j, k, 0) = 0.0;
+      write_diag(a, g, CELL_OK, nullptr);
+    }
+    return;
+  }
+  double y = l < NSP ? b.rY.at(i, j, k, l) : l == NSP ? b.T.at(i, j, k, 0) : 0.0;
+  const double rhoe0 = b.rE.at(i, j, k, 0);
+  const double rhoesrc = b.rEsrc.p ? b.rEsrc.at(i, j, k, 0) : 0.0;
+  const double srcl = b.rYsrc.p && l < NSP ? b.rYsrc.at(i, j, k, l) : 0.0;
+  if (!(Grp::sum(l < NSP ? y : 0.0) > 0.0) || !(Grp::bcast(y, NSP) > 0.0) || !(a.dt > 0.0)) {
+    if (l == 0) {
+      atomicAdd(&a.ctr[CT_FAILED], 1ull);
+      if (b.FC.p) b.FC.at(i, j, k, 0) = 0.0;
+      write_diag(a, g, CELL_BADINPUT, nullptr);
+    }
+    return;
+  }
+  const Rk64Params& p = a.rk;
+  const double at = l < NV ? p.atolv[l] : 1.0, tm = M::G_TMID[l], dt = a.dt;
+  const double hmin = dt / p.nsub_max, hmax = dt / p.nsub_min, tend_tol = 100.0 * cv::UROUND * dt;
+  double h = dt / p.nsub_guess, t = 0.0;
+  Counters cn{};
+  int status = CELL_OK;
+  while (dt - t > tend_tol) {
+    if (cn.nst + cn.netf >= p.max_steps) {
+      status = CELL_MAXSTEPS;
+      break;
+    }
+    const double hu = (t + h >= dt - tend_tol) ? dt - t : h;
+    double Q = y, S = y, E = 0.0;
+#pragma unroll 1
+    for (int s = 0; s < 6; ++s) {
+      const double f = K::rhs(t + rk::stage_c(s) * hu, S, l, rhoe0, rhoesrc, srcl, tm, sh,
+                              xt);
+      cn.nfe++;
+      E += rk::ERR[s] * hu * f;
+      S = Q + rk::ALPHA[s] * hu * f;
+      Q = S + rk::BETA[s] * hu * f;
+    }
+    const double ei = fabs(E) / (p.rtol * fabs(y) + at);
+    if (K::any(!(isfinite(ei) && isfinite(Q)))) {
+      if (hu <= hmin) {
+        status = CELL_ERRFAIL;
+        break;
+      }
+      cn.netf++;
+      h = fmax(0.2 * hu, hmin);
+      continue;
+    }
+    const double en = Grp::max(ei);
+    const double fac = en > 0.0 ? 0.9 / sqrt(sqrt(en)) : 5.0;
+    if (en <= 1.0 || hu <= hmin) {
+      y = Q;
+      t += hu;
+      cn.nst++;
+      h = fmin(fmax(hu * fmin(fmax(fac, 0.2), 5.0), hmin), hmax);
+    } else {
+      cn.netf++;
+      h = fmax(hu * fmax(fac, 0.2), hmin);
+    }
+  }
+  store_whole<M>(a, g, status, cn, y, l, tm, rhoe0, rhoesrc);
 }
 
 // The compaction check a graph makes between two iterations (the host makes the same check between

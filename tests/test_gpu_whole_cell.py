@@ -133,3 +133,13 @@ def test_singular_newton_matrix(wl):
         np.testing.assert_array_equal(out["diag"][row], v)
     for k in ("rY", "T", "rE"):
         np.testing.assert_array_equal(out[k], d[k])
+
+
+@pytest.mark.parametrize("wl,dt", [("lidryer_32", None), ("drm19_64", 1e-7), ("gri30_flat", 1e-8)])
+def test_rk64_cells_do_not_depend_on_the_call(wl, dt, big):
+    d, _ = big(wl)
+    ref = react(wl, d, np.arange(NBIG), dt=dt, rk64=True)
+    assert ref["nfail"] == 0 and (ref["diag"][1][d["mask"] == 1] > 0).all()
+    for first, n in ((0, 1), (2, 3), (64, 8), (1, 63), (60, 65)):
+        idx = np.arange(first, first + n)
+        same(react(wl, d, idx, dt=dt, rk64=True), ref, idx)
