@@ -141,7 +141,7 @@ struct prc_reactor {
   // lanes, and the waves of k_cell that fit the GPU (0: not looked up yet)
   double* wws = nullptr;
   int64_t wws_groups = 0;
-  int whole_blocks = 0;
+  int whole_blocks = 0, adj_blocks = 0;
   int64_t whole_cells = 0;  // cells in flight of the last whole-cell call (0: the last was not one)
   // PELEC_AMD_TRACE=1: one stderr line per graph replay of the batched form (live-cell counts)
   bool trace = false;
@@ -659,6 +659,51 @@ void launch_rk64(const Args& a, const Args* dargs, hipStream_t s) {
   }
 }
 
+// Adjoint: workspace (doubles; the rate multipliers first) and grid of a call. With the lane-group
+// tables a group of lanes owns a workspace and takes cells in turn; else every cell has its own.
+struct AdjGrid {
+  size_t words = 0, rmul = 0;
+  int blocks = 0, gpw = 1;
+};
+template <class M = Mech>
+int adjoint_grid(prc_reactor* r, int64_t ncells, AdjGrid& g) {
+  const size_t hist = (size_t)r->adj_kmax * CKW + (size_t)r->adj_tcap * TRS;
+  if constexpr (whole_ok<M>() && ADJ_OK) {
+    if (!r->adj_blocks) {
+      int dev = 0, o = 0;
+      HIP_OK(hipGetDevice(&dev));
+      HIP_OK(hipDeviceGetAttribute(&r->ncu, hipDeviceAttributeMultiprocessorCount, dev));
+      HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, k_adjoint_g<M>, 64, 0));
+      r->adj_blocks = std::max(o, 1) * r->ncu;
+    }
+    constexpr int GPW = whole_gpw<M>();
+    const int64_t per = (ncells + r->adj_blocks - 1) / r->adj_blocks;
+    g.gpw = (int)std::min<int64_t>(per, GPW);
+    g.blocks = (int)std::min<int64_t>((ncells + g.gpw - 1) / g.gpw, r->adj_blocks);
+    g.rmul = (size_t)((GroupKin<M>::P + 1) & ~1);
+    g.words = g.rmul + (size_t)g.blocks * GPW * (hist + 2 * GroupKin<M>::JAC_SIZE);
+  } else {
+    g.blocks = (int)((ncells + 63) / 64);
+    g.rmul = (size_t)M::NRXN;
+    g.words = g.rmul + (size_t)ncells * (hist + (size_t)ADJ_MATS * NV * NV);
+  }
+  return PRC_OK;
+}
+template <class M = Mech>
+void launch_adjoint(prc_reactor* r, AdjArgs& a, const AdjGrid& g, const double* logA, double* rmul,
+                    hipStream_t s) {
+  if constexpr (whole_ok<M>() && ADJ_OK) {
+    hipLaunchKernelGGL(k_exp_lanes<M>, dim3((GroupKin<M>::P + 63) / 64), dim3(64), 0, s, logA, rmul);
+    hipLaunchKernelGGL(k_set_counter, dim3(1), dim3(64), 0, s, r->d_ctr, (int)CT_NEXT, 0ull);
+    hipLaunchKernelGGL(k_adjoint_g<M>, dim3(g.blocks), dim3(64), 0, s, a, r->d_ctr + CT_NEXT, g.gpw);
+  } else {
+    a.tape = a.ckpt + (size_t)a.ncells * a.kmax * CKW;
+    a.mats = a.tape + (size_t)a.ncells * a.tcap * TRS;
+    hipLaunchKernelGGL(k_exp, dim3((M::NRXN + 63) / 64), dim3(64), 0, s, (int)M::NRXN, logA, rmul);
+    hipLaunchKernelGGL(k_adjoint<NV>, dim3(g.blocks), dim3(64), 0, s, a);
+  }
+}
+
 // One react call: a.box (single box) or a.boxes / a.nboxes (device table), a.ncells cells.
 int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_counters = true) {
   if (r->integrator == 1 && r->rk_min > r->rk_max) return PRC_EINVAL;
@@ -801,7 +846,7 @@ void release(prc_reactor* r) {
   if (r->wws) (void)hipFree(r->wws);
   r->wws = nullptr;
   r->wws_groups = 0;
-  r->whole_blocks = 0;
+  r->whole_blocks = r->adj_blocks = 0;
   r->whole_cells = 0;
   r->graph_lu_fp32 = -1;
   r->ncu = 0;
@@ -1488,9 +1533,10 @@ int prc_adjoint(prc_reactor* r, int64_t ncells, const double* rY0, const double*
     return PRC_EINVAL;
   if (tape && (tape_cap < 1 || !tape_count)) return PRC_EINVAL;
   hipStream_t s = (hipStream_t)stream;
-  const size_t per_cell =
-      (size_t)r->adj_kmax * CKW + (size_t)r->adj_tcap * TRS + (size_t)ADJ_MATS * NV * NV;
-  const size_t bytes = sizeof(double) * ((size_t)ncells * per_cell + (size_t)Mech::NRXN);
+  AdjGrid ag;
+  e = adjoint_grid(r, ncells, ag);
+  if (e) return e;
+  const size_t bytes = sizeof(double) * ag.words;
   if (bytes > r->aws_bytes) {
     if (r->aws) (void)hipFree(r->aws);
     r->aws = nullptr;
@@ -1522,16 +1568,12 @@ int prc_adjoint(prc_reactor* r, int64_t ncells, const double* rY0, const double*
   a.prm.max_steps = r->max_steps;
   a.seg = r->adj_seg;
   a.kmax = r->adj_kmax;
-  a.ckpt = r->aws + Mech::NRXN;
+  a.ckpt = r->aws + ag.rmul;
   a.tcap = r->adj_tcap;
-  a.tape = a.ckpt + (size_t)ncells * r->adj_kmax * CKW;
-  a.mats = a.tape + (size_t)ncells * r->adj_tcap * TRS;
   a.full_cap = tape ? tape_cap : 0;
   a.full_tape = tape;
   a.full_count = tape_count;
-  hipLaunchKernelGGL(k_exp, dim3((Mech::NRXN + 63) / 64), dim3(64), 0, s, (int)Mech::NRXN, logA,
-                     rmul);
-  hipLaunchKernelGGL(k_adjoint<NV>, dim3((unsigned)((ncells + 63) / 64)), dim3(64), 0, s, a);
+  launch_adjoint(r, a, ag, logA, rmul, s);
   HIP_OK(hipGetLastError());
   return PRC_OK;
 }

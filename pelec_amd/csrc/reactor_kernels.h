@@ -14,6 +14,7 @@
 #include "bdf_cell.h"
 #include "rk64.h"
 #include "adjoint.h"
+#include "adjoint_group.h"
 #include "whole_cell.h"
 
 namespace {
@@ -1325,6 +1326,14 @@ __global__ void k_exp(int n, const double* x, double* y) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = x ? exp(x[i]) : 1.0;
 }
+// the same in the lane groups' order of the reactions (Mech::G_RORD; 1 where there is none)
+template <class M>
+__global__ void k_exp_lanes(const double* x, double* y) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= GroupKin<M>::P) return;
+  const int j = M::G_RORD[p];
+  y[p] = x && j >= 0 ? exp(x[j]) : 1.0;
+}
 
 using AdjCell = BdfCell<Mech, double, GTape<NV>, true, true, true>;
 constexpr int ADJ_MATS = 5;  // savedJ, M, Jx (forward) and J, Mf (backward) per cell
@@ -1485,6 +1494,147 @@ __global__ void __launch_bounds__(64) k_adjoint(const AdjArgs a) {
   for (int k = 0; k < NSP; ++k) a.g_rY0[k * nc + c] = adj.gy0[k];
   a.g_rE0[c] = adj.ge;
   for (int j = 0; j < Mech::NRXN; ++j) a.g_p[j * nc + c] = adj.gp[j];
+  }
+}
+
+// The same with one cell per group of lanes; groups take cells from a counter. Bound by the serial chain
+// of a cell's steps while cells are few, then by instruction issue. One cell per lane kept 15 to
+// 24 KB of private memory per lane and its matrices in device memory, and 512 cells are 8 waves:
+// drm19, dt = 1e-4 s, 512 cells forward and backward 163 -> 2.8 ms, 16,384 cells 10.2 ms.
+template <class M>
+__global__ void __launch_bounds__(64, 2) k_adjoint_g(const AdjArgs a, unsigned long long* next,
+                                                     int gpw) {
+  using K = GroupKin<M>;
+  using C = AdjGroup<M>;
+  constexpr int G = K::G, GPW = 64 / G;
+  using Grp = Group<G>;
+  __shared__ __attribute__((aligned(16))) double lds[GPW * K::WORDS + XT_WORDS];
+  __shared__ BdfScalars scl[GPW];
+  fill_tables(lds_ptr(lds) + GPW * K::WORDS);
+  const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
+  if (gid >= gpw) return;
+  const int64_t nc = a.ncells, w = (int64_t)blockIdx.x * GPW + gid;
+  C cell(scl[gid]);
+  cell.l = l;
+  cell.sh = lds + gid * K::WORDS;
+  cell.xt = lds + GPW * K::WORDS;
+  cell.tm = M::G_TMID[l];
+  cell.at = l < NV ? a.prm.atolv[l] : 1.0;
+  cell.prm = a.prm;
+  cell.rmul = a.rmul;
+  // workspace of the group: checkpoints, segment tape, two Jacobians
+  double* ck = a.ckpt + w * ((int64_t)a.kmax * CKW + (int64_t)a.tcap * TRS + 2 * K::JAC_SIZE);
+  double* tp = ck + (int64_t)a.kmax * CKW;
+  cell.ws = tp + (int64_t)a.tcap * TRS;
+  cell.wx = cell.ws + K::JAC_SIZE;
+  for (;;) {
+    unsigned long long nx = 0;
+    if (l == 0) nx = atomicAdd(next, 1ull);
+    const int64_t c = (int64_t)__shfl(nx, 0, G);
+    if (c >= nc) return;
+    const double y0 = l < NSP ? a.rY0[l * nc + c] : l == NSP ? a.T0[c] : 0.0;
+    cell.rhoe0 = a.rE0[c];
+    cell.rhoesrc = a.rEsrc ? a.rEsrc[c] : 0.0;
+    cell.srcl = a.rYsrc && l < NSP ? a.rYsrc[l * nc + c] : 0.0;
+    cell.ge = cell.gy0 = 0.0;
+#pragma unroll
+    for (int r = 0; r < K::RR; ++r) cell.gp[r] = 0.0;
+    // status st with the state yl, T and the gradients held in `cell`
+    auto finish = [&](int st, double yl, double T) {
+      if (l < NSP) {
+        a.rY_out[l * nc + c] = yl;
+        a.g_rY0[l * nc + c] = cell.gy0;
+      }
+      if (l == 0) {
+        a.status[c] = st;
+        a.T_out[c] = T;
+        a.g_rE0[c] = cell.ge;
+      }
+#pragma unroll
+      for (int r = 0; r < K::RR; ++r) {
+        const int j = M::G_RORD[G * r + l];
+        if (j >= 0) a.g_p[j * nc + c] = cell.gp[r];
+      }
+    };
+    auto fail = [&](int st) {
+      cell.ge = cell.gy0 = 0.0;
+#pragma unroll
+      for (int r = 0; r < K::RR; ++r) cell.gp[r] = 0.0;
+      finish(st, y0, Grp::bcast(y0, NSP));
+    };
+    if (!(Grp::sum(l < NSP ? y0 : 0.0) > 0.0) || !(Grp::bcast(y0, NSP) > 0.0) || !(a.dt > 0.0)) {
+      fail(CELL_BADINPUT);
+      continue;
+    }
+    // forward pass
+    cell.base = a.full_tape ? a.full_tape + c * a.full_cap * TRS : nullptr;
+    cell.cap = (int)a.full_cap;
+    cell.count = 0;
+    cell.overflow = false;
+    cell.last_correct = nullptr;
+    cell.start(y0, a.dt);
+    int st;
+    do {
+      st = cell.advance();
+      if (st < 0 && cell.S.nst % a.seg == 0) {
+        const int k = cell.S.nst / a.seg;
+        if (k >= a.kmax) {
+          st = CELL_ADJ_STORAGE;
+          break;
+        }
+        cell.save(ck + (int64_t)k * CKW);
+      }
+    } while (st < 0);
+    if (a.full_tape && l == 0) a.full_count[c] = cell.overflow ? -1 : cell.count;
+    if (st != CELL_OK) {
+      fail(st);
+      continue;
+    }
+    const int nst = cell.S.nst;
+    const double yend = cell.z[0];
+    const double irho = 1.0 / Grp::sum(l < NSP ? yend : 0.0);
+    double ec[6], ek, cvk;
+    const double Tend = K::T_from_e((cell.rhoe0 + a.dt * cell.rhoesrc) * irho,
+                                    l < NSP ? yend * irho : 0.0, l, Grp::bcast(yend, NSP), cell.tm,
+                                    ec, ek, cvk);
+    if (!a.ct_rY && !a.ct_T) {  // no cotangents: forward only
+      finish(CELL_OK, yend, Tend);
+      continue;
+    }
+    // backward pass, from the cotangents of rhoY_end and of T_end = T(e_end, Y_end)
+    const double D = Grp::sum(l < NSP ? yend * cvk : 0.0);
+    const double ctT = a.ct_T ? a.ct_T[c] : 0.0;
+#pragma unroll
+    for (int j = 1; j <= BDF_QMAX; ++j) cell.lam[j] = 0.0;
+    cell.lam[0] = l < NSP ? (a.ct_rY ? a.ct_rY[l * nc + c] : 0.0) - ctT * ek / D : 0.0;
+    cell.ge = ctT / D;
+    const int nseg = (nst + a.seg - 1) / a.seg;
+    bool ok = true;
+    for (int s = nseg - 1; s >= 0 && ok; --s) {
+      cell.base = tp;
+      cell.cap = a.tcap;
+      cell.count = 0;
+      cell.overflow = false;
+      cell.last_correct = nullptr;
+      if (s == 0) {
+        cell.start(y0, a.dt);  // records the initial z_1 = h0 f(0, y0)
+      } else {
+        cell.load(ck + (int64_t)s * CKW);
+        cell.tstop = a.dt;
+      }
+      const int target = min((s + 1) * a.seg, nst);
+      while (cell.S.nst < target)
+        if (cell.advance() >= 0) break;
+      ok = !cell.overflow && cell.S.nst == target;
+      // the tape was written by other lanes of the group
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+      Grp::sync();
+      for (int r = cell.count - 1; r >= 0 && ok; --r) cell.back(tp + (int64_t)r * TRS);
+    }
+    if (ok)
+      finish(CELL_OK, yend, Tend);
+    else
+      fail(CELL_ADJ_STORAGE);
   }
 }
 

@@ -143,3 +143,33 @@ def test_rk64_cells_do_not_depend_on_the_call(wl, dt, big):
     for first, n in ((0, 1), (2, 3), (64, 8), (1, 63), (60, 65)):
         idx = np.arange(first, first + n)
         same(react(wl, d, idx, dt=dt, rk64=True), ref, idx)
+
+
+@pytest.mark.parametrize("mech,wl", [("LiDryer", "lidryer_32"), ("drm19", "drm19_adj")])
+def test_adjoint_cells_do_not_depend_on_the_call(mech, wl):
+    W = inputs.WORKLOADS[wl]
+    d = inputs.make_inputs(wl, 130)
+    rng = np.random.default_rng(5)
+    rho = d["rY"].sum(0)
+    d = dict(d, ct_rY=rng.normal(size=d["rY"].shape) / rho, ct_T=rng.normal(size=rho.size) / 1000.0,
+             rYsrc=rng.normal(0, 1e-4, d["rY"].shape) * d["rY"], rEsrc=rng.normal(0, 1e8, rho.size))
+    logA = rng.normal(0, 0.05, M.load(mech).nrxn)
+
+    def go(idx):
+        r = Reactor(mech)
+        r.configure(rtol=W.rtol, atol=W.atol)
+        x = {k: to_dev(d[k][..., idx]) for k in d if k in
+             ("rY", "T", "rE", "ct_rY", "ct_T", "rYsrc", "rEsrc")}
+        out = r.adjoint(x["rY"], x["T"], x["rE"], W.dt, logA=to_dev(logA), ct_rY=x["ct_rY"],
+                        ct_T=x["ct_T"], rYsrc=x["rYsrc"], rEsrc=x["rEsrc"])
+        torch.cuda.synchronize()
+        res = {k: v.cpu().numpy() for k, v in out.items() if v is not None}
+        r.close()
+        return res
+
+    ref = go(np.arange(130))
+    assert (ref["status"] == 0).all()
+    for first, n in ((0, 1), (5, 2), (1, 63), (63, 65)):
+        idx = np.arange(first, first + n)
+        for k, v in go(idx).items():
+            np.testing.assert_array_equal(v, ref[k][..., idx], err_msg=f"{k} {first} {n}")
