@@ -134,6 +134,7 @@ struct prc_reactor {
   hipGraphExec_t graph_tail = nullptr;  // Shape::tail_slots: the graph with k_newton_g
   int graph_lu_fp32 = -1;
   Shape shape, graph_shape;
+  bool coop_set = false;  // prc.cooperative or prc.coop_tail_slots was set (or autotuned)
   int ncu = 0;
   int occ_newton = 1, occ_jac = 1, occ_lu = 1, occ_tail = 1;
   int64_t last_iterations = 0;
@@ -432,6 +433,28 @@ int eager_accumulate(prc_reactor* r) {
   return PRC_OK;
 }
 
+// The queue's kernels when neither prc.cooperative nor prc.coop_tail_slots was set: the cooperative
+// Jacobian, and the cooperative Newton kernel while at most this many slots are in use. One cell per
+// lane pays off only once its waves fill the GPU: drm19, FP32 factors, 5001 cells take 127 ms with one
+// cell per lane throughout, 28 ms in groups; 65,536 cells 208 and 78 ms; 262,144 cells 320 and 297 ms,
+// 175 ms with the switch. H2/air (a third of the work per iteration) crosses between 5001 cells
+// (5.5 and 3.5 ms) and 32,768 (6.6 and 11.7 ms).
+constexpr int AUTO_TAIL_SLOTS = NV <= 16 ? 12288 : 65536;
+
+// The handle's shape with that choice made, for the length of a call.
+struct ShapeInUse {
+  prc_reactor* r;
+  Shape set;
+  explicit ShapeInUse(prc_reactor* h) : r(h), set(h->shape) {
+    if (COOP && !r->coop_set) {
+      r->shape.coop = 2;
+      r->shape.tail_slots = AUTO_TAIL_SLOTS;
+      r->shape.bpc_tail = std::max(set.bpc_tail, 8);
+    }
+  }
+  ~ShapeInUse() { r->shape = set; }
+};
+
 // The batched form of one call. `dargs` / `dctr` are the device argument block and counters
 // (the handle's, or the no-allocation entry point's scratch). With `graphs`, iterations run as
 // replays of the handle's captured graphs, which read the handle's argument block; without, they
@@ -439,6 +462,7 @@ int eager_accumulate(prc_reactor* r) {
 template <typename LUT>
 int run_batched(prc_reactor* r, Args& a, hipStream_t s, Args* dargs, unsigned long long* dctr,
                 bool graphs) {
+  const ShapeInUse in_use(r);
   if (r->graph_lu_fp32 != r->lu_fp32 || !r->ncu || !(r->graph_shape == r->shape)) {
     const int e = occupancy_setup<LUT>(r);
     if (e) return e;
@@ -1005,10 +1029,11 @@ int prc_set_param_int(prc_reactor* r, const char* key, int v) {
   } else if (!std::strcmp(key, "prc.cooperative")) {
     if (v < 0 || v > 3 || (v && !COOP)) return PRC_EINVAL;
     r->shape.coop = v;
+    r->coop_set = true;
   } else if (!std::strcmp(key, "prc.coop_tail_slots")) {
     if (v < 0 || (v && !COOP)) return PRC_EINVAL;
     r->shape.tail_slots = v;
-
+    r->coop_set = true;
   } else if (!std::strcmp(key, "prc.blocks_tail")) {
     if (v < 0 || v > 64) return PRC_EINVAL;
     r->shape.bpc_tail = v;
@@ -1354,13 +1379,16 @@ int prc_autotune(prc_reactor* r, int64_t ncells, const double* rY, const double*
   int rc = PRC_OK;
   double best = 0.0;
   {
-    // occupancy-derived defaults are the starting point
+    // occupancy-derived defaults are the starting point; every candidate says which kernels it runs
     Shape base = r->shape;
+    const bool base_set = r->coop_set;
+    r->coop_set = true;
     if (!r->ncu) rc = queue_occupancy(r);
     if (!rc) rc = measure(best);
     Shape cur = r->shape;
     if (WHOLE && !r->lu_fp32) {
       // one launch whose grid follows from the occupancy: no shape to search
+      r->coop_set = base_set;
       r->diag = diag;
       r->diag_cap = diag_cap;
       (void)hipEventDestroy(e0);
@@ -1421,6 +1449,7 @@ int prc_autotune(prc_reactor* r, int64_t ncells, const double* rY, const double*
       }
     }
     r->shape = rc ? base : cur;
+    if (rc) r->coop_set = base_set;
   }
   r->diag = diag;
   r->diag_cap = diag_cap;

@@ -173,3 +173,21 @@ def test_adjoint_cells_do_not_depend_on_the_call(mech, wl):
         idx = np.arange(first, first + n)
         for k, v in go(idx).items():
             np.testing.assert_array_equal(v, ref[k][..., idx], err_msg=f"{k} {first} {n}")
+
+
+@pytest.mark.parametrize("n", [1, 12288, 12289])
+def test_fp32_queue_shape_of_its_own(n, oracle_lib):
+    """FP32 factors with neither prc.cooperative nor prc.coop_tail_slots set: H2/air cells run in
+    groups from the start up to 12,288 slots, one per lane until that many are left above; both sides
+    of the line meet the gate, and an explicit choice stands."""
+    wl = "lidryer_32"
+    W = inputs.WORKLOADS[wl]
+    d = inputs.make_inputs(wl, n)
+    ref = oracle_lib.OracleMech(M.load(W.mech)).react(d["rY"], d["T"], d["rE"], W.dt, rtol=W.rtol,
+                                                      atol=W.atol)
+    rho = ref["rY"].sum(0)
+    for kw in ({}, {"cooperative": 0}):
+        out = react(wl, d, np.arange(n), lu_fp32=True, **kw)
+        assert out["nfail"] == 0
+        assert np.abs(out["T"] - ref["T"]).max() <= GATE_T
+        assert (np.abs(out["rY"] - ref["rY"]) / rho).max() <= GATE_Y
