@@ -116,12 +116,21 @@ def _parse_side(side: str, names: Dict[str, int]):
     return out, collider
 
 
-def load(name_or_path: str) -> Mechanism:
+def source(name_or_path: str) -> bytes:
+    """The mechanism file's contents."""
     path = name_or_path
     if not os.path.exists(path):
         path = os.path.join(MECH_DIR, f"{name_or_path}.yaml")
     with open(path, "rb") as f:
-        raw = f.read()
+        return f.read()
+
+
+def load(name_or_path: str) -> Mechanism:
+    return parse(source(name_or_path))
+
+
+def parse(raw: bytes) -> Mechanism:
+    """The mechanism in a file of these contents."""
     doc = yaml.safe_load(raw)
     units = doc.get("units", {})
     if units.get("activation-energy", "cal/mol") != "cal/mol":
