@@ -583,6 +583,8 @@ constexpr int WHOLE_WAVES = NV <= 32 ? 3 : 2;
 // Grid of a call: one wave per block, as many as fit the GPU at once. With fewer cells than groups
 // of lanes each wave takes fewer cells at a time (gpw): the groups of a wave run in lockstep, so a
 // cell alone on its wave never waits for another cell's phases, and the spare waves cost nothing.
+// One cell per wave against full waves: 700 drm19 cells 3.20 and 3.38 ms, 512 H2/air cells 0.52 and
+// 0.54 ms, 3000 (as many waves as fit) 0.64 and 0.62 ms.
 struct WholeGrid {
   int blocks = 0, gpw = 0;
   int64_t groups = 0;  // groups of lanes that own workspace
