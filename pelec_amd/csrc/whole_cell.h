@@ -96,6 +96,11 @@ __device__ inline double flog(double x, const lds_double* xt) {
   return fma((double)e, 0.69314718055994530942, l) + q;
 }
 
+// The kinetics are inlined wherever they are used: as soon as two kernels of a library call them the
+// compiler makes them functions, and a call in k_cell's loop costs 100 to 140 B of scratch per lane
+// (drm19, 65,536 cells: 15.1 ms against 13.5).
+#define PELEC_INLINE __device__ __forceinline__
+
 // What jac() leaves beside the matrix: the lane's e_k, rho c_v, and df/d(rho e0) of its component.
 struct JacOut {
   double ek, D, fe;
@@ -131,18 +136,18 @@ struct GroupKin {
   static constexpr int JAC_SIZE = Mech::G_JC * G;
 
   // Jacobian elements are written by whichever lane sums them and read by their row's lane: from the L2.
-  __device__ static double load_l2(const double* p) {
+  PELEC_INLINE static double load_l2(const double* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
   // any lane of the caller's group
-  __device__ static bool any(bool p) {
+  PELEC_INLINE static bool any(bool p) {
     const unsigned long long b = __ballot(p);
     if constexpr (G == 64) return b != 0ull;
     const unsigned long long m = ((1ull << (G & 63)) - 1ull) << (threadIdx.x & 63 & ~(G - 1));
     return (b & m) != 0ull;
   }
-  __device__ static void load_e(double (&c)[6], bool lo, int l) {
+  PELEC_INLINE static void load_e(double (&c)[6], bool lo, int l) {
     const dv2* p = reinterpret_cast<const dv2*>(&Mech::G_E[lo ? 0 : 1][0][l][0]);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -151,7 +156,7 @@ struct GroupKin {
       c[2 * i + 1] = v.y;
     }
   }
-  __device__ static void e_cv(const double (&c)[6], double T, double& e, double& cv) {
+  PELEC_INLINE static void e_cv(const double (&c)[6], double T, double& e, double& cv) {
     e = fma(T, fma(T, fma(T, fma(T, fma(T, c[5], c[4]), c[3]), c[2]), c[1]), c[0]);
     cv = fma(T, fma(T, fma(T, fma(T, 5.0 * c[5], 4.0 * c[4]), 3.0 * c[3]), 2.0 * c[2]), c[1]);
   }
@@ -160,7 +165,7 @@ struct GroupKin {
   // The iteration also ends after |dT| <= 1e-7 T: it converges quadratically, so the next
   // correction would be below (cv'/2cv) dT^2 ~ 1e-14 T -- unless a species' fit changed branch.
   // On return ec holds the lane's coefficients at T and ek, cvk are evaluated at T.
-  __device__ static double T_from_e(double e, double Yl, int l, double T, double tm,
+  PELEC_INLINE static double T_from_e(double e, double Yl, int l, double T, double tm,
                                     double (&ec)[6], double& ek, double& cvk) {
     bool lo = T < tm;
     load_e(ec, lo, l);
@@ -188,14 +193,14 @@ struct GroupKin {
     double ear;
     uint64_t pk;
   };
-  __device__ static Record record(int p) {
+  PELEC_INLINE static Record record(int p) {
     return Record{reinterpret_cast<const dv2*>(&Mech::G_RA[0][0])[p], Mech::G_RE[p],
                   Mech::G_RP[p]};
   }
 
   // Reaction at position p (lane l of a round). JAC: also its derivatives into rb (8 x G).
   template <bool JAC, bool MUL>
-  __device__ static void reaction(const Record& rc_, int p, int l, double T, double lnT,
+  PELEC_INLINE static void reaction(const Record& rc_, int p, int l, double T, double lnT,
                                   double invT, lds_double* sh, const lds_double* xt,
                                   const double* rmul) {
     const dv2 ab = rc_.ab;
@@ -296,7 +301,7 @@ struct GroupKin {
   }
 
   // Species thermo of lane l into LDS and the third-body sums: what the reactions read.
-  __device__ static void load_g(double (&c)[8], bool lo, int l) {
+  PELEC_INLINE static void load_g(double (&c)[8], bool lo, int l) {
     const dv2* p = reinterpret_cast<const dv2*>(&Mech::G_G[lo ? 0 : 1][0][l][0]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -307,7 +312,7 @@ struct GroupKin {
   }
   // c: the g/RT coefficients of branch lo0, loaded before T was known
   template <bool JAC>
-  __device__ static void prelude(double T, double lnT, double invT, double Cl, int l, double tm,
+  PELEC_INLINE static void prelude(double T, double lnT, double invT, double Cl, int l, double tm,
                                  double (&c)[8], bool lo0, lds_double* sh, const lds_double* xt) {
     const bool lo = T < tm;
     if (any(lo != lo0)) load_g(c, lo, l);
@@ -342,12 +347,12 @@ struct GroupKin {
 
   // production rate of species l from the q in LDS: a chunk of entries per lane, then the chunks
   // of each species
-  __device__ static void load_gather(uv4 (&e)[Mech::G_L8], int l) {
+  PELEC_INLINE static void load_gather(uv4 (&e)[Mech::G_L8], int l) {
 #pragma unroll
     for (int i = 0; i < Mech::G_L8; ++i)
       e[i] = *reinterpret_cast<const uv4*>(&Mech::G_GE[i][l][0]);
   }
-  __device__ static double gather(const uv4 (&e)[Mech::G_L8], int l, lds_double* sh) {
+  PELEC_INLINE static double gather(const uv4 (&e)[Mech::G_L8], int l, lds_double* sh) {
     double acc = 0.0;
     const lds_char* q = (const lds_char*)(sh + O_Q);
 #pragma unroll
@@ -371,13 +376,13 @@ struct GroupKin {
   }
 
   // log of a temperature (NaN where it is not one)
-  __device__ static double log_T(double T, const lds_double* xt) {
+  PELEC_INLINE static double log_T(double T, const lds_double* xt) {
     return T > 0.0 ? flog(T, xt) : __builtin_nan("");
   }
 
   // f(t, y) for the lane's component (0 on lanes >= n).
   template <bool MUL = false>
-  __device__ static double rhs(double t, double yl, int l, double rhoe0, double rhoesrc,
+  PELEC_INLINE static double rhs(double t, double yl, int l, double rhoe0, double rhoesrc,
                                double srcl, double tm, lds_double* sh, const lds_double* xt,
                                const double* rmul = nullptr) {
     l = after(l, yl);
@@ -419,7 +424,7 @@ struct GroupKin {
   // per SIMD) or an L2 atomic per term (107 k to 312 k cycles a Jacobian, n = 22 to 54; 34 k to 65 k
   // this way).
   template <bool MUL = false>
-  __device__ static JacOut jac(double t, double yl, int l, double rhoe0, double rhoesrc, double srcl,
+  PELEC_INLINE static JacOut jac(double t, double yl, int l, double rhoe0, double rhoesrc, double srcl,
                              double tm, lds_double* sh, const lds_double* xt, double* ws,
                              const double* rmul = nullptr) {
     l = after(l, yl);
@@ -516,12 +521,12 @@ struct GroupKin {
 
   // a b + c into a register of its own: the row shift of invert() would otherwise cost a move per
   // column (the compiler prefers the two-address form).
-  __device__ static double fma3(double a, double b, double c) {
+  PELEC_INLINE static double fma3(double a, double b, double c) {
     double r;
     __asm__("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
   }
-  __device__ static double fma3_uniform(double a, double b, double c) {  // b in scalar registers
+  PELEC_INLINE static double fma3_uniform(double a, double b, double c) {  // b in scalar registers
     double r;
     __asm__("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
     return r;
@@ -529,7 +534,7 @@ struct GroupKin {
 
   // The group's pivot for a column: the largest of the rows' high words of |a| with the lane in the
   // low six bits (used rows: the lane alone), so the pivot is within 2^-14 of the largest entry.
-  __device__ static unsigned pivot_key(double a, bool used, int l) {
+  PELEC_INLINE static unsigned pivot_key(double a, bool used, int l) {
     const unsigned hi = (unsigned)__double2hiint(a) & 0x7fffffc0u;
     unsigned x = (used ? 0u : hi) | (unsigned)l;
     if constexpr (G > 32) {
@@ -556,7 +561,7 @@ struct GroupKin {
   // other rows' multipliers carry 1 / pivot. Measured: GRI-Mech 3.0 (n = 54), 16,384 cells, 25.4 ms
   // through LDS, 23.0 ms by v_readlane; four cells per wave (n = 10) 7.7 k cycles an inversion
   // through LDS, 11.5 k by v_readlane. Returns 0, or k + 1 when column k has no usable pivot.
-  __device__ static int invert(double (&a)[n], int l, int& kap, lds_double* sh) {
+  PELEC_INLINE static int invert(double (&a)[n], int l, int& kap, lds_double* sh) {
     l = after(l, a[0]);
     [[maybe_unused]] lds_dv2* pr = (lds_dv2*)(sh + O_PR);
     bool used = l >= n;
@@ -631,7 +636,7 @@ struct GroupKin {
   }
 
   // x_l of M x = b from invert()'s rows; b_l on lane l (0 on lanes >= n).
-  __device__ static double solve(const double (&a)[n], int kap, double b, int l, lds_double* sh) {
+  PELEC_INLINE static double solve(const double (&a)[n], int kap, double b, int l, lds_double* sh) {
     lds_double* v = sh + O_V;
     if (l < n) v[kap] = b;
     Grp::sync();
