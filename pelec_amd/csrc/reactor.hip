@@ -142,6 +142,8 @@ struct prc_reactor {
   // lanes, and the waves of k_cell that fit the GPU (0: not looked up yet)
   double* wws = nullptr;
   int64_t wws_groups = 0;
+  void* ord = nullptr;  // order_bytes() of the largest call so far
+  size_t ord_bytes = 0;
   int whole_blocks = 0, adj_blocks = 0;
   int64_t whole_cells = 0;  // cells in flight of the last whole-cell call (0: the last was not one)
   // PELEC_AMD_TRACE=1: one stderr line per graph replay of the batched form (live-cell counts)
@@ -628,9 +630,32 @@ constexpr size_t whole_bytes() {
     return 0;
 }
 
+// Workspace of the cells' order (k_cell_keys): counts, keys and the order itself. 0: the cells go in the
+// order they come in -- all of them are in flight at once, or n <= 16, where costs differ little (H2/air
+// 32^3: the longest cell takes 1.5 times the mean, with drm19 6 times) and the rate says nothing about
+// them. Without and with, ms: drm19 64^3 47.0 and 43.7, GRI-Mech 3.0, 16,384 cells, 22.3 and 19.9,
+// dodecane_lu, 8192 cells, 36.2 and 33.9; H2/air 32^3 1.93 and 1.95.
+size_t order_bytes(int64_t ncells, const WholeGrid& w) {
+  if (NV <= 16 || ncells <= (int64_t)w.blocks * w.gpw || ncells > INT32_MAX) return 0;
+  const size_t n = (size_t)((ncells + 15) & ~15);
+  return 2 * CELL_KEYS * sizeof(unsigned) + n * (sizeof(int32_t) + sizeof(uint8_t));
+}
+
+// `ord`: order_bytes() of workspace, or null: no order.
 template <class M = Mech>
-int run_whole(prc_reactor* r, Args& a, hipStream_t s, const WholeGrid& w, double* J) {
+int run_whole(prc_reactor* r, Args& a, hipStream_t s, const WholeGrid& w, double* J, void* ord) {
   if constexpr (whole_ok<M>()) {
+    int32_t* order = nullptr;
+    if (ord) {
+      unsigned* hist = static_cast<unsigned*>(ord);
+      order = reinterpret_cast<int32_t*>(hist + 2 * CELL_KEYS);
+      uint8_t* key = reinterpret_cast<uint8_t*>(order + ((a.ncells + 15) & ~15));
+      const unsigned nb = (unsigned)((a.ncells + CELLS_PER_BLOCK - 1) / CELLS_PER_BLOCK);
+      hipLaunchKernelGGL(k_cell_keys<M>, dim3(r->whole_blocks), dim3(64), 0, s, a, key, hist);
+      hipLaunchKernelGGL(k_cell_count, dim3(nb), dim3(CELL_KEYS), 0, s, key, a.ncells, hist);
+      hipLaunchKernelGGL(k_cell_order, dim3(nb), dim3(CELL_KEYS), 0, s, key, a.ncells, hist, order);
+      HIP_OK(hipGetLastError());
+    }
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (r->kernel_timing) {
       while (r->kt_ev.size() < 2) {
@@ -644,7 +669,7 @@ int run_whole(prc_reactor* r, Args& a, hipStream_t s, const WholeGrid& w, double
     hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(64), 0, s, a.ctr, (int64_t)0, 0);
     if (e0) HIP_OK(hipEventRecord(e0, s));
     hipLaunchKernelGGL((k_cell<M, WHOLE_WAVES>), dim3(w.blocks), dim3(64), 0, s, a,
-                       CellArgs{J, w.gpw});
+                       CellArgs{J, w.gpw, order});
     HIP_OK(hipGetLastError());
     if (e1) HIP_OK(hipEventRecord(e1, s));
     HIP_OK(hipStreamSynchronize(s));
@@ -782,7 +807,18 @@ int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_coun
     a.has_src = has_src ? 1 : 0;
     a.test_lu_fail = r->test_lu_fail;
     r->whole_cells = (int64_t)w.blocks * w.gpw;
-    return run_whole(r, a, s, w, r->wws);
+    // (without memory for an order the cells go as they come)
+    const size_t ob = order_bytes(a.ncells, w);
+    if (ob > r->ord_bytes) {
+      if (r->ord) (void)hipFree(r->ord);
+      r->ord = nullptr;
+      r->ord_bytes = 0;
+      if (hipMalloc(&r->ord, ob) == hipSuccess)
+        r->ord_bytes = ob;
+      else
+        (void)hipGetLastError();
+    }
+    return run_whole(r, a, s, w, r->wws, ob ? r->ord : nullptr);
   }
   r->whole_cells = 0;
   e = ensure_workspace(r, a.ncells, has_src);
@@ -872,6 +908,9 @@ void release(prc_reactor* r) {
   if (r->wws) (void)hipFree(r->wws);
   r->wws = nullptr;
   r->wws_groups = 0;
+  if (r->ord) (void)hipFree(r->ord);
+  r->ord = nullptr;
+  r->ord_bytes = 0;
   r->whole_blocks = r->adj_blocks = 0;
   r->whole_cells = 0;
   r->graph_lu_fp32 = -1;
@@ -1231,7 +1270,11 @@ int prc_react_flat_noalloc(prc_reactor* r, double* rY, const double* rYsrc, doub
     const int64_t fit = (int64_t)((NOALLOC_SCRATCH_BYTES - o_ws) / whole_bytes()) / whole_gpw();
     w.blocks = (int)std::min<int64_t>(w.blocks, fit);
     if (w.blocks < 1) return PRC_ENOMEM;
-    e = run_whole(r, a, s, w, reinterpret_cast<double*>(base + o_ws));
+    // the cells' order where the array has room for it beside the groups' workspace
+    const size_t o_ord = o_ws + whole_bytes() * whole_gpw() * (size_t)w.blocks;
+    const size_t ob = order_bytes(ncells, w);
+    e = run_whole(r, a, s, w, reinterpret_cast<double*>(base + o_ws),
+                  ob && o_ord + ob <= NOALLOC_SCRATCH_BYTES ? base + o_ord : nullptr);
     if (e) return e;
     HIP_OK(hipMemcpyAsync(r->d_ctr, dctr, CT_COUNT * sizeof(unsigned long long),
                           hipMemcpyDeviceToDevice, s));

@@ -101,6 +101,25 @@ def test_refilled_groups(wl, max_slots, big):
     same(react(wl, d, idx, max_slots=max_slots), ref, idx)
 
 
+@pytest.mark.parametrize("n", [1001, 4096, 4097])
+def test_cells_in_order_of_their_rates(n):
+    """More cells than groups (prc.max_slots), counted and placed by one and two blocks of the counting
+    sort, masked and bad-input cells among them, against the call that has them all in flight."""
+    wl = "drm19_64"
+    d = dict(inputs.make_inputs(wl, n))
+    d["mask"] = (np.random.default_rng(8).uniform(size=n) > 0.5).astype(np.int32)
+    d["mask"][700] = 1
+    d["T"] = d["T"].copy()
+    d["T"][700] = -1.0
+    idx = np.arange(n)
+    ref = react(wl, d, idx)
+    assert ref["nfail"] == 1 and ref["diag"][0][700] != 0
+    for noalloc in (False, True):
+        out = react(wl, d, idx, max_slots=1000, noalloc=noalloc)
+        assert out["nfail"] == 1
+        same(out, ref, idx)
+
+
 def test_noalloc_gives_the_same_cells(big):
     for wl in WORKLOADS[:2]:
         d, ref = big(wl)
