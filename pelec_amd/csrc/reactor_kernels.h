@@ -1034,13 +1034,12 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
   const RegV<NV, G> v{{}, z, ac, ew, l < NV ? a.prm.atolv[l] : 1.0};
   int ph = gid < ca.gpw ? CP_FETCH : CP_IDLE;
   int kap = 0;
-  int64_t g = 0;
-  double rhoe0 = 0.0, rhoesrc = 0.0, srcl = 0.0;
+  double srcl = 0.0;
   for (;;) {
     while (ph == CP_FETCH) {
       unsigned long long nx = 0;
       if (l == 0) nx = atomicAdd(&a.ctr[CT_NEXT], 1ull);
-      g = (int64_t)__shfl(nx, 0, G);
+      int64_t g = (int64_t)__shfl(nx, 0, G);
       if (g >= a.ncells) {
         ph = CP_IDLE;
         break;
@@ -1060,11 +1059,12 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
         }
         continue;
       }
-      rhoe0 = c.rhoe0;
-      rhoesrc = c.rhoesrc;
       srcl = c.src;
       Grp::sync();
       scalars_reset(S, a.prm.qmax);
+      cs.g = g;
+      cs.rhoe0 = c.rhoe0;
+      cs.rhoesrc = c.rhoesrc;
       z[0] = c.y;
 #pragma unroll
       for (int e = 1; e <= BDF_QMAX; ++e) z[e] = 0.0;
@@ -1090,7 +1090,7 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
         t += cs.hg;
       }
       LaneVal f;
-      f.x = K::rhs(t, yl, l, rhoe0, rhoesrc, srcl, tm, sh, xt);
+      f.x = K::rhs(t, yl, l, cs.rhoe0, cs.rhoesrc, srcl, tm, sh, xt);
       S.nfe++;
       if (ph == CP_NEWTON) {
         const int r = newton_correct<NV>(S, v, f, [&](LaneVal& b) {
@@ -1185,7 +1185,7 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
     if (att) predict<NV>(S, v, a.dt);
     if (att || nxt) need_setup |= attempt_setup<RegV<NV, G>>(S);
     if (need_setup) {
-      if (jac_decide(S)) K::jac(S.tn, z[0], l, rhoe0, rhoesrc, srcl, tm, sh, xt, Jg);
+      if (jac_decide(S)) K::jac(S.tn, z[0], l, cs.rhoe0, cs.rhoesrc, srcl, tm, sh, xt, Jg);
       const double gamma = S.gamma;
       // (the columns' addresses and the diagonal's masks are formed here, not kept across the cell loop)
       const int lo = after(l, gamma);
@@ -1209,7 +1209,7 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
       }
     }
     if (status >= 0) {
-      store_whole<M>(a, g, status, counters(S), z[0], l, tm, rhoe0, rhoesrc);
+      store_whole<M>(a, cs.g, status, counters(S), z[0], l, tm, cs.rhoe0, cs.rhoesrc);
       ph = CP_FETCH;
     }
   }

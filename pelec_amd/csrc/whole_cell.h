@@ -310,10 +310,29 @@ struct GroupKin {
       c[2 * i + 1] = v.y;
     }
   }
+  // Concentrations into LDS and the third-body sums, which need no temperature.
+  PELEC_INLINE static void third_bodies(double Cl, int l, lds_double* sh) {
+    if (l <= N) sh[O_RP + 2 * l] = l < N ? Cl : 1.0;
+    if (l == 0) sh[O_Q + P] = 0.0;
+    if constexpr (NS > 0) {
+      double md[Mech::G_MN];
+      int mi[Mech::G_MN];
+#pragma unroll
+      for (int e = 0; e < Mech::G_MN; ++e) {  // (0 on lanes without a set)
+        md[e] = Mech::G_MD[e][l];
+        mi[e] = Mech::G_MI[e][l];
+      }
+      double M = Grp::sum(Cl);
+      Grp::sync();
+#pragma unroll
+      for (int e = 0; e < Mech::G_MN; ++e) M += md[e] * sh[O_RP + 2 * mi[e]];
+      if (l < NS) sh[O_M + l] = M;
+    }
+  }
   // c: the g/RT coefficients of branch lo0, loaded before T was known
   template <bool JAC>
   PELEC_INLINE static void prelude(double T, double lnT, double invT, double Cl, int l, double tm,
-                                 double (&c)[8], bool lo0, lds_double* sh, const lds_double* xt) {
+                                   double (&c)[8], bool lo0, lds_double* sh, const lds_double* xt) {
     const bool lo = T < tm;
     if (any(lo != lo0)) load_g(c, lo, l);
     const double gRT = fma(T, fma(T, fma(T, fma(T, c[4], c[3]), c[2]), c[1]), c[0]) - c[5] * lnT +
@@ -321,25 +340,12 @@ struct GroupKin {
     const double E = fexp(gRT, xt);
     const double iE = recip(E);  // lanes >= N: coefficients 0, so E = iE = 1
     if (l <= N) {
-      const double C = l < N ? Cl : 1.0;
-      ((lds_dv2*)(sh + O_RP))[l] = dv2{C, iE};
-      ((lds_dv2*)(sh + O_PP))[l] = dv2{C, E};
+      sh[O_RP + 2 * l + 1] = iE;
+      ((lds_dv2*)(sh + O_PP))[l] = dv2{l < N ? Cl : 1.0, E};
       if (JAC) {
         const dv2* p = reinterpret_cast<const dv2*>(&Mech::G_H[lo ? 0 : 1][0][l][0]);
         const dv2 h0 = p[0], h1 = p[G], h2 = p[2 * G];
         sh[O_HR + l] = fma(T, fma(T, fma(T, fma(T, h2.x, h1.y), h1.x), h0.y), h0.x) + h2.y * invT;
-      }
-    }
-    if (l == 0) sh[O_Q + P] = 0.0;
-    if constexpr (NS > 0) {
-      const double ctot = Grp::sum(Cl);
-      Grp::sync();
-      if (l < NS) {
-        double M = ctot;
-#pragma unroll
-        for (int e = 0; e < Mech::G_MN; ++e)
-          M += Mech::G_MD[e][l] * sh[O_RP + 2 * Mech::G_MI[e][l]];
-        sh[O_M + l] = M;
       }
     }
     Grp::sync();
@@ -347,19 +353,26 @@ struct GroupKin {
 
   // production rate of species l from the q in LDS: a chunk of entries per lane, then the chunks
   // of each species
-  PELEC_INLINE static void load_gather(uv4 (&e)[Mech::G_L8], int l) {
+  struct Gather {
+    uv4 e[Mech::G_L8];
+    int cp;
+  };
+  PELEC_INLINE static Gather load_gather(int l) {
+    Gather g;
 #pragma unroll
     for (int i = 0; i < Mech::G_L8; ++i)
-      e[i] = *reinterpret_cast<const uv4*>(&Mech::G_GE[i][l][0]);
+      g.e[i] = *reinterpret_cast<const uv4*>(&Mech::G_GE[i][l][0]);
+    g.cp = Mech::G_CP[l];
+    return g;
   }
-  PELEC_INLINE static double gather(const uv4 (&e)[Mech::G_L8], int l, lds_double* sh) {
+  PELEC_INLINE static double gather(const Gather& g, int l, lds_double* sh) {
     double acc = 0.0;
     const lds_char* q = (const lds_char*)(sh + O_Q);
 #pragma unroll
     for (int i = 0; i < Mech::G_L8; ++i)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const unsigned w = e[i][u];
+        const unsigned w = g.e[i][u];
         const double q0 = *(const lds_double*)(q + (w & 0xfff));
         const double q1 = *(const lds_double*)(q + ((w >> 16) & 0xfff));
         acc = fma((double)((int)(w << 16) >> 28), q0, acc);
@@ -367,7 +380,7 @@ struct GroupKin {
       }
     sh[O_PS + l] = acc;
     Grp::sync();
-    const int cp = Mech::G_CP[l], b = cp & 255, m = cp >> 8;
+    const int b = g.cp & 255, m = g.cp >> 8;
     double wd = 0.0;
 #pragma unroll
     for (int u = 0; u < Mech::G_CMAX; ++u)
@@ -390,17 +403,21 @@ struct GroupKin {
     const double ys = sp ? yl : 0.0;
     // the tables of the first phases are loaded ahead of the temperature
     Record nx = record(l);
+    const double iwt = Mech::G_IWT[l];
     const double Tg = Grp::bcast(yl, N);
     const bool lo0 = Tg < tm;
     double gc[8];
     load_g(gc, lo0, l);
+    const double Cl = ys * iwt;
+    third_bodies(Cl, l, sh);
     const double irho = recip(Grp::sum(ys));
     double ec[6], ek, cvk;
     const double T = T_from_e((rhoe0 + t * rhoesrc) * irho, ys * irho, l, Tg, tm, ec, ek, cvk);
     const double lnT = log_T(T, xt), invT = recip(T);
-    prelude<false>(T, lnT, invT, ys * Mech::G_IWT[l], l, tm, gc, lo0, sh, xt);
-    uv4 ge[Mech::G_L8];
-    load_gather(ge, after(l, T));
+    prelude<false>(T, lnT, invT, Cl, l, tm, gc, lo0, sh, xt);
+    const Gather ge = load_gather(after(l, T));
+    const double Wk = Mech::G_WT[after(l, T)];
+    const double D = Grp::sum(ys * cvk);
 #pragma unroll 1
     for (int r = 0; r < RR; ++r) {
       const Record rc = nx;
@@ -410,9 +427,8 @@ struct GroupKin {
     }
     Grp::sync();
     const double wd = gather(ge, l, sh);
-    const double fk = sp ? Mech::G_WT[l] * wd + srcl : 0.0;
+    const double fk = sp ? Wk * wd + srcl : 0.0;
     const double num = rhoesrc - Grp::sum(ek * fk);
-    const double D = Grp::sum(ys * cvk);
     Grp::sync();
     return l == N ? num * recip(D) : fk;
   }
@@ -437,19 +453,20 @@ struct GroupKin {
     const bool lo0 = Tg < tm;
     double gc[8];
     load_g(gc, lo0, l);
+    const double Cl = ys * Mech::G_IWT[l];
+    third_bodies(Cl, l, sh);
     const double irho = 1.0 / Grp::sum(ys);
     double ec[6], ek, cvk;
     const double T = T_from_e((rhoe0 + t * rhoesrc) * irho, ys * irho, l, Tg, tm, ec, ek, cvk);
     const double lnT = log_T(T, xt), invT = recip(T);
-    prelude<true>(T, lnT, invT, ys * Mech::G_IWT[l], l, tm, gc, lo0, sh, xt);
+    prelude<true>(T, lnT, invT, Cl, l, tm, gc, lo0, sh, xt);
     if (l == 0) sh[O_JV + Mech::G_NJ] = 0.0;
 #pragma unroll 1
     for (int r = 0; r < RR; ++r) {
       const int p = after(G * r + l, lnT);
       reaction<true, MUL>(record(p), p, l, T, lnT, invT, sh, xt, rmul);
     }
-    uv4 ge[Mech::G_L8];
-    load_gather(ge, after(l, T));
+    const Gather ge = load_gather(after(l, T));
     // the zeros are in memory before other lanes store over them; the terms are in LDS
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
     Grp::sync();
@@ -668,6 +685,8 @@ struct CellState {
   BdfScalars S;
   double hg, hub, hlb;  // cvHin's iteration
   int count, pad;
+  int64_t g;  // the cell
+  double rhoe0, rhoesrc;
 };
 
 }  // namespace pelec
