@@ -586,7 +586,11 @@ constexpr int WHOLE_WAVES = NV <= 32 ? 3 : 2;
 // of lanes each wave takes fewer cells at a time (gpw): the groups of a wave run in lockstep, so a
 // cell alone on its wave never waits for another cell's phases, and the spare waves cost nothing.
 // One cell per wave against full waves: 700 drm19 cells 3.20 and 3.38 ms, 512 H2/air cells 0.52 and
-// 0.54 ms, 3000 (as many waves as fit) 0.64 and 0.62 ms.
+// 0.54 ms, 3000 (as many waves as fit) 0.64 and 0.62 ms. Where the cells go by their rates
+// (order_bytes) that holds up to as many cells as there are groups: the slowest have a wave each and the
+// rest follow as waves come free. drm19: 3500 cells 4.0 ms two to a wave, 3.5 one; 5000 4.4 and
+// 3.6; 9000 4.2 and 4.5; 30,000 6.4 and 8.6.
+constexpr bool BY_RATE = NV > 16;
 struct WholeGrid {
   int blocks = 0, gpw = 0;
   int64_t groups = 0;  // groups of lanes that own workspace
@@ -613,6 +617,7 @@ int whole_grid(prc_reactor* r, int64_t ncells, WholeGrid& w) {
     if (r->max_slots > 0) groups = std::min<int64_t>(groups, r->max_slots);
     const int64_t per = (groups + r->whole_blocks - 1) / r->whole_blocks;
     w.gpw = (int)std::min<int64_t>(std::max<int64_t>(per, 1), whole_gpw());
+    if (BY_RATE && ncells <= (int64_t)r->whole_blocks * whole_gpw()) w.gpw = 1;
     // (prc.max_slots is a bound on the cells in flight)
     const int64_t up = groups < ncells ? groups / w.gpw : (groups + w.gpw - 1) / w.gpw;
     w.blocks = (int)std::min<int64_t>(std::max<int64_t>(up, 1), r->whole_blocks);
@@ -636,7 +641,7 @@ constexpr size_t whole_bytes() {
 // them. Without and with, ms: drm19 64^3 47.0 and 43.7, GRI-Mech 3.0, 16,384 cells, 22.3 and 19.9,
 // dodecane_lu, 8192 cells, 36.2 and 33.9; H2/air 32^3 1.93 and 1.95.
 size_t order_bytes(int64_t ncells, const WholeGrid& w) {
-  if (NV <= 16 || ncells <= (int64_t)w.blocks * w.gpw || ncells > INT32_MAX) return 0;
+  if (!BY_RATE || ncells <= (int64_t)w.blocks * w.gpw || ncells > INT32_MAX) return 0;
   const size_t n = (size_t)((ncells + 15) & ~15);
   return 2 * CELL_KEYS * sizeof(unsigned) + n * (sizeof(int32_t) + sizeof(uint8_t));
 }
