@@ -582,14 +582,17 @@ constexpr int WHOLE_WAVES = PELEC_WHOLE_WAVES;
 constexpr int WHOLE_WAVES = NV <= 32 ? 3 : 2;
 #endif
 
-// Grid of a call: one wave per block, as many as fit the GPU at once. With fewer cells than groups
-// of lanes each wave takes fewer cells at a time (gpw): the groups of a wave run in lockstep, so a
-// cell alone on its wave never waits for another cell's phases, and the spare waves cost nothing.
-// One cell per wave against full waves: 700 drm19 cells 3.20 and 3.38 ms, 512 H2/air cells 0.52 and
-// 0.54 ms, 3000 (as many waves as fit) 0.64 and 0.62 ms. Where the cells go by their rates
-// (order_bytes) that holds up to as many cells as there are groups: the slowest have a wave each and the
-// rest follow as waves come free. drm19: 3500 cells 4.0 ms two to a wave, 3.5 one; 5000 4.4 and
-// 3.6; 9000 4.2 and 4.5; 30,000 6.4 and 8.6.
+// Grid of a call: one wave per block, as many as fit the GPU at once. The groups of a wave run in lockstep
+// and wait for each other's phases, and waves share a SIMD's issue slots, so a call that does not
+// fill the GPU gives each wave gpw <= 64 / G cells:
+// - n <= 16: enough to make about 1.5 waves per SIMD. H2/air, ms with 1, 2 and 4 cells to a wave: 1000 cells
+//   0.49, 0.51, -; 2000 0.59, 0.56, 0.61; 3000 0.63, 0.56, 0.61; 6144 -, 0.76, 0.68.
+// - else one, up to as many cells as there are groups: the cells go by their rates (order_bytes), so the
+//   slowest have a wave each and the rest follow as waves come free. drm19: 3500 cells 4.0 ms
+//   two to a wave, 3.4 one; 5000 4.4 and 3.5; 30,000 7.0 and 8.6. Where every cell could have a wave at
+//   once, one wave per SIMD and the rest in turn: drm19, 3000 cells 4.0 -> 3.4; GRI-Mech 3.0, 1500 cells
+//   9.3 -> 8.0; dodecane_lu, 1500 cells 19.4 -> 15.8 (3000, more than the waves that fit: 21.1 with
+//   all of them, 23.7 with one per SIMD).
 constexpr bool BY_RATE = NV > 16;
 struct WholeGrid {
   int blocks = 0, gpw = 0;
@@ -615,12 +618,17 @@ int whole_grid(prc_reactor* r, int64_t ncells, WholeGrid& w) {
     }
     int64_t groups = std::max<int64_t>(ncells, 1);
     if (r->max_slots > 0) groups = std::min<int64_t>(groups, r->max_slots);
-    const int64_t per = (groups + r->whole_blocks - 1) / r->whole_blocks;
-    w.gpw = (int)std::min<int64_t>(std::max<int64_t>(per, 1), whole_gpw());
-    if (BY_RATE && ncells <= (int64_t)r->whole_blocks * whole_gpw()) w.gpw = 1;
+    int64_t waves = r->whole_blocks;
+    if (BY_RATE) {
+      w.gpw = ncells <= waves * whole_gpw() ? 1 : whole_gpw();
+      if (ncells <= waves) waves = std::min<int64_t>(waves, 4 * r->ncu);
+    } else {
+      const int64_t some = std::max<int64_t>(waves / 2, 1);
+      w.gpw = (int)std::min<int64_t>((groups + some - 1) / some, whole_gpw());
+    }
     // (prc.max_slots is a bound on the cells in flight)
     const int64_t up = groups < ncells ? groups / w.gpw : (groups + w.gpw - 1) / w.gpw;
-    w.blocks = (int)std::min<int64_t>(std::max<int64_t>(up, 1), r->whole_blocks);
+    w.blocks = (int)std::min<int64_t>(std::max<int64_t>(up, 1), waves);
     w.groups = (int64_t)w.blocks * whole_gpw();
   }
   return PRC_OK;

@@ -101,6 +101,20 @@ def test_refilled_groups(wl, max_slots, big):
     same(react(wl, d, idx, max_slots=max_slots), ref, idx)
 
 
+@pytest.mark.parametrize("wl,sizes", [("lidryer_32", (12289, 1536, 1537, 4609)),
+                                      ("drm19_64", (6145, 1025, 3072, 3073, 6144)),
+                                      ("gri30_flat", (2049, 1024, 1025, 2048))])
+def test_grid_rules(wl, sizes):
+    """Calls on both sides of the grid's lines (256 CUs: 1024, 1536, 2048, 3072 waves; 6144 and 12,288
+    groups) give the bits of the first, larger one."""
+    d = inputs.make_inputs(wl, sizes[0])
+    ref = react(wl, d, np.arange(sizes[0]))
+    assert ref["nfail"] == 0
+    for n in sizes[1:]:
+        idx = np.arange(n)
+        same(react(wl, d, idx), ref, idx)
+
+
 @pytest.mark.parametrize("n", [1001, 4096, 4097])
 def test_cells_in_order_of_their_rates(n):
     """More cells than groups (prc.max_slots), counted and placed by one and two blocks of the counting
