@@ -36,11 +36,11 @@ def log(msg):
 
 
 def measured_traffic(workload, fp32):
-    """HBM bytes per Newton-branch launch from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE
-    summary of this workload and form (profiles/k_newton_<fp32lu|fp64lu>_<workload>_traffic.txt),
-    or None if not measured."""
-    form = "fp32lu" if fp32 else "fp64lu"
-    path = os.path.join(ROOT, "profiles", f"k_newton_{form}_{workload}_traffic.txt")
+    """HBM bytes per launch of the form's dominant kernel from the committed rocprofv3 FETCH_SIZE /
+    WRITE_SIZE summary of this workload (profiles/k_newton_fp32lu_<workload>_traffic.txt,
+    profiles/k_cell_<workload>_traffic.txt), or None if not measured."""
+    form = "k_newton_fp32lu" if fp32 else "k_cell"
+    path = os.path.join(ROOT, "profiles", f"{form}_{workload}_traffic.txt")
     if not os.path.exists(path):
         return None
     for line in open(path):
@@ -486,9 +486,9 @@ def main():
     shape = head["shape"]
     log(f"headline form: {hkey}")
 
-    # per-kernel device time of the headline form: one extra call with HIP events around every
+    # device time of the headline form's kernels: one extra call with HIP events around every
     # k_newton / k_jac / k_lu launch (eager launches; the graph replays of the timed calls are
-    # the same kernels on the same streams)
+    # the same kernels on the same streams), or around the one k_cell launch of the FP64 form
     kt = time_form(torch, Reactor, wl, d0, "batched", head["fp32"], 1, 0, kernel_timing=True,
                    shape=shape)
     t_head = float(np.median(head["times"]))
@@ -500,11 +500,17 @@ def main():
     dg = head["diag"].astype(np.float64)
     W = flops.work(wl.mech, dg[2].sum(), dg[3].sum(), dg[4].sum(), dg[5].sum(), dg[1].sum())
     achieved_call = W / t_head
-    # dominant kernel k_newton: each launch does one Newton iteration (RHS + solve) for every
-    # Newton-phase cell, plus the step completion of the cells that converged
+    # dominant kernel. FP64: k_cell, one launch that does the whole call. FP32 factors: k_newton, each
+    # launch one Newton iteration (RHS + solve) for every Newton-phase cell, plus the step
+    # completion of the cells that converged
     costs = flops.mechanism_costs(wl.mech)
     dk = kt["diag"].astype(np.float64)
-    W_newton = (dk[5].sum() * (costs["F_rhs"] + costs["F_solve"]) + dk[1].sum() * costs["F_step"])
+    whole = kt["kernel_ms"]["k_jac"] == 0 and kt["kernel_ms"]["k_lu"] == 0
+    if whole:
+        W_newton = flops.work(wl.mech, dk[2].sum(), dk[3].sum(), dk[4].sum(), dk[5].sum(), dk[1].sum())
+    else:
+        W_newton = (dk[5].sum() * (costs["F_rhs"] + costs["F_solve"])
+                    + dk[1].sum() * costs["F_step"])
     t_newton = kt["kernel_ms"]["k_newton"] * 1e-3
     launches = max(1, kt["kernel_launches"])
     achieved = W_newton / t_newton
@@ -545,7 +551,8 @@ def main():
         "data": "synthetic",
         "config": {"workload": wl.name, "mechanism": wl.mech, "ncells": n, "dt": wl.dt,
                    "rtol": wl.rtol, "atol": wl.atol,
-                   "form": ("batched work-queue, FP64 throughout" if not head["fp32"] else
+                   "form": ("batched, one lane group per cell, FP64 throughout"
+                            if not head["fp32"] else
                             "batched work-queue, Newton-matrix LU in FP32 (equilibrated) with one "
                             "FP64 refinement step per solve, FP64 elsewhere"),
                    "headline_form": hkey, "launch_shape": shape},
@@ -561,7 +568,8 @@ def main():
         "roofline": {"bound": "fp64-valu", "achieved": achieved / 1e12,
                      "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_FP64,
                      "traffic": traffic,
-                     "kernel": ("Newton branch of " + hkey + ": k_newton (k_newton_g where the "
+                     "kernel": ("k_cell: the whole integrations of " + hkey if whole else
+                                "Newton branch of " + hkey + ": k_newton (k_newton_g where the "
                                 "launch shape or the mechanism selects the cooperative kernel)"),
                      "launches": int(launches), "avg_launch_ms": t_newton / launches * 1e3,
                      "flops_per_launch": W_newton / launches,
