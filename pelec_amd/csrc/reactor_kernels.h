@@ -1002,13 +1002,13 @@ __global__ void __launch_bounds__(CELL_KEYS) k_cell_order(const uint8_t* key, in
 // initial-step iteration, a Newton iteration or an order-1 restart -- so the kinetics are one copy
 // of code that all groups of a wave run together whatever phase their cells are in.
 //
-// What bounds it: vector instruction issue. At drm19 64^3 the VALUs are busy 66 % of the time
-// (dodecane_lu 64^3: 79 %; waves per SIMD: 3 and 2, by the registers of the state), 42 % of the vector
-// instructions are FP64 arithmetic and the rest moves, selects and lane exchanges; HBM carries
-// 28 GB per call, 0.55 TB/s, nearly all of it Jacobian workspace. Compulsory traffic is 146 MB.
+// What bounds it: vector instruction issue. At drm19 64^3 the VALUs are busy 74 % of the time
+// (dodecane_lu 64^3: 87 %; waves per SIMD: 3 and 2, by the registers of the state), 42 % of the vector
+// instructions are FP64 arithmetic (37 %) and the rest moves, selects and lane exchanges; HBM carries
+// 24 GB per call, 0.55 TB/s, nearly all of it Jacobian workspace. Compulsory traffic is 146 MB.
 // Measured against the work queue (a cell's state crossing HBM on every Newton iteration, 16 to 1100
-// launches a call): drm19 64^3 300 -> 50 ms, H2/air 32^3 6.5 -> 1.9 ms, 512 cells 4.6 -> 0.53 ms,
-// dodecane_lu 8192 cells 281 -> 39 ms.
+// launches a call): drm19 64^3 295 -> 44 ms, H2/air 32^3 6.5 -> 1.9 ms, 512 cells 4.6 -> 0.54 ms,
+// dodecane_lu 8192 cells 283 -> 34 ms.
 template <class M, int MINW>
 __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs ca) {
   using K = GroupKin<M>;
@@ -1219,7 +1219,7 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
 // S and E are one value per lane. A static grid: cells share nothing, so the scheduler is the queue.
 // Bound as k_cell is, by the instruction issue of the right-hand side. One cell per lane holds Q, S, E
 // and the kinetics in private memory and 4096 cells are 64 waves: drm19, dt = 1e-7 s, 4096 cells
-// 17.5 ms, 1.5 ms in groups.
+// 17.4 ms, 1.3 ms in groups.
 template <class M>
 __global__ void __launch_bounds__(64) react_rk64_g(const Args a) {
   using K = GroupKin<M>;
