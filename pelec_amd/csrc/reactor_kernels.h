@@ -3,8 +3,10 @@
 //   plain    react_plain: one cell per lane over a static grid, the whole integration of the cell
 //            in one call, working set in private memory -- the straightforward drop-in for
 //            ReactorCvode::react (Source/React.cpp:222-228) and the baseline.
-//   batched  device work queue of per-cell BDF phases (batched.h): k_start, then iterations of
-//            k_jac / k_lu / k_newton over live slots, compaction when half the slots are done.
+//   batched  FP64 factors: k_cell, one lane group integrates a whole cell in registers
+//            (whole_cell.h). FP32 factors, and mechanisms without lane-group tables: a device work
+//            queue of per-cell BDF phases (batched.h): k_start, then iterations of k_jac / k_lu /
+//            k_newton over live slots, compaction when half the slots are done.
 #pragma once
 #include <hip/hip_runtime.h>
 
