@@ -650,26 +650,54 @@ class Gen:
         arr("T_CSR_EFF", "int", [eff[j] for j, _ in flat] + [-1] * pad, [len(flat) + pad])
 
     # ------------------------------------------------------------------ lane-group tables
+    def group_shape(self):
+        """Lanes per cell, rounds of reactions, and positions (lanes times rounds)."""
+        G = 16 if self.N < 16 else 32 if self.N < 32 else 64
+        RR = (self.R + G - 1) // G
+        return G, RR, RR * G
+
+    def group_form_issue(self):
+        """Why the lane-group tables cannot represent this mechanism (None when they can): the work
+        queue, the one-cell-per-lane kernels and, with data tables, the cooperative kernels then
+        run for it. The limits are those of the fields that the lanes decode (whole_cell.h)."""
+        issue = self.table_form_issue()
+        if issue is not None:
+            return issue
+        if self.N > 63:
+            return "more than 63 species"
+        G, _, P = self.group_shape()
+        values = P  # of the Jacobian's terms: dq/dT, dq/dM and dq/dC of each mass-action slot
+        for r in self.m.reactions:
+            sides = (r.reactants, r.products) if r.reversible else (r.reactants,)
+            if any(sum(s.values()) > 3 for s in sides):
+                return f"{r.equation}: order above 3"
+            if any(v != int(v) or not -8 <= v <= 7 for v in self.nu_of(r).values()):
+                return f"{r.equation}: net coefficient not a whole number of -8..7 (4 bits)"
+            values += int(sum(sum(s.values()) for s in sides)) + (r.kind != "elementary")
+        if len(self.effsets) > G:
+            return f"more than {G} efficiency sets (one per lane)"
+        if 8 * P >= 1 << 12:
+            return f"{P} reaction positions: byte offsets above 12 bits"
+        if values >= 1 << 12:
+            return f"{values} Jacobian terms: indices above 12 bits"
+        if (self.N + 1 + len(self.effsets) + 1) * G >= 1 << 15:
+            return "Jacobian elements: indices above 15 bits"
+        return None
+
     def emit_group_tables(self):
         """The mechanism as data in the order the lanes of a group read it (whole_cell.h): species k
         on lane k, reaction at position p = G r + l of T_RORD on lane l in round r, every table
         [...][lane] so that a group's loads are contiguous. Entries of absent lanes and positions are
         neutral: species slot N (concentration and exp(g/RT) of 1), coefficient 0."""
-        if self.table_form_issue() is not None:
+        issue = self.group_form_issue()
+        if issue is not None:
+            self.w(f"  // no lane-group tables: {issue}")
             self.w("  static constexpr bool G_OK = false;")
             return
         N, R, rx, sp = self.N, self.R, self.m.reactions, self.m.species
-        for r in rx:
-            sides = (r.reactants, r.products) if r.reversible else (r.reactants,)
-            nu = list(self.nu_of(r).values())
-            if any(sum(s.values()) > 3 for s in sides) or any(v != int(v) for v in nu) or N > 63:
-                self.w("  static constexpr bool G_OK = false;")
-                return
         w = self.w
         n = N + 1
-        G = 16 if n <= 16 else 32 if n <= 32 else 64
-        RR = (R + G - 1) // G
-        P = RR * G
+        G, RR, P = self.group_shape()
 
         def arr(name, ctype, vals, shape):
             dims = "".join(f"[{d}]" for d in shape)
@@ -819,7 +847,6 @@ class Gen:
                 sched[lane].append(o | (nu & 0xf) << 12 | (1 << 16 if last else 0)
                                    | (c * G + k) << 17)
         JT = (max(load) + 3) // 4 * 4
-        assert NJ < 4096 and (n + ns_ + 1) * G < 1 << 15
         pad = DM + NFO + NTB  # an entry that stays 0
         sched = [x + [pad] * (JT - len(x)) for x in sched]
         w(f"  static constexpr int G_NJ = {NJ};  // values per cell")

@@ -5,6 +5,7 @@ schedule of terms (elements dealt to lanes, columns beyond n for the efficiency 
 Bound: 1e-11 of a row's largest entry (sums of up to ~140 terms in another order than the oracle's,
 each rounded to 1.1e-16, amplified by the cancellation within a rate)."""
 import ast
+import dataclasses
 import re
 
 import numpy as np
@@ -17,7 +18,10 @@ MECHS = ("LiDryer", "drm19", "drm19_inert40", "gri30", "dodecane_lu")
 
 
 def tables(mech):
-    txt = open(mechgen.generate(mech)).read()
+    return decode(open(mechgen.generate(mech)).read())
+
+
+def decode(txt):
     out = {"REFC": M.P_ATM / M.R_ERG}
     for m in re.finditer(r"static constexpr (\w+) G_(\w+)((?:\[\d+\])*) = ([^;]+);", txt):
         ctype, name, dims, val = m.groups()
@@ -149,8 +153,11 @@ def evaluate(t, N, C, T):
 
 @pytest.mark.parametrize("name", MECHS)
 def test_group_tables_against_oracle(name, oracle_lib):
-    mech = M.load(name)
-    t, om, N = tables(name), oracle_lib.OracleMech(mech), mech.nsp
+    check(M.load(name), tables(name), oracle_lib)
+
+
+def check(mech, t, oracle_lib):
+    name, om, N = mech.name, oracle_lib.OracleMech(mech), mech.nsp
     assert t["W"] >= N + 1 and t["NJ"] < 4096 and t["JC"] * t["W"] < 1 << 15
     rng = np.random.default_rng(3)
     nu = np.zeros((mech.nrxn, N))
@@ -169,3 +176,64 @@ def test_group_tables_against_oracle(name, oracle_lib):
         magJ = (np.abs(nu.T) @ np.abs(dqdC)).max(1, keepdims=True) + 1e-300
         assert (np.abs(J - Jr) <= 1e-11 * magJ).all(), name
         assert (np.abs(dT - Tr) <= 1e-10 * (np.abs(nu.T) @ np.abs(dqdT) + 1e-300)).all(), name
+
+
+def repeated(name, nrxn):
+    """The mechanism with its elementary reactions repeated until it has nrxn reactions."""
+    m = M.load(name)
+    el = [r for r in m.reactions if r.kind == "elementary"]
+    more = [el[i % len(el)] for i in range(nrxn - m.nrxn)]
+    return dataclasses.replace(m, reactions=m.reactions + more)
+
+
+def with_reaction(name, **kw):
+    m = M.load(name)
+    r = dataclasses.replace(next(r for r in m.reactions if r.kind == "elementary"), **kw)
+    return dataclasses.replace(m, reactions=m.reactions + [r])
+
+
+def with_sets(name, nsets):
+    """The mechanism with nsets distinct efficiency sets."""
+    m = M.load(name)
+    r = next(r for r in m.reactions if r.kind == "three-body")
+    have = len({tuple(x.efficiencies) for x in m.reactions if x.efficiencies})
+    more = [dataclasses.replace(r, efficiencies=[2.0 + i] + r.efficiencies[1:])
+            for i in range(nsets - have)]
+    return dataclasses.replace(m, reactions=m.reactions + more)
+
+
+#: on either side of each field's limit: 12-bit byte offsets of the reaction positions (448, 480 and
+#: 496 reactions at 64, 32 and 16 lanes), 4-bit net coefficients (of irreversible reactions: the
+#: reverse rate allows three species), one efficiency set per lane, three slots per side
+LIMITS = {
+    "gri30 448": (lambda: repeated("gri30", 448), True),
+    "gri30 449": (lambda: repeated("gri30", 449), False),
+    "gri30 512": (lambda: repeated("gri30", 512), False),
+    "gri30 900": (lambda: repeated("gri30", 900), False),
+    "drm19 480": (lambda: repeated("drm19", 480), True),
+    "drm19 481": (lambda: repeated("drm19", 481), False),
+    "LiDryer 496": (lambda: repeated("LiDryer", 496), True),
+    "LiDryer 497": (lambda: repeated("LiDryer", 497), False),
+    "LiDryer nu 7": (lambda: with_reaction("LiDryer", reactants={0: 1.0}, products={1: 7.0},
+                                           reversible=False), True),
+    "LiDryer nu 8": (lambda: with_reaction("LiDryer", reactants={0: 1.0}, products={1: 8.0},
+                                           reversible=False), False),
+    "LiDryer order 4": (lambda: with_reaction("LiDryer", reactants={0: 2.0, 1: 2.0},
+                                              products={2: 2.0}, reversible=False), False),
+    "LiDryer 16 sets": (lambda: with_sets("LiDryer", 16), True),
+    "LiDryer 17 sets": (lambda: with_sets("LiDryer", 17), False),
+}
+
+
+@pytest.mark.parametrize("case", LIMITS)
+def test_field_limits(case, oracle_lib):
+    """Mechanisms at the limits of the packed fields get tables that hold, those above get none (and
+    a header all the same)."""
+    make, fits = LIMITS[case]
+    mech = make()
+    txt = mechgen.Gen(mech).generate()
+    assert f"static constexpr bool G_OK = {'true' if fits else 'false'};" in txt
+    if fits:
+        check(mech, decode(txt), oracle_lib)
+    else:
+        assert "G_GE" not in txt and "static constexpr bool T_OK = true;" in txt
