@@ -277,8 +277,9 @@ int prc_eos_rty2wdot(int64_t ncells, const double* rho, const double* T, const d
  * ReactorCvodeJacobian, CMake/BuildPelePhysicsLib.cmake:132-141). y = [rhoY_0..N-1, T] and ydot
  * component-major (n x ncells, n = N+1); rhoe0 per cell; rhoesrc (rho e forcing) and rYsrc
  * (N x ncells) may be null; J (ncells x n x n, row-major per cell) may be null. cooperative = 0
- * evaluates one cell per lane, 1 one cell per 32-lane group (the kinetics of the cooperative
- * batched kernels). Device pointers. */
+ * evaluates one cell per lane, 1 one cell per group of lanes with the kinetics of the batched form's
+ * FP64 kernel (without its tables, of the work queue's cooperative kernels), 2 with the work queue's.
+ * PRC_EINVAL for a mechanism that has neither. Device pointers. */
 int prc_model_eval(int64_t ncells, double t, const double* y, const double* rhoe0,
                    const double* rhoesrc, const double* rYsrc, double* ydot, double* J,
                    int cooperative, void* stream);

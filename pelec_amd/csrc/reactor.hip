@@ -853,16 +853,22 @@ int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_coun
   return run_queue(r, a, s, r->d_args, r->d_ctr, true);
 }
 
-// prc_model_eval with one cell per group of lanes; false: the mechanism has no lane-group tables.
+// prc_model_eval with one cell per group of lanes: the whole-cell form's kinetics, or, for a
+// mechanism without its tables and with `queue`, the cooperative queue kernels'. False: neither.
 template <class M = Mech>
-bool launch_model(int64_t nc, double t, const double* y, const double* rhoe0, const double* rhoesrc,
-                  const double* src, double* ydot, double* J, hipStream_t s) {
-  if constexpr (whole_ok<M>()) {
-    constexpr int CPB = 64 / M::G_W;  // cells per block
-    hipLaunchKernelGGL(k_model_cell<M>, dim3((unsigned)((nc + CPB - 1) / CPB)), dim3(64), 0, s, nc,
+bool launch_model(bool queue, int64_t nc, double t, const double* y, const double* rhoe0,
+                  const double* rhoesrc, const double* src, double* ydot, double* J, hipStream_t s) {
+  auto go = [&](auto kern, int per_block) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)((nc + per_block - 1) / per_block)), dim3(64), 0, s, nc,
                        t, y, rhoe0, rhoesrc, src, ydot, J);
     return true;
-  }
+  };
+  if constexpr (whole_ok<M>())
+    if (!queue) return go(k_model_cell<M>, 64 / M::G_W);
+  if constexpr (COOP)
+    return go(k_model_group<GModel>, 2);
+  else if constexpr (COOP64)
+    return go(k_model_group<GroupModel<M, 64>>, 1);
   return false;
 }
 
@@ -1706,7 +1712,8 @@ int prc_model_eval(int64_t nc, double t, const double* y, const double* rhoe0,
   if (nc == 0) return PRC_OK;
   hipStream_t s = (hipStream_t)stream;
   if (cooperative) {
-    if (!launch_model(nc, t, y, rhoe0, rhoesrc, rYsrc, ydot, J, s)) return PRC_EINVAL;
+    if (!launch_model(cooperative == 2, nc, t, y, rhoe0, rhoesrc, rYsrc, ydot, J, s))
+      return PRC_EINVAL;  // this mechanism has no data tables
   } else
     hipLaunchKernelGGL(k_model_lane, dim3((unsigned)((nc + 63) / 64)), dim3(64), 0, s, nc, t, y,
                        rhoe0, rhoesrc, rYsrc, ydot, J);

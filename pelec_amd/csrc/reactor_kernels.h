@@ -1945,7 +1945,27 @@ __global__ void __launch_bounds__(64) k_model_lane(int64_t nc, double t, const d
   if (J) Model::template jac<double>(t, yy, rhoe0[c], r1, src ? src + c : nullptr, nc, J + c * (int64_t)(NV * NV));
 }
 
-// ... or one cell per group of lanes (GroupKin, the whole-cell form's kinetics), 64 / G per block.
+// ... or one cell per G-lane group with the kinetics of the work queue's cooperative kernels
+// (GroupModel), 64 / G per block ...
+template <class GM>
+__global__ void __launch_bounds__(64) k_model_group(int64_t nc, double t, const double* y,
+                                                     const double* rhoe0, const double* rhoesrc,
+                                                     const double* src, double* ydot, double* J) {
+  constexpr int G = GM::GS;
+  __shared__ double lds[64 / G * GM::JAC_WORDS];
+  const int64_t c = (int64_t)blockIdx.x * (64 / G) + threadIdx.x / G;
+  const int l = threadIdx.x & (G - 1);
+  if (c >= nc) return;
+  double* sh = lds + (threadIdx.x / G) * GM::JAC_WORDS;
+  const double yl = l < NV ? y[l * nc + c] : 0.0;
+  const double srcl = (src && l < NSP) ? src[l * nc + c] : 0.0;
+  const double r1 = rhoesrc ? rhoesrc[c] : 0.0;
+  const double f = GM::rhs(t, yl, l, rhoe0[c], r1, srcl, sh);
+  if (l < NV) ydot[l * nc + c] = f;
+  if (J) GM::jac(t, yl, l, rhoe0[c], r1, srcl, sh, J + c * (int64_t)(NV * NV));
+}
+
+// ... or with those of the whole-cell form (GroupKin).
 template <class M>
 __global__ void __launch_bounds__(64) k_model_cell(int64_t nc, double t, const double* y,
                                                     const double* rhoe0, const double* rhoesrc,

@@ -427,14 +427,16 @@ class Eos:
 
     def model(self, t, y, rhoe0, rhoesrc=None, rYsrc=None, jacobian=True, cooperative=False,
               stream=None):
-        """Reactor RHS (and exact Jacobian) at states y (n x ncells): (ydot, J or None)."""
+        """Reactor RHS (and exact Jacobian) at states y (n x ncells): (ydot, J or None).
+        cooperative: False / 0 one cell per lane, True / 1 one cell per lane group with the batched
+        FP64 kernel's kinetics, 2 with those of the work queue's cooperative kernels."""
         import torch
         nc = y.shape[1]
         ydot = torch.empty_like(y)
         J = torch.empty((nc, y.shape[0], y.shape[0]), dtype=y.dtype, device=y.device) \
             if jacobian else None
         _check(self.lib.prc_model_eval(nc, float(t), _ptr(y), _ptr(rhoe0), _ptr(rhoesrc),
-                                       _ptr(rYsrc), _ptr(ydot), _ptr(J), int(bool(cooperative)),
+                                       _ptr(rYsrc), _ptr(ydot), _ptr(J), int(cooperative),
                                        _stream_handle(stream)), "prc_model_eval")
         return ydot, J
 

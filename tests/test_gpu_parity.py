@@ -202,11 +202,11 @@ def test_react_batched_cooperative_lidryer(oracles):
 
 
 @pytest.mark.parametrize("mech,wl", [("LiDryer", "lidryer_32"), ("drm19", "drm19_64")])
-@pytest.mark.parametrize("cooperative", [False, True])
+@pytest.mark.parametrize("cooperative", [False, True, 2])
 def test_model_eval_vs_oracle(mech, wl, cooperative, oracles):
     """RHS and exact Jacobian at given states (prc_model_eval) against the oracle's, for the
-    one-cell-per-lane model and the cooperative (one cell per 32-lane group, table-driven
-    kinetics) model. States: the workload's initial cells and the oracle's end states of the same
+    one-cell-per-lane model, the whole-cell kernel's (one cell per group of lanes) and the work
+    queue's cooperative kernels' (2: one cell per 32-lane group, table-driven kinetics). States: the workload's initial cells and the oracle's end states of the same
     cells (radical pools), with and without rhoY / rho e forcing. Bounds: species rates within
     1e-9 of the cell's largest species rate, the T rate within 1e-9 of its energy scale
     max_k |e_k f_k| / (rho c_v), and Jacobian rows within 1e-8 of the row's largest entry."""
