@@ -24,7 +24,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 #: mechanisms built by default
-DEFAULT_MECHS = ("LiDryer", "drm19", "drm19_inert40", "gri30", "dodecane_lu")
+DEFAULT_MECHS = ("LiDryer", "LiDryer_order4", "drm19", "drm19_inert40", "gri30", "dodecane_lu")
 
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
