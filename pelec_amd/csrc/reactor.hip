@@ -714,9 +714,12 @@ void fill_params(const prc_reactor* r, Args& a, unsigned long long* ctr) {
 template <class M = Mech>
 void launch_rk64(const Args& a, const Args* dargs, hipStream_t s) {
   if constexpr (whole_ok<M>()) {
-    constexpr int CPB = 64 / M::G_W;  // cells per block
-    hipLaunchKernelGGL(react_rk64_g<M>, dim3((unsigned)((a.box.ncells + CPB - 1) / CPB)), dim3(64),
-                       0, s, a);
+    // a launch has fewer than 2^32 threads, which are 2^26 cells at 64 lanes each
+    constexpr int64_t CPB = 64 / M::G_W, BLOCKS = 1 << 24;  // cells per block, blocks per launch
+    for (int64_t c0 = 0; c0 < a.box.ncells; c0 += BLOCKS * CPB) {
+      const int64_t nb = std::min((a.box.ncells - c0 + CPB - 1) / CPB, BLOCKS);
+      hipLaunchKernelGGL(react_rk64_g<M>, dim3((unsigned)nb), dim3(64), 0, s, a, c0);
+    }
   } else {
     hipLaunchKernelGGL(react_rk64<M>, dim3((unsigned)((a.box.ncells + 63) / 64)), dim3(64), 0, s,
                        dargs);

@@ -1223,7 +1223,7 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
 // and the kinetics in private memory and 4096 cells are 64 waves: drm19, dt = 1e-7 s, 4096 cells
 // 17.4 ms, 1.3 ms in groups.
 template <class M>
-__global__ void __launch_bounds__(64) react_rk64_g(const Args a) {
+__global__ void __launch_bounds__(64) react_rk64_g(const Args a, int64_t c0) {
   using K = GroupKin<M>;
   constexpr int G = K::G;
   using Grp = Group<G>;
@@ -1232,7 +1232,7 @@ __global__ void __launch_bounds__(64) react_rk64_g(const Args a) {
   fill_tables(xt);
   const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
   lds_double* sh = lds_ptr(lds) + gid * K::RHS_WORDS;
-  const int64_t c = (int64_t)blockIdx.x * (64 / G) + gid;
+  const int64_t c = c0 + (int64_t)blockIdx.x * (64 / G) + gid;
   const BoxDev& b = a.box;
   if (c >= b.ncells) return;
   int i, j, k;

@@ -178,6 +178,34 @@ def test_rk64_cells_do_not_depend_on_the_call(wl, dt, big):
         same(react(wl, d, idx, dt=dt, rk64=True), ref, idx)
 
 
+def test_rk64_more_lanes_than_a_launch_has(big):
+    """2^27 + 5 drm19 cells of 32 lanes each are more than the 2^32 threads of a launch: all but a
+    few are masked, at both ends, across the launches' seam and in between."""
+    d, _ = big("drm19_64")
+    n = 2 ** 27 + 5
+    at = torch.tensor([0, 1, 2 ** 25 - 1, 2 ** 25, 2 ** 25 + 1, 2 ** 26 + 7, 2 ** 27 - 1, 2 ** 27,
+                       n - 1], device=DEV)
+    idx = np.arange(at.numel())
+    d = {k: d[k][..., :idx.size] for k in ("rY", "T", "rE")}
+    ref = react("drm19_64", d, idx, dt=1e-7, rk64=True)
+    W = inputs.WORKLOADS["drm19_64"]
+    a = {k: torch.zeros(*d[k].shape[:-1], n, dtype=torch.float64, device=DEV) for k in d}
+    for k in a:
+        a[k][..., at] = to_dev(d[k])
+    mask = torch.zeros(n, dtype=torch.int32, device=DEV)
+    mask[at] = 1
+    r = Reactor(W.mech, chem_integrator="ReactorRK64")
+    r.configure(rtol=W.rtol, atol=W.atol)
+    print(f"[gpu-test] rk64 n={n}", flush=True)
+    r.react_flat(a["rY"], a["T"], a["rE"], 1e-7, mask=mask)
+    torch.cuda.synchronize()
+    r.close()
+    for k in a:
+        np.testing.assert_array_equal(a[k][..., at].cpu().numpy(), ref[k], err_msg=k)
+        a[k][..., at] = 0.0
+        assert not a[k].any()
+
+
 @pytest.mark.parametrize("mech,wl", [("LiDryer", "lidryer_32"), ("drm19", "drm19_adj")])
 def test_adjoint_cells_do_not_depend_on_the_call(mech, wl):
     W = inputs.WORKLOADS[wl]
