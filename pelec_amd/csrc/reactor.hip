@@ -710,19 +710,28 @@ void fill_params(const prc_reactor* r, Args& a, unsigned long long* ctr) {
   a.ctr = ctr;
 }
 
-// ReactorRK64 on a.box: one cell per group of lanes where the mechanism has its tables.
+// ReactorRK64 on a.box: one cell per group of lanes where the mechanism has its tables. For n <= 16
+// the lane kernel's straight-line kinetics take fewer instructions a cell, and it is the faster one
+// once it has waves enough. H2/air, dt = 1e-6 s: groups 0.58 ms for 16,384 cells, 0.74 for 20,480, 0.99
+// for 32,768 and 6.4 for 262,144; lanes 0.74 from 24,577 to 65,536 cells, one wave's time, and 2.6
+// for 262,144. (drm19, 262,144 cells: groups 28, lanes 155.)
+constexpr int64_t RK64_LANE_CELLS = NV <= 16 ? 20480 : INT64_MAX;
 template <class M = Mech>
 void launch_rk64(const Args& a, const Args* dargs, hipStream_t s) {
+  bool lanes = true;
+  if constexpr (whole_ok<M>()) lanes = a.box.ncells > RK64_LANE_CELLS;
+  if constexpr (!whole_ok<M>() || RK64_LANE_CELLS < INT64_MAX)
+    if (lanes)
+      hipLaunchKernelGGL(react_rk64<M>, dim3((unsigned)((a.box.ncells + 63) / 64)), dim3(64), 0, s,
+                         dargs);
   if constexpr (whole_ok<M>()) {
+    if (lanes) return;
     // a launch has fewer than 2^32 threads, which are 2^26 cells at 64 lanes each
     constexpr int64_t CPB = 64 / M::G_W, BLOCKS = 1 << 24;  // cells per block, blocks per launch
     for (int64_t c0 = 0; c0 < a.box.ncells; c0 += BLOCKS * CPB) {
       const int64_t nb = std::min((a.box.ncells - c0 + CPB - 1) / CPB, BLOCKS);
       hipLaunchKernelGGL(react_rk64_g<M>, dim3((unsigned)nb), dim3(64), 0, s, a, c0);
     }
-  } else {
-    hipLaunchKernelGGL(react_rk64<M>, dim3((unsigned)((a.box.ncells + 63) / 64)), dim3(64), 0, s,
-                       dargs);
   }
 }
 

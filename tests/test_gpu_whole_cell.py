@@ -178,6 +178,24 @@ def test_rk64_cells_do_not_depend_on_the_call(wl, dt, big):
         same(react(wl, d, idx, dt=dt, rk64=True), ref, idx)
 
 
+@pytest.mark.parametrize("n", [20480, 20481])
+def test_rk64_on_both_sides_of_the_lane_kernels_line(n, oracle_lib):
+    """H2/air cells go one per group of lanes up to 20,480 of them, one per lane above."""
+    wl = "lidryer_32"
+    W = inputs.WORKLOADS[wl]
+    d = dict(inputs.make_inputs(wl, n))
+    d["mask"] = (np.random.default_rng(3).uniform(size=n) > 0.2).astype(np.int32)
+    out = react(wl, d, np.arange(n), rk64=True)
+    assert out["nfail"] == 0
+    idx = np.r_[0:80, n - 80:n]
+    ref = oracle_lib.OracleMech(M.load(W.mech)).react_rk64(
+        d["rY"][:, idx], d["T"][idx], d["rE"][idx], W.dt, rtol=W.rtol, atol=W.atol,
+        mask=d["mask"][idx], nthreads=8)
+    assert np.abs(out["T"][idx] - ref["T"]).max() <= GATE_T
+    assert (np.abs(out["rY"][:, idx] - ref["rY"]) / ref["rY"].sum(0)).max() <= GATE_Y
+    np.testing.assert_array_equal(out["diag"][1][idx], ref["stats"][:, 0])
+
+
 def test_rk64_more_lanes_than_a_launch_has(big):
     """2^27 + 5 drm19 cells of 32 lanes each are more than the 2^32 threads of a launch: all but a
     few are masked, at both ends, across the launches' seam and in between."""
