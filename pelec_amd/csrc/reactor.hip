@@ -620,7 +620,8 @@ int whole_grid(prc_reactor* r, int64_t ncells, WholeGrid& w) {
     if (r->max_slots > 0) groups = std::min<int64_t>(groups, r->max_slots);
     int64_t waves = r->whole_blocks;
     if (BY_RATE) {
-      w.gpw = ncells <= waves * whole_gpw() ? 1 : whole_gpw();
+      // (fewer cells in flight than waves, by prc.max_slots: one to a wave)
+      w.gpw = groups <= waves || ncells <= waves * whole_gpw() ? 1 : whole_gpw();
       if (ncells <= waves) waves = std::min<int64_t>(waves, 4 * r->ncu);
     } else {
       const int64_t some = std::max<int64_t>(waves / 2, 1);

@@ -101,6 +101,29 @@ def test_refilled_groups(wl, max_slots, big):
     same(react(wl, d, idx, max_slots=max_slots), ref, idx)
 
 
+@pytest.mark.parametrize("wl,n", [("lidryer_32", 12300), ("drm19_64", 6200)])
+@pytest.mark.parametrize("max_slots", [1, 2, 3, 0])
+def test_max_slots_bounds_the_cells_in_flight(wl, n, max_slots):
+    """In a call of more cells than the grid has groups (all but a few masked), where a wave would
+    take several cells."""
+    W = inputs.WORKLOADS[wl]
+    d = inputs.make_inputs(wl, n)
+    on = np.arange(0, n, n // 10)
+    mask = np.zeros(n, np.int32)
+    mask[on] = 1
+    r = Reactor(W.mech)
+    r.configure(rtol=W.rtol, atol=W.atol, form="batched", lu_fp32=False, max_slots=max_slots)
+    a = {k: to_dev(d[k]) for k in ("rY", "T", "rE")}
+    r.react_flat(a["rY"], a["T"], a["rE"], W.dt, mask=to_dev(mask, torch.int32))
+    torch.cuda.synchronize()
+    slots = r.get_param("prc.slots")
+    assert r.last_failures() == 0 and 1 <= slots <= (max_slots or n)
+    r.close()
+    few = react(wl, {k: d[k] for k in a}, on)
+    for k in a:
+        np.testing.assert_array_equal(a[k].cpu().numpy()[..., on], few[k], err_msg=k)
+
+
 @pytest.mark.parametrize("wl,sizes", [("lidryer_32", (12289, 1536, 1537, 4609)),
                                       ("drm19_64", (6145, 1025, 3072, 3073, 6144)),
                                       ("gri30_flat", (2049, 1024, 1025, 2048))])
