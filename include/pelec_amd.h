@@ -114,8 +114,8 @@ int prc_set_param_real(prc_reactor* r, const char* key, double value);
  * every this many iterations while no cell waits for a slot; 0 = only between replays),
  * prc.coop_tail_slots (once at most this many slots are in
  * use, the Newton kernel runs one cell per 32-lane group; 0 = never; while neither this nor
- * prc.cooperative has been set, a call chooses both by its slots in use) and prc.blocks_tail (its
- * blocks per CU), prc.max_slots (slots of the batched form's work queue: 0 = one per cell while
+ * prc.cooperative has been set, a call chooses both, and they read back as chosen) and
+ * prc.blocks_tail (its blocks per CU; 0 = occupancy-derived, 8 where the call chooses), prc.max_slots (slots of the batched form's work queue: 0 = one per cell while
  * half the free device memory holds them; a call with more cells than slots refills the slots
  * that finished cells free, from the call's cell queue); for tests, prc.test_lu_fail = 1 makes
  * the batched form's factorisation report every Newton matrix as singular, which drives CVODE's

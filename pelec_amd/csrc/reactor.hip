@@ -443,17 +443,22 @@ int eager_accumulate(prc_reactor* r) {
 // (5.5 and 3.5 ms) and 32,768 (6.6 and 11.7 ms).
 constexpr int AUTO_TAIL_SLOTS = NV <= 16 ? 12288 : 65536;
 
-// The handle's shape with that choice made, for the length of a call.
+// The shape that a queue call of the handle runs with: its own, with that choice made.
+Shape shape_in_use(const prc_reactor* r) {
+  Shape sh = r->shape;
+  if (COOP && !r->coop_set) {
+    sh.coop = 2;
+    sh.tail_slots = AUTO_TAIL_SLOTS;
+    if (sh.bpc_tail == 0) sh.bpc_tail = 8;
+  }
+  return sh;
+}
+
+// The handle's shape replaced by it for the length of a call.
 struct ShapeInUse {
   prc_reactor* r;
   Shape set;
-  explicit ShapeInUse(prc_reactor* h) : r(h), set(h->shape) {
-    if (COOP && !r->coop_set) {
-      r->shape.coop = 2;
-      r->shape.tail_slots = AUTO_TAIL_SLOTS;
-      r->shape.bpc_tail = std::max(set.bpc_tail, 8);
-    }
-  }
+  explicit ShapeInUse(prc_reactor* h) : r(h), set(h->shape) { r->shape = shape_in_use(r); }
   ~ShapeInUse() { r->shape = set; }
 };
 
@@ -1140,24 +1145,26 @@ int prc_set_param_int(prc_reactor* r, const char* key, int v) {
 
 int prc_get_param_int(prc_reactor* r, const char* key, int* v) {
   if (!r || !key || !v) return PRC_EINVAL;
+  // (calls with FP64 factors run no queue where the mechanism has the whole-cell form)
+  const Shape sh = WHOLE && !r->lu_fp32 ? r->shape : shape_in_use(r);
   if (!std::strcmp(key, "prc.iters_per_graph"))
-    *v = r->shape.iters;
+    *v = sh.iters;
   else if (!std::strcmp(key, "prc.blocks_newton"))
-    *v = r->shape.bpc_newton > 0 ? r->shape.bpc_newton : r->occ_newton;
+    *v = sh.bpc_newton > 0 ? sh.bpc_newton : r->occ_newton;
   else if (!std::strcmp(key, "prc.blocks_jac"))
-    *v = r->shape.bpc_jac > 0 ? r->shape.bpc_jac : r->occ_jac;
+    *v = sh.bpc_jac > 0 ? sh.bpc_jac : r->occ_jac;
   else if (!std::strcmp(key, "prc.blocks_lu"))
-    *v = r->shape.bpc_lu > 0 ? r->shape.bpc_lu : r->occ_lu;
+    *v = sh.bpc_lu > 0 ? sh.bpc_lu : r->occ_lu;
   else if (!std::strcmp(key, "prc.compact_pct"))
-    *v = r->shape.compact_pct;
+    *v = sh.compact_pct;
   else if (!std::strcmp(key, "prc.compact_every"))
-    *v = r->shape.compact_every;
+    *v = sh.compact_every;
   else if (!std::strcmp(key, "prc.cooperative"))
-    *v = r->shape.coop;
+    *v = sh.coop;
   else if (!std::strcmp(key, "prc.coop_tail_slots"))
-    *v = r->shape.tail_slots;
+    *v = sh.tail_slots;
   else if (!std::strcmp(key, "prc.blocks_tail"))
-    *v = r->shape.bpc_tail > 0 ? r->shape.bpc_tail : r->occ_tail;
+    *v = sh.bpc_tail > 0 ? sh.bpc_tail : r->occ_tail;
   else if (!std::strcmp(key, "prc.form"))
     *v = r->form;
   else if (!std::strcmp(key, "prc.lu_fp32"))

@@ -73,6 +73,35 @@ def test_argument_validation_without_gpu():
     assert lib.prc_destroy(h) == 0
 
 
+def test_queue_shape_readback():
+    """The launch-shape knobs report what a queue call runs with: the kernels it chooses itself while
+    neither prc.cooperative nor prc.coop_tail_slots was set, and every explicit choice."""
+    r = reactor.load_library("drm19")
+    h = ctypes.c_void_p()
+    assert r.prc_create(b"ReactorCvode", ctypes.byref(h)) == 0
+    put = lambda k, v: r.prc_set_param_int(h, k, v)  # noqa: E731
+
+    def get():
+        v = ctypes.c_int()
+        out = []
+        for k in (b"prc.cooperative", b"prc.coop_tail_slots", b"prc.blocks_tail"):
+            assert r.prc_get_param_int(h, k, ctypes.byref(v)) == 0
+            out.append(v.value)
+        return tuple(out)
+
+    assert put(b"prc.form", 1) == 0
+    assert get()[:2] == (0, 0)  # FP64 factors: no queue
+    assert put(b"prc.lu_fp32", 1) == 0
+    assert get() == (2, 65536, 8)
+    assert put(b"prc.blocks_tail", 3) == 0
+    assert get() == (2, 65536, 3)
+    assert put(b"prc.cooperative", 1) == 0
+    assert get() == (1, 0, 3)
+    assert put(b"prc.coop_tail_slots", 77) == 0
+    assert get() == (1, 77, 3)
+    assert r.prc_destroy(h) == 0
+
+
 SHIM_HARNESS = r"""
 // AMReX-shaped stand-ins: the shim binds to any Box / Array4 with these members.
 #include <cstdio>
