@@ -119,7 +119,8 @@ int prc_set_param_real(prc_reactor* r, const char* key, double value);
  * half the free device memory holds them; a call with more cells than slots refills the slots
  * that finished cells free, from the call's cell queue); for tests, prc.test_lu_fail = 1 makes
  * the batched form's factorisation report every Newton matrix as singular, which drives CVODE's
- * convergence-failure handling) */
+ * convergence-failure handling, and prc.test_max_groups = g has the FP64 form's workspace refused for
+ * more than g groups of lanes, as if the memory were not there; 0 = never) */
 int prc_set_param_int(prc_reactor* r, const char* key, int value);
 /* Read back an integer knob (the prc.* launch-shape knobs report the values in use; "prc.slots"
  * gives the slot count of the batched workspace now allocated, or, after a call with FP64 factors,

@@ -164,6 +164,8 @@ struct prc_reactor {
   // prc.test_lu_fail: the batched form's factorisation kernel reports every Newton matrix as
   // singular, so tests can drive the convergence-failure handling from the host
   int test_lu_fail = 0;
+  // prc.test_max_groups: an allocation of more groups' workspace than this counts as refused (0: none)
+  int test_max_groups = 0;
   double kt_ms[3] = {0.0, 0.0, 0.0};  // newton, jac, lu
   int64_t kt_launches = 0;
   std::vector<hipEvent_t> kt_ev;
@@ -829,10 +831,17 @@ int launch(prc_reactor* r, Args& a, bool has_src, hipStream_t s, bool reset_coun
     e = whole_grid(r, a.ncells, w);
     if (e) return e;
     if (w.groups > r->wws_groups) {
+      // (waves the free memory has no workspace for take their cells in turn)
       if (r->wws) (void)hipFree(r->wws);
       r->wws = nullptr;
       r->wws_groups = 0;
-      if (hipMalloc(&r->wws, whole_bytes() * w.groups) != hipSuccess) return PRC_ENOMEM;
+      while ((r->test_max_groups && w.groups > r->test_max_groups) ||
+             hipMalloc(&r->wws, whole_bytes() * w.groups) != hipSuccess) {
+        (void)hipGetLastError();
+        if (w.blocks == 1) return PRC_ENOMEM;
+        w.blocks /= 2;
+        w.groups = (int64_t)w.blocks * whole_gpw();
+      }
       r->wws_groups = w.groups;
     }
     a.has_src = has_src ? 1 : 0;
@@ -1137,6 +1146,9 @@ int prc_set_param_int(prc_reactor* r, const char* key, int v) {
     r->kernel_timing = v ? 1 : 0;
   } else if (!std::strcmp(key, "prc.test_lu_fail")) {
     r->test_lu_fail = v ? 1 : 0;
+  } else if (!std::strcmp(key, "prc.test_max_groups")) {
+    if (v < 0) return PRC_EINVAL;
+    r->test_max_groups = v;
   } else {
     return PRC_EINVAL;
   }

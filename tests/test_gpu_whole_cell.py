@@ -138,6 +138,33 @@ def test_grid_rules(wl, sizes):
         same(react(wl, d, idx), ref, idx)
 
 
+@pytest.mark.parametrize("wl", WORKLOADS)
+def test_workspace_as_the_memory_allows(wl, big):
+    """Workspace refused for more groups than a few waves have: the grid is halved until it fits and
+    the cells go in turn; refused for a single wave: PRC_ENOMEM, and the next call is served."""
+    d, ref = big(wl)
+    W = inputs.WORKLOADS[wl]
+    per_wave = 1 if M.load(W.mech).nsp >= 32 else 2 if M.load(W.mech).nsp >= 16 else 4
+    r = Reactor(W.mech)
+    r.configure(rtol=W.rtol, atol=W.atol, form="batched", lu_fp32=False)
+    a = {k: to_dev(d[k]) for k in ("rY", "T", "rE")}
+    kw = dict(rYsrc=to_dev(d["rYsrc"]), rEsrc=to_dev(d["rEsrc"]), mask=to_dev(d["mask"], torch.int32))
+    if per_wave > 1:
+        r.set_param("prc.test_max_groups", per_wave - 1)
+        with pytest.raises(Exception, match="ENOMEM"):
+            r.react_flat(a["rY"], a["T"], a["rE"], W.dt, **kw)
+    for groups in (per_wave, 9 * per_wave):
+        r.set_param("prc.test_max_groups", groups)
+        for k in a:
+            a[k].copy_(to_dev(d[k]))
+        r.react_flat(a["rY"], a["T"], a["rE"], W.dt, **kw)
+        torch.cuda.synchronize()
+        assert r.last_failures() == 0 and 1 <= r.get_param("prc.slots") <= groups
+        for k in a:
+            np.testing.assert_array_equal(a[k].cpu().numpy(), ref[k], err_msg=k)
+    r.close()
+
+
 @pytest.mark.parametrize("n", [1001, 4096, 4097])
 def test_cells_in_order_of_their_rates(n):
     """More cells than groups (prc.max_slots), counted and placed by one and two blocks of the counting
