@@ -137,7 +137,6 @@ struct prc_reactor {
   bool coop_set = false;  // prc.cooperative or prc.coop_tail_slots was set (or autotuned)
   int ncu = 0;
   int occ_newton = 1, occ_jac = 1, occ_lu = 1, occ_tail = 1;
-  int64_t last_iterations = 0;
   // whole-cell form: device memory for the Jacobians of the cells in flight, its size in groups of
   // lanes, and the waves of k_cell that fit the GPU (0: not looked up yet)
   double* wws = nullptr;
@@ -561,7 +560,6 @@ int run_batched(prc_reactor* r, Args& a, hipStream_t s, Args* dargs, unsigned lo
       }
     }
   }
-  r->last_iterations = iters;
   return PRC_OK;
 }
 
