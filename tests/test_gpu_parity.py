@@ -173,8 +173,7 @@ def test_react_plain_fp64_vs_oracle(wl, n, oracles):
     np.testing.assert_array_equal(out["rE"], d["rE"])
 
 
-@pytest.mark.parametrize("lu_fp32,cooperative", [(False, False), (True, False), (False, True),
-                                                   (True, True)])
+@pytest.mark.parametrize("lu_fp32,cooperative", [(False, False), (True, False), (True, True)])
 def test_react_batched_vs_oracle(lu_fp32, cooperative, oracles):
     wl, n = "drm19_64", 4096
     W = inputs.WORKLOADS[wl]
@@ -512,14 +511,17 @@ def test_graph_compaction_matches_host_compaction(oracles):
     """prc.compact_every: the captured graph compacts the work queue itself (gate kernel, then the
     compaction kernels) between iterations. Compaction only moves slots, so with no tail graph the
     end states are bit-identical to host-only compaction, in graph replays and in the eager,
-    event-timed iterations; both meet the oracle gates (drm19, 16384 cells, FP64 factors)."""
+    event-timed iterations; both meet the oracle gates (drm19, 16384 cells, FP32 factors: those with
+    FP64 factors run no queue)."""
     wl, n = "drm19_64", 16384
     W = inputs.WORKLOADS[wl]
     d = inputs.make_inputs(wl, n)
     outs = {}
     for every, kt in ((0, False), (3, False), (3, True)):
         r = Reactor(W.mech)
-        r.configure(rtol=W.rtol, atol=W.atol, form="batched", lu_fp32=False, kernel_timing=kt)
+        r.configure(rtol=W.rtol, atol=W.atol, form="batched", lu_fp32=True, kernel_timing=kt,
+                    cooperative=0)
+        r.set_param("prc.coop_tail_slots", 0)
         r.set_param("prc.iters_per_graph", 15)
         r.set_param("prc.compact_pct", 90)
         r.set_param("prc.compact_every", every)
