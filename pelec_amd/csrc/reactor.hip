@@ -763,7 +763,7 @@ int adjoint_grid(prc_reactor* r, int64_t ncells, AdjGrid& g) {
     g.gpw = (int)std::min<int64_t>(per, GPW);
     g.blocks = (int)std::min<int64_t>((ncells + g.gpw - 1) / g.gpw, r->adj_blocks);
     g.rmul = (size_t)((GroupKin<M>::P + 1) & ~1);
-    g.words = g.rmul + (size_t)g.blocks * GPW * (hist + 2 * GroupKin<M>::JAC_SIZE);
+    g.words = g.rmul + (size_t)g.blocks * g.gpw * (hist + 2 * GroupKin<M>::JAC_SIZE);
   } else {
     g.blocks = (int)((ncells + 63) / 64);
     g.rmul = (size_t)M::NRXN;

@@ -1611,7 +1611,7 @@ __global__ void __launch_bounds__(64, 2) k_adjoint_g(const AdjArgs a, unsigned l
   fill_tables(lds_ptr(lds) + GPW * K::WORDS);
   const int l = threadIdx.x & (G - 1), gid = threadIdx.x / G;
   if (gid >= gpw) return;
-  const int64_t nc = a.ncells, w = (int64_t)blockIdx.x * GPW + gid;
+  const int64_t nc = a.ncells, w = (int64_t)blockIdx.x * gpw + gid;
   C cell(scl[gid]);
   cell.l = l;
   cell.sh = lds + gid * K::WORDS;

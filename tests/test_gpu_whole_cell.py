@@ -304,6 +304,34 @@ def test_adjoint_cells_do_not_depend_on_the_call(mech, wl):
             np.testing.assert_array_equal(v, ref[k][..., idx], err_msg=f"{k} {first} {n}")
 
 
+def test_adjoint_workspace_is_one_share_per_cell():
+    """A single cell with many checkpoints (320 MB of them at n = 10) takes one group's share of
+    workspace, not that of the four groups of its wave."""
+    wl, n, ck = "lidryer_32", 10, 200000
+    W = inputs.WORKLOADS[wl]
+    d = inputs.make_inputs(wl, 1)
+    a = [to_dev(d[k]) for k in ("rY", "T", "rE")]
+
+    def go(r):
+        out = r.adjoint(*a, W.dt, ct_rY=torch.ones_like(a[0]), ct_T=torch.ones_like(a[1]))
+        torch.cuda.synchronize()
+        assert int(out["status"][0]) == 0
+        return {k: v.cpu().numpy() for k, v in out.items()}
+
+    r = Reactor(W.mech)
+    r.configure(rtol=W.rtol, atol=W.atol)
+    ref = go(r)
+    free0 = torch.cuda.mem_get_info()[0]
+    r.set_param("adj.max_checkpoints", ck)
+    out = go(r)
+    used = free0 - torch.cuda.mem_get_info()[0]
+    r.close()
+    share = 8 * ck * ((6 + n) * n + 60)  # a checkpoint: z, the Jacobian, the integrator's scalars
+    assert 0.5 * share <= used <= 2.0 * share, (used, share)
+    for k in ref:
+        np.testing.assert_array_equal(out[k], ref[k], err_msg=k)
+
+
 @pytest.mark.parametrize("n", [1, 12288, 12289])
 def test_fp32_queue_shape_of_its_own(n, oracle_lib):
     """FP32 factors with neither prc.cooperative nor prc.coop_tail_slots set: H2/air cells run in
