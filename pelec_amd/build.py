@@ -32,8 +32,8 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
     # machine-level loop-invariant code motion hoists the literals and table loads of the kinetics
-    # out of the kernels' cell loops and keeps them in registers: k_cell at n = 22 needs 168 VGPRs and
-    # 436 B of scratch per lane with it, 164 VGPRs and no scratch without
+    # out of the kernels' cell loops and keeps them in registers: at n = 22, bytes of scratch per lane
+    # with it and without, k_cell (168 VGPRs) 348 and 88, k_adjoint_g (256) 672 and 288
     "-mllvm", "-disable-machine-licm",
     # per-kernel register / scratch / LDS figures, checked below
     "-Rpass-analysis=kernel-resource-usage",

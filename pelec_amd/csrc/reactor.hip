@@ -438,10 +438,10 @@ int eager_accumulate(prc_reactor* r) {
 
 // The queue's kernels when neither prc.cooperative nor prc.coop_tail_slots was set: the cooperative
 // Jacobian, and the cooperative Newton kernel while at most this many slots are in use. One cell per
-// lane pays off only once its waves fill the GPU: drm19, FP32 factors, 5001 cells take 127 ms with one
-// cell per lane throughout, 28 ms in groups; 65,536 cells 208 and 78 ms; 262,144 cells 320 and 297 ms,
-// 175 ms with the switch. H2/air (a third of the work per iteration) crosses between 5001 cells
-// (5.5 and 3.5 ms) and 32,768 (6.6 and 11.7 ms).
+// lane pays off only once its waves fill the GPU: drm19, FP32 factors, 5001 cells take 128 ms with one
+// cell per lane throughout, 28 ms in groups; 65,536 cells 210 and 79 ms; 262,144 cells 321 and 300 ms,
+// 228 ms with the switch. H2/air (a third of the work per iteration) crosses between 5001 cells
+// (5.4 and 4.0 ms) and 32,768 (6.5 and 12.5 ms, 5.8 ms with the switch).
 constexpr int AUTO_TAIL_SLOTS = NV <= 16 ? 12288 : 65536;
 
 // The shape that a queue call of the handle runs with: its own, with that choice made.
