@@ -893,44 +893,50 @@ __device__ inline bool reached_tstop(BdfScalars& S, double tstop) {
   return false;
 }
 
+// cvHin's control: bounds of the initial step from the largest |f_i| / (0.1 |y_i| + 1/ewt_i), and the
+// first trial hg. True: no step lies between them, hg it is.
+__device__ inline bool hin_bounds(double tn, double tout, double hub_inv, double& hlb, double& hub,
+                                  double& hg) {
+  hlb = 100.0 * cv::UROUND * fmax(fabs(tn), fabs(tout));
+  hub = 0.1 * (tout - tn);
+  if (hub * hub_inv > 1.0) hub = 1.0 / hub_inv;
+  hg = sqrt(hlb * hub);
+  return hub < hlb;
+}
+// ... and the next trial from ||y''|| at the count-th, hg (1, 2, ...). True: hg is now the initial step.
+__device__ inline bool hin_next(double yddnrm, int count, double hlb, double hub, double& hg) {
+  double hnew = (yddnrm * hub * hub > 2.0) ? sqrt(2.0 / yddnrm) : sqrt(hg * hub);
+  const double hrat = hnew / hg;
+  bool last = count == 4 || (hrat > 0.5 && hrat < 2.0);
+  if (!last && count > 1 && hrat > 2.0) {
+    hnew = hg;
+    last = true;
+  }
+  hg = last ? fmin(fmax(0.5 * hnew, hlb), hub) : hnew;
+  return last;
+}
+
 // cvHin: initial step size from an estimate of ||y''||; zn[1] holds f(t0, y0) on entry.
 // f(t, y, out) evaluates the RHS (and counts it).
 template <int n, class V, class F>
 __device__ inline double hin(BdfScalars& S, const V& v, double tout, F&& f) {
-  const double tdist = tout - S.tn;
-  const double tround = cv::UROUND * fmax(fabs(S.tn), fabs(tout));
-  const double hlb = 100.0 * tround;
   double hub_inv = 0.0;
 #pragma unroll
   for (int i = v.c0(); i < n; i += V::kStep) {
     const double d = 0.1 * fabs(v.Z(0, i)) + 1.0 / v.E(i);
     hub_inv = fmax(hub_inv, fabs(v.Z(1, i)) / d);
   }
-  hub_inv = v.max(hub_inv);
-  double hub = 0.1 * tdist;
-  if (hub * hub_inv > 1.0) hub = 1.0 / hub_inv;
-  double hg = sqrt(hlb * hub);
-  if (hub < hlb) return hg;
-  double hnew = hg;
+  double hlb, hub, hg;
+  if (hin_bounds(S.tn, tout, v.max(hub_inv), hlb, hub, hg)) return hg;
   typename V::template Arr<n> y, t;
-  for (int count1 = 1; count1 <= 4; ++count1) {
+  for (int count = 1;; ++count) {
 #pragma unroll
     for (int i = v.c0(); i < n; i += V::kStep) y[i] = v.Z(0, i) + hg * v.Z(1, i);
     f(S.tn + hg, y, t);
 #pragma unroll
     for (int i = v.c0(); i < n; i += V::kStep) t[i] = (t[i] - v.Z(1, i)) / hg;
-    const double yddnrm = wrms_reg<n>(v, t);
-    hnew = (yddnrm * hub * hub > 2.0) ? sqrt(2.0 / yddnrm) : sqrt(hg * hub);
-    if (count1 == 4) break;
-    const double hrat = hnew / hg;
-    if (hrat > 0.5 && hrat < 2.0) break;
-    if (count1 > 1 && hrat > 2.0) {
-      hnew = hg;
-      break;
-    }
-    hg = hnew;
+    if (hin_next(wrms_reg<n>(v, t), count, hlb, hub, hg)) return hg;
   }
-  return fmin(fmax(0.5 * hnew, hlb), hub);
 }
 
 // One Newton correction (after f(tn, y) is in ftemp): tempv = M^{-1}(gamma f - rl1 zn1 - acor),

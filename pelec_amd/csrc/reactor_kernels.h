@@ -1136,41 +1136,24 @@ __global__ void __launch_bounds__(64, MINW) k_cell(const Args a, const CellArgs 
         ph = CP_NEWTON;
       } else {
         // f(t0, y0), then cvHin's iteration (hin), one evaluation per turn
-        bool have_h = false;
-        double h0 = 0.0;
+        bool have_h;
+        double h0;
         if (ph == CP_F0) {
           z[1] = f.x;  // 0 on lanes without a component
-          const double tdist = a.dt - S.tn;
-          const double hlb = 100.0 * cv::UROUND * fmax(fabs(S.tn), fabs(a.dt));
           const double hub_inv = Grp::max(fabs(z[1]) / (0.1 * fabs(z[0]) + 1.0 / ew));
-          double hub = 0.1 * tdist;
-          if (hub * hub_inv > 1.0) hub = 1.0 / hub_inv;
-          h0 = sqrt(hlb * hub);
-          have_h = hub < hlb;
-          cs.hg = h0;
+          double hlb, hub;
+          have_h = hin_bounds(S.tn, a.dt, hub_inv, hlb, hub, h0);
           cs.hub = hub;
           cs.hlb = hlb;
           cs.count = 1;
           ph = CP_HIN;
         } else {
-          const double hg = cs.hg, hub = cs.hub;
-          const double w = (f.x - z[1]) / hg * ew;
-          const double yddnrm = sqrt(Grp::sum(w * w) / NV);
-          double hnew = (yddnrm * hub * hub > 2.0) ? sqrt(2.0 / yddnrm) : sqrt(hg * hub);
-          const double hrat = hnew / hg;
-          bool last = cs.count == 4 || (hrat > 0.5 && hrat < 2.0);
-          if (!last && cs.count > 1 && hrat > 2.0) {
-            hnew = hg;
-            last = true;
-          }
-          if (last) {
-            h0 = fmin(fmax(0.5 * hnew, cs.hlb), hub);
-            have_h = true;
-          } else {
-            cs.hg = hnew;
-            cs.count++;
-          }
+          h0 = cs.hg;
+          const double w = (f.x - z[1]) / h0 * ew;
+          have_h = hin_next(sqrt(Grp::sum(w * w) / NV), cs.count, cs.hlb, cs.hub, h0);
+          cs.count++;
         }
+        cs.hg = h0;
         if (have_h) {
           S.h = h0;
           if ((S.tn + S.h - a.dt) * S.h > 0.0) S.h = (a.dt - S.tn) * (1.0 - 4.0 * cv::UROUND);
