@@ -185,8 +185,8 @@ int prc_react_boxes(prc_reactor* r, int nboxes, const prc_box_args* boxes, doubl
  * work-queue counters and the batched workspace live in a static device array of
  * PRC_NOALLOC_SCRATCH_BYTES per GPU (held by the library until the process ends, located at
  * prc_init), and the work queue gets as many slots as that array holds (drm19 about 13,000,
- * GRI-Mech 3.0 about 3,000), refilled from the call's cells, so any ncells up to INT32_MAX is
- * accepted. PRC_ENOMEM if not even 64 slots fit; PRC_ESTATE if the handle was initialised on
+ * GRI-Mech 3.0 about 3,000; with FP64 factors as many lane groups), refilled from the call's cells, so
+ * any ncells up to INT32_MAX is accepted. PRC_ENOMEM if not even 64 slots, or one wave's groups, fit; PRC_ESTATE if the handle was initialised on
  * another device. Iterations are enqueued directly (no graph is instantiated). Every call on a
  * GPU shares that GPU's array: calls that overlap on one GPU -- from any handle of this
  * mechanism's library -- race, and must be serialised by the caller. Blocks like prc_react_flat;
